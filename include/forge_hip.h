@@ -277,10 +277,12 @@ int64_t forge_rmsnorm_bwd_workspace(int dtype, int64_t rows, int64_t cols);
 /* C[m, n] = act(alpha * sum_k A[m*a_sm + k*a_sk] * B[k*b_sk + n*b_sn]
  *               + beta * C[m, n] + bias[n])   (bias of the operand dtype,
  * optional; act = FORGE_GEMM_ACT_NONE, _SILU, _RELU or _GELU, the tanh form)
- * with one fp32 fmaf per k in increasing k order (deterministic).  Operands
- * of `dtype` (fp32, fp16 or bf16); C of c_dtype = fp32 or dtype, row stride
- * ldc.  Any shape and stride: the path for fp32 / fp16 models and for K or
- * pitches that are not multiples of 8, which the bf16 MFMA core does not take.
+ * with fp32 accumulation and one rounding (deterministic).  Operands of
+ * `dtype` (fp32, fp16 or bf16); C of c_dtype = fp32 or dtype, row stride ldc.
+ * Any shape and stride.  fp16 / bf16 products without a bias whose operands
+ * are 16-byte aligned, have a unit stride along one dimension with an extent
+ * that is a multiple of 8, and a pitch that is a multiple of 8 run on the MFMA
+ * core; the others do one fp32 fmaf per k in increasing k order.
  * Replaces the cuBLAS products of the fused linear + cross-entropy path
  * (kernels/cross_entropy/experiments/v2/fused_linear_cross_entropy.py:142-144,
  * 207-219: logits = X W^T + b, dX = dlogits W, dW += dlogits^T X,
@@ -306,9 +308,9 @@ enum { FORGE_LAYOUT_ROW = 0, FORGE_LAYOUT_COL = 1 };
  * means every column.  Segments with disjoint column ranges make several
  * independent products one launch (e.g. [dQ B_q | dK B_k | dV B_v]). */
 typedef struct forge_gemm_segment {
-  const void* a;  /* bf16 */
+  const void* a;  /* bf16 (forge_gemm_f16: fp16) */
   int64_t lda;    /* multiple of 8, at most 4,194,303 (256 rows < 2^31 bytes) */
-  const void* b;  /* bf16 */
+  const void* b;  /* as a */
   int64_t ldb;    /* as lda */
   int64_t k;      /* extent of this segment along K (multiple of 8) */
   int64_t n_lo, n_hi;
@@ -347,6 +349,14 @@ int forge_gemm(int64_t M, int64_t N, const forge_gemm_segment* segs, int n_segs,
                int a_layout, int b_layout,
                void* c, int64_t ldc, int c_dtype, float alpha, float beta,
                int epilogue, int split_k, void* stream);
+
+/* forge_gemm with fp16 operands; c_dtype is FORGE_DTYPE_F16 or
+ * FORGE_DTYPE_F32 (FORGE_EPI_ATOMIC_F32 is bf16 only).  The fp16 models of
+ * the LoRA paths (kernels/lora_mlp/tests/test_lora_mlp.py:507-549). */
+int forge_gemm_f16(int64_t M, int64_t N, const forge_gemm_segment* segs, int n_segs,
+                   int a_layout, int b_layout,
+                   void* c, int64_t ldc, int c_dtype, float alpha, float beta,
+                   int epilogue, int split_k, void* stream);
 
 /* ------------------------------------------------------------------------
  * Fused LoRA entry points (bf16 storage, fp32 accumulation)

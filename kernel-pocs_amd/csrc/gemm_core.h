@@ -44,6 +44,19 @@ namespace fgemm {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 fp16x8 __attribute__((ext_vector_type(8)));
+
+// The engines move operands as 16-bit words (bf16x8 is their 16-byte
+// fragment); the element type T (bf16_t or fp16_t) decides the MFMA
+// instruction, which has one shape, lane layout and rate for both types, and
+// the conversions of a STORE epilogue's 16-bit C.  Both accumulate in fp32.
+template <class T>
+__device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
+  if constexpr (std::is_same_v<T, fp16_t>)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(fp16x8, a), __builtin_bit_cast(fp16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
 
 constexpr int BK = 64;
 constexpr int LDS_PITCH = BK + 8;  // bf16 elements per LDS row
@@ -73,7 +86,7 @@ struct Seg {
 constexpr int MAX_SEGS = 6;
 
 enum Epi {
-  EPI_STORE_BF16 = 0,   // C = alpha*acc + beta*C
+  EPI_STORE_BF16 = 0,   // C = alpha*acc + beta*C, C of the operands' 16-bit type
   EPI_STORE_F32 = 1,     // C = alpha*acc + beta*C; with split-K, one partial slice per split
   EPI_ATOMIC_F32 = 2,   // C += alpha*acc
   EPI_SWIGLU_FWD = 3,   // dual: e, g, h = silu(e) * g
@@ -149,6 +162,7 @@ struct GemmArgs {
   int n_segs;
   Seg segs[MAX_SEGS];
   int split_k;   // number of K partitions (grid z)
+  int f16;       // operands (and a 16-bit C) are fp16 instead of bf16
   EpiArgs ep;
   // Dispatch order of the column tiles when their K work differs (column-
   // ranged segments of different lengths): n_col_order = tiles_n (at most
@@ -444,19 +458,26 @@ __device__ __forceinline__ void st16(void* p, uint4 v) {
   const u32x4_t w = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(w, reinterpret_cast<u32x4_t*>(p));
 }
+template <class T = bf16_t>
 __device__ __forceinline__ void unpack8(uint4 v, float (&f)[8]) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    f[2 * i] = __uint_as_float(w[i] << 16);
-    f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    if constexpr (std::is_same_v<T, fp16_t>) {
+      f[2 * i] = (float)__builtin_bit_cast(fp16_t, (uint16_t)(w[i] & 0xffffu));
+      f[2 * i + 1] = (float)__builtin_bit_cast(fp16_t, (uint16_t)(w[i] >> 16));
+    } else {
+      f[2 * i] = __uint_as_float(w[i] << 16);
+      f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
   }
 }
+template <class T = bf16_t>
 __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
   uint32_t w[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const __bf16 lo = (__bf16)f[2 * i], hi = (__bf16)f[2 * i + 1];
+    const T lo = (T)f[2 * i], hi = (T)f[2 * i + 1];
     w[i] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
   }
   return make_uint4(w[0], w[1], w[2], w[3]);
@@ -481,7 +502,7 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-template <int WAVES_M, int WAVES_N, int BMODE, int EPI>
+template <class T, int WAVES_M, int WAVES_N, int BMODE, int EPI>
 __device__ __forceinline__ void epilogue_staged(const GemmArgs& args,
                                                 f32x16 (&acc)[256 / WAVES_M / 32][256 / WAVES_N / 32], int64_t m0,
                                                 int64_t n0, int lane, int wm, int wn, float* lds) {
@@ -712,24 +733,24 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs& args,
             }
             v[q] *= a;
           }
-          __bf16* cp = (__bf16*)ep.c + m * ep.ldc + n;
+          T* cp = (T*)ep.c + m * ep.ldc + n;
           if (full) {
             if (ep.beta != 0.f) {
               float cv[8];
-              unpack8(ld16(cp), cv);
+              unpack8<T>(ld16(cp), cv);
 #pragma unroll
               for (int q = 0; q < 8; ++q) v[q] += ep.beta * cv[q];
             }
             if (ep.act)
 #pragma unroll
               for (int q = 0; q < 8; ++q) v[q] = epi_act(ep.act, v[q]);
-            st16(cp, pack8(v));
+            st16(cp, pack8<T>(v));
           } else {
             for (int q = 0; q < 8 && n + q < N; ++q) {
               float o = v[q];
               if (ep.beta != 0.f) o += ep.beta * (float)cp[q];
               if (ep.act) o = epi_act(ep.act, o);
-              cp[q] = (__bf16)o;
+              cp[q] = (T)o;
             }
           }
         }
@@ -738,7 +759,7 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs& args,
   }
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int EPI>
+template <class T, int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int EPI>
 __device__ __forceinline__ void epilogue(const GemmArgs& args, f32x16 (&acc)[BM / WAVES_M / 32][BN / WAVES_N / 32],
                                          int64_t m0, int64_t n0, int lane, int wm, int wn) {
   constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N;
@@ -766,11 +787,11 @@ __device__ __forceinline__ void epilogue(const GemmArgs& args, f32x16 (&acc)[BM 
           if (m >= M) continue;
           const float v = col_alpha * acc[i][j][r];
           if constexpr (EPI == EPI_STORE_BF16) {
-            __bf16* cp = (__bf16*)ep.c + m * ep.ldc + n;
+            T* cp = (T*)ep.c + m * ep.ldc + n;
             float o = v;
             if (ep.beta != 0.f) o += ep.beta * (float)(*cp);
             if (ep.act) o = epi_act(ep.act, o);
-            *cp = (__bf16)o;
+            *cp = (T)o;
           } else if constexpr (EPI == EPI_STORE_F32) {
             float* cp = (float*)ep.c + (int64_t)blockIdx.z * ep.split_stride + m * ep.ldc + n;
             float o = v;
@@ -868,7 +889,8 @@ __device__ __forceinline__ void epilogue(const GemmArgs& args, f32x16 (&acc)[BM 
   }
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int A_LAYOUT, int B_LAYOUT, int BMODE, int EPI, bool STAGED>
+template <class T, int BM, int BN, int WAVES_M, int WAVES_N, int A_LAYOUT, int B_LAYOUT, int BMODE, int EPI,
+          bool STAGED>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_kernel(GemmArgs args) {
   constexpr int NT = WAVES_M * WAVES_N * 64;
@@ -1001,7 +1023,7 @@ void gemm_kernel(GemmArgs args) {
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[slot][i], bfr[slot][j], acc[i][j], 0, 0, 0);
+          acc[i][j] = mfma32<T>(af[slot][i], bfr[slot][j], acc[i][j]);
       __builtin_amdgcn_sched_group_barrier(SG_MFMA, FM * FN, 0);
       if (ks + 2 < BK / 16) {
         read_frags(ks + 2, slot);
@@ -1035,9 +1057,9 @@ void gemm_kernel(GemmArgs args) {
 
   if constexpr (STAGED) {
     static_assert(staged_ok(BM, BN, WAVES_M, WAVES_N, EPI), "staged epilogue: 256 x 256 tile, wave tiles of <= 128 rows");
-    epilogue_staged<WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
+    epilogue_staged<T, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
   } else {
-    epilogue<BM, BN, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn);
+    epilogue<T, BM, BN, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn);
   }
 }
 
@@ -1218,8 +1240,8 @@ __device__ __forceinline__ void wait_vmcnt() {
 // AT / BT: A stored [K][M] / B stored [K][N] (token-major, see DmaLoaderT).
 // CPA / CPB: cache-policy bits of the A / B buffer loads (0 = default; 2 =
 // nontemporal, for an operand that no other workgroup reads again).
-template <int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int EPI, int BKT, int NSTAGE, bool STAGED, int WPE,
-          bool AT = false, bool BT = false, int CPA = 0, int CPB = 0>
+template <class T, int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int EPI, int BKT, int NSTAGE, bool STAGED,
+          int WPE, bool AT = false, bool BT = false, int CPA = 0, int CPB = 0>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void gemm_dma_kernel(GemmArgs args) {
   constexpr int NT = WAVES_M * WAVES_N * 64;
@@ -1372,7 +1394,7 @@ void gemm_dma_kernel(GemmArgs args) {
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[sl][i], bfr[sl][j], acc[i][j], 0, 0, 0);
+          acc[i][j] = mfma32<T>(af[sl][i], bfr[sl][j], acc[i][j]);
       __builtin_amdgcn_sched_group_barrier(SG_MFMA, FM * FN, 0);
       if (ks + 2 < KS) {
         read_frags(ks + 2, sl);
@@ -1414,9 +1436,9 @@ void gemm_dma_kernel(GemmArgs args) {
   }
   if constexpr (STAGED) {
     static_assert(staged_ok(BM, BN, WAVES_M, WAVES_N, EPI), "staged epilogue: 256 x 256 tile, wave tiles of <= 128 rows");
-    epilogue_staged<WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
+    epilogue_staged<T, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
   } else {
-    epilogue<BM, BN, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn);
+    epilogue<T, BM, BN, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn);
   }
 }
 

@@ -3,9 +3,15 @@
 // Any strides (so every layout: X W^T, dY W, dY^T X), fp32 / fp16 / bf16
 // operands, fp32 accumulation with one fmaf per k in increasing k order
 // (deterministic, and exact to fp32 rounding).  It is the path for what the
-// bf16 MFMA core does not take: fp32 and fp16 models, and K or row pitches
-// that are not multiples of 8.  The fused linear + cross-entropy path uses it
-// for those shapes; bf16 shapes with aligned pitches go to the MFMA core.
+// MFMA core does not take: fp32 models, and 16-bit operands whose extents or
+// row pitches are not multiples of 8.  16-bit products that the core does
+// take (mfma_segment below) run there: same products, fp32 accumulation, one
+// rounding, another summation order.
+//
+// Why: this kernel does one fmaf per multiply (no matrix instruction) and is
+// bound by its LDS reads at 70 TFLOP/s; [2048, 2048] x [2048, 8192] in fp16
+// takes 989 us here, 67 us on the MFMA core with W as stored [N][K] and
+// 75-90 us with W as stored [K][N] (MI355X).
 //
 // Tiling: 64 x 64 output tiles, 16-deep K tiles staged in LDS as fp32,
 // 256 threads with 4 x 4 outputs each.  Operand loads are coalesced along
@@ -119,6 +125,30 @@ int launch_generic(const GenArgs& g, int c_dtype, hipStream_t s) {
   return FORGE_OK;
 }
 
+// The product as one segment of the MFMA core (fp16 or bf16 operands), or
+// false.  The core fetches 16-byte chunks along each operand's unit-stride
+// dimension, so that dimension's extent and the other's stride must be
+// multiples of 8 (and a pitch at most 2^31 / 512 elements, so that a tile's
+// byte offsets fit 31 bits); it has no bias.
+bool mfma_segment(const GenArgs& g, forge_gemm_segment& seg, int& al, int& bl) {
+  if (g.bias || g.K == 0 || !aligned16(g.a) || !aligned16(g.b)) return false;
+  constexpr int64_t kMaxPitch = (int64_t(1) << 31) / 512 - 1;
+  if (g.a_sk == 1) al = 0, seg.lda = g.a_sm;       // [M][K]
+  else if (g.a_sm == 1) al = 1, seg.lda = g.a_sk;  // [K][M]
+  else return false;
+  if (g.b_sk == 1) bl = 1, seg.ldb = g.b_sn;       // [N][K]
+  else if (g.b_sn == 1) bl = 0, seg.ldb = g.b_sk;  // [K][N]
+  else return false;
+  if (seg.lda % 8 || seg.ldb % 8 || seg.lda < 0 || seg.ldb < 0 || seg.lda > kMaxPitch || seg.ldb > kMaxPitch) return false;
+  if ((al == 0 || bl == 1) && g.K % 8) return false;
+  if ((al == 1 && g.M % 8) || (bl == 0 && g.N % 8)) return false;
+  seg.a = g.a;
+  seg.b = g.b;
+  seg.k = g.K;
+  seg.n_lo = seg.n_hi = 0;
+  return true;
+}
+
 }  // namespace
 
 extern "C" int forge_gemm_generic(int64_t M, int64_t N, int64_t K, int dtype, const void* a, int64_t a_sm,
@@ -137,6 +167,15 @@ extern "C" int forge_gemm_generic(int64_t M, int64_t N, int64_t K, int dtype, co
   if (!c || (K > 0 && (!a || !b))) return forge_set_error(FORGE_ERR_INVALID, "gemm_generic: null operand");
   GenArgs g{M, N, K, a, a_sm, a_sk, b, b_sk, b_sn, c, ldc, bias, alpha, beta, act};
   hipStream_t s = (hipStream_t)stream;
+  forge_gemm_segment seg;
+  int al, bl;
+  if (dtype != FORGE_DTYPE_F32 && mfma_segment(g, seg, al, bl)) {
+    const int epi = act == FORGE_GEMM_ACT_SILU ? FORGE_EPI_SILU
+                  : act == FORGE_GEMM_ACT_RELU ? FORGE_EPI_RELU
+                  : act == FORGE_GEMM_ACT_GELU ? FORGE_EPI_GELU : FORGE_EPI_STORE;
+    return (dtype == FORGE_DTYPE_F16 ? forge_gemm_f16 : forge_gemm)(M, N, &seg, 1, al, bl, c, ldc, c_dtype, alpha, beta,
+                                                                    epi, 1, stream);
+  }
   switch (dtype) {
     case FORGE_DTYPE_F32: return launch_generic<float>(g, c_dtype, s);
     case FORGE_DTYPE_F16: return launch_generic<fp16_t>(g, c_dtype, s);

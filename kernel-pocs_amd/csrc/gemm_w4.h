@@ -140,7 +140,7 @@ struct W4Loader {
 constexpr int W4_NHALF = 5;
 constexpr int W4_HALF = 256 * 64 * 2;  // bytes per half-slot
 
-template <int BMODE, int EPI, bool STAGED>
+template <class T, int BMODE, int EPI, bool STAGED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_w4_kernel(GemmArgs args) {
   constexpr int BM = 256, BN = 256, WAVES_M = 2, WAVES_N = 2, BKT = 64;
@@ -281,7 +281,7 @@ void gemm_w4_kernel(GemmArgs args) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int m = 2 * p + u, i = m / FN, j = m % FN;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[sl][j], af[sl][i], acc[i][j], 0, 0, 0);
+      acc[i][j] = mfma32<T>(bfr[sl][j], af[sl][i], acc[i][j]);
     }
   };
   constexpr int NPAIR = FM * FN / 2;  // 8 MFMA pairs per k-step ...
@@ -383,9 +383,9 @@ void gemm_w4_kernel(GemmArgs args) {
     if constexpr (BMODE == B_DUAL)
       w4_epilogue_staged_dual<EPI>(args, acc, m0, n0, lane, wm, wn, lds);
     else  // (STORE_BF16 is launched staged at beta = 0 only)
-      w4_epilogue_staged<EPI>(args, acc, m0, n0, lane, wm, wn, lds);
+      w4_epilogue_staged<T, EPI>(args, acc, m0, n0, lane, wm, wn, lds);
   } else {
-    w4_epilogue_direct<BMODE, EPI>(args, acc, m0, n0, lane, wm, wn);
+    w4_epilogue_direct<T, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn);
   }
 }
 

@@ -40,11 +40,12 @@ constexpr bool w4_staged_epi(int epi) {
   return epi == EPI_STORE_BF16 || epi == EPI_ROPE || glu_fwd_epi(epi) || glu_bwd_epi(epi);
 }
 
+template <class T = bf16_t>
 __device__ __forceinline__ uint2 pack4(const float (&f)[4]) {
   uint32_t w[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const __bf16 lo = (__bf16)f[2 * i], hi = (__bf16)f[2 * i + 1];
+    const T lo = (T)f[2 * i], hi = (T)f[2 * i + 1];
     w[i] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
   }
   return make_uint2(w[0], w[1]);
@@ -61,7 +62,7 @@ __device__ __forceinline__ float col_alpha(const EpiArgs& ep, int64_t n) {
 // ---------------------------------------------------------------------------
 // Direct epilogue: every element from registers, bounds-checked.
 // ---------------------------------------------------------------------------
-template <int BMODE, int EPI>
+template <class T, int BMODE, int EPI>
 __device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x16 (&acc)[4][4], int64_t m0, int64_t n0,
                                                    int lane, int wm, int wn) {
   const EpiArgs& ep = args.ep;
@@ -151,12 +152,12 @@ __device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x16 
             for (int q = 0; q < 4 && nb + q < N; ++q)
               atomicAdd((float*)ep.c + m * ep.ldc + nb + q, col_alpha(ep, nb + q) * acc[i][j][4 * g + q]);
           } else if constexpr (EPI == EPI_STORE_BF16) {
-            __bf16* cp = (__bf16*)ep.c + m * ep.ldc + nb;
+            T* cp = (T*)ep.c + m * ep.ldc + nb;
             for (int q = 0; q < 4 && nb + q < N; ++q) {
               float o = col_alpha(ep, nb + q) * acc[i][j][4 * g + q];
               if (ep.beta != 0.f) o += ep.beta * (float)cp[q];
               if (ep.act) o = epi_act(ep.act, o);
-              cp[q] = (__bf16)o;
+              cp[q] = (T)o;
             }
           } else if constexpr (glu_bwd_epi(EPI)) {
             for (int q = 0; q < 4 && nb + q < N; ++q) {
@@ -403,7 +404,7 @@ __device__ __forceinline__ void w4_rank_partial_any(const __bf16* lds, const __b
 // the whole 256 x 256 tile in LDS as bf16, then each thread owns column chunk
 // c = 8 (tid % 32) and walks rows tid / 32 + 8 it.
 // ---------------------------------------------------------------------------
-template <int EPI>
+template <class T, int EPI>
 __device__ __forceinline__ void w4_epilogue_staged(const GemmArgs& args, f32x16 (&acc)[4][4], int64_t m0, int64_t n0,
                                                    int lane, int wm, int wn, __bf16* lds) {
   const EpiArgs& ep = args.ep;
@@ -424,7 +425,7 @@ __device__ __forceinline__ void w4_epilogue_staged(const GemmArgs& args, f32x16 
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = alpha * acc[i][j][4 * g + q];
         *reinterpret_cast<uint2*>(lds + (wm * 128 + i * 32 + lane % 32) * W4_SP + wn * 128 + 32 * j + 8 * g + cl) =
-            pack4(v);
+            pack4<T>(v);
       }
   lds_barrier();
   constexpr int IT = 256 / 8, GRP = 4;  // rows per thread; side inputs of 4 rows in flight

@@ -118,6 +118,7 @@ forge_gemm = _decl(
     "forge_gemm",
     [c_i64, c_i64, ctypes.POINTER(GemmSegment), c_int, c_int, c_int, c_vp, c_i64, c_int, c_f32, c_f32, c_int, c_int, c_vp],
 )
+forge_gemm_f16 = _decl("forge_gemm_f16", forge_gemm.argtypes)
 forge_lora_mlp_gate_up = _decl(
     "forge_lora_mlp_gate_up",
     [c_i64] * 4 + [c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_vp, c_vp, c_i64, c_int, c_vp],
@@ -194,7 +195,7 @@ EXPORTED = [
     "forge_swiglu_fwd", "forge_swiglu_bwd", "forge_geglu_fwd", "forge_geglu_bwd", "forge_rope",
     "forge_ce_fwd", "forge_ce_target_stats", "forge_ce_fwd_reduce", "forge_ce_stats_wait", "forge_ce_scale",
     "forge_sum_f32",
-    "forge_gemm", "forge_lora_mlp_gate_up", "forge_lora_mlp_gate_up_v", "forge_lora_mlp_down_bwd", "forge_lora_mlp_down_bwd_v", "forge_lora_mlp_glu_bwd",
+    "forge_gemm", "forge_gemm_f16", "forge_lora_mlp_gate_up", "forge_lora_mlp_gate_up_v", "forge_lora_mlp_down_bwd", "forge_lora_mlp_down_bwd_v", "forge_lora_mlp_glu_bwd",
     "forge_lora_qkv_rope", "forge_lora_qkv_rope_bwd",
     "forge_lora_a", "forge_lora_a_noalloc", "forge_zero", "forge_copy", "forge_cast_f32_bf16", "forge_splitk_reduce",
     "forge_ce_target_prob", "forge_row_scale", "forge_gemm_generic", "forge_transpose_2b", "forge_transpose_2b_batch",
