@@ -378,9 +378,12 @@ void gemm_w4_kernel(GemmArgs args) {
     wait_vmcnt<0>();  // no zero-fill DMA may land in the staged epilogue's LDS
   }
   if constexpr (STAGED) {
-    static_assert(w4_staged_epi(EPI), "staged epilogue: bf16 outputs");
+    static_assert(w4_staged_epi(EPI), "staged epilogue: 16-bit or fp32 outputs");
+    static_assert(RING >= W4_F32_BYTES, "the fp32 epilogue's slabs reuse the ring");
     __bf16* lds = reinterpret_cast<__bf16*>(smem);
-    if constexpr (BMODE == B_DUAL)
+    if constexpr (EPI == EPI_STORE_F32)
+      w4_epilogue_f32(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
+    else if constexpr (BMODE == B_DUAL)
       w4_epilogue_staged_dual<EPI>(args, acc, m0, n0, lane, wm, wn, lds);
     else  // (STORE_BF16 is launched staged at beta = 0 only)
       w4_epilogue_staged<T, EPI>(args, acc, m0, n0, lane, wm, wn, lds);

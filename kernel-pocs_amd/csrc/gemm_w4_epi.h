@@ -21,8 +21,8 @@
 // whole 8192 x 14336 output (K = 0 launches): fp32 staging of 128-row halves
 // 16.2 us per round of 256 tiles.
 //
-// The direct epilogue (fp32 and atomic outputs, beta != 0, and buffers whose
-// alignment rules out 16-byte vectors) works per element from registers.
+// The direct epilogue (atomic outputs, a 16-bit C with beta != 0, and buffers
+// whose alignment rules out 16-byte vectors) works per element from registers.
 #pragma once
 
 #include "gemm_core.h"
@@ -37,7 +37,7 @@ constexpr int W4_DUAL_BYTES = 3 * 128 * W4_DP * 2;    // dual B: e, g, h of 128 
 // Epilogues staged through LDS (with ep.vec_ok; STORE_BF16 only with a plain
 // alpha: no beta, no activation, no per-column alpha groups).
 constexpr bool w4_staged_epi(int epi) {
-  return epi == EPI_STORE_BF16 || epi == EPI_ROPE || glu_fwd_epi(epi) || glu_bwd_epi(epi);
+  return epi == EPI_STORE_BF16 || epi == EPI_STORE_F32 || epi == EPI_ROPE || glu_fwd_epi(epi) || glu_bwd_epi(epi);
 }
 
 template <class T = bf16_t>
@@ -131,22 +131,10 @@ __device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x16 
             float v[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) v[q] = col_alpha(ep, nb + q) * acc[i][j][4 * g + q];
-            if (ep.vec_ok && nb + 4 <= N) {  // 16-byte aligned: ldc % 8 == 0, nb % 4 == 0
-              float4* c4 = reinterpret_cast<float4*>(cp);
-              if (ep.beta != 0.f) {
-                const float4 o = *c4;
-                v[0] += ep.beta * o.x; v[1] += ep.beta * o.y; v[2] += ep.beta * o.z; v[3] += ep.beta * o.w;
-              }
-              if (ep.act)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) v[q] = epi_act(ep.act, v[q]);
-              *c4 = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
-              for (int q = 0; q < 4 && nb + q < N; ++q) {
-                float o = v[q];
-                if (ep.beta != 0.f) o += ep.beta * cp[q];
-                cp[q] = ep.act ? epi_act(ep.act, o) : o;
-              }
+            for (int q = 0; q < 4 && nb + q < N; ++q) {
+              float o = v[q];
+              if (ep.beta != 0.f) o += ep.beta * cp[q];
+              cp[q] = ep.act ? epi_act(ep.act, o) : o;
             }
           } else if constexpr (EPI == EPI_ATOMIC_F32) {
             for (int q = 0; q < 4 && nb + q < N; ++q)
@@ -170,6 +158,83 @@ __device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x16 
             }
           }
         }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// fp32 C (split-K partial slices, beta accumulation): each wave moves its own
+// 128 x 128 block through a private LDS slab, 32 rows at a time (two slabs,
+// so a slab's global stores overlap the next one's LDS writes; no workgroup
+// barrier).  A store instruction then covers two whole 512-byte row runs; the
+// direct epilogue's covers 32 rows of 32 bytes, a quarter of a cache line
+// each.  Bound by the writes.  Measured on MI355X, the GEMM and its reduction:
+// [2048, 8192], K = 2048 split 8 ways 829 -> 304 us; [1003, 4096], K = 14336
+// split 4 ways 176 -> 110 us; [256, 4096], K = 4096 split 8 ways 87 -> 33 us
+// (with every case unrolled in one loop the last two took 130 and 52 us: the
+// code outgrew the instruction cache).
+// ---------------------------------------------------------------------------
+constexpr int W4_FP = 128 + 4;                      // floats per staged row (4 banks apart)
+constexpr int W4_F32_BYTES = 4 * 2 * 32 * W4_FP * 4;  // 4 waves x 2 slabs of 32 rows
+
+__device__ __forceinline__ void w4_epilogue_f32(const GemmArgs& args, f32x16 (&acc)[4][4], int64_t m0, int64_t n0,
+                                                int lane, int wm, int wn, float* lds) {
+  const EpiArgs& ep = args.ep;
+  const int64_t M = args.M, N = args.N;
+  const int cl = 4 * (lane / 32);
+  lds_barrier();  // the main loop's LDS reads are done in every wave
+  float* base = lds + (wn * 2 + wm) * 2 * 32 * W4_FP;
+  const int c = (lane % 32) * 4;
+  const int64_t n = n0 + wn * 128 + c;
+  float* cbase = (float*)ep.c + (int64_t)blockIdx.z * ep.split_stride;
+  const bool plain = ep.beta == 0.f && !ep.act && ep.alpha_group == 0 && n0 + 256 <= N;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float* slab = base + (i & 1) * 32 * W4_FP;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4*>(slab + (lane % 32) * W4_FP + 32 * j + 8 * g + cl) =
+            make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's slab is written
+    const int64_t mb = m0 + wm * 128 + i * 32;
+    if (plain) {  // a store per row run, nothing read
+#pragma unroll
+      for (int it = 0; it < 16; ++it) {
+        const int rr = it * 2 + lane / 32;
+        const float4 v = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
+        if (mb + rr < M)
+          *reinterpret_cast<float4*>(cbase + (mb + rr) * ep.ldc + n) =
+              make_float4(ep.alpha * v.x, ep.alpha * v.y, ep.alpha * v.z, ep.alpha * v.w);
+      }
+      continue;
+    }
+    // beta, activations, per-column alphas and the last columns of a ragged N
+    // (loops kept rolled: unrolled, this code is fetched from memory by every
+    // launch and costs more than the stores)
+#pragma unroll 1
+    for (int it = 0; it < 16; ++it) {
+      const int rr = it * 2 + lane / 32;
+      float* cp = cbase + (mb + rr) * ep.ldc + n;
+      if (mb + rr >= M) continue;
+      if (n + 4 <= N && !ep.act && ep.alpha_group == 0) {  // 16-byte aligned: ldc % 8 == 0
+        const float4 a4 = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
+        float4* c4 = reinterpret_cast<float4*>(cp);
+        float4 v = make_float4(ep.alpha * a4.x, ep.alpha * a4.y, ep.alpha * a4.z, ep.alpha * a4.w);
+        if (ep.beta != 0.f) {
+          const float4 o = *c4;
+          v.x += ep.beta * o.x; v.y += ep.beta * o.y; v.z += ep.beta * o.z; v.w += ep.beta * o.w;
+        }
+        *c4 = v;
+        continue;
+      }
+#pragma unroll 1
+      for (int q = 0; q < 4 && n + q < N; ++q) {
+        float o = col_alpha(ep, n + q) * slab[rr * W4_FP + c + q];
+        if (ep.beta != 0.f) o += ep.beta * cp[q];
+        cp[q] = ep.act ? epi_act(ep.act, o) : o;
+      }
     }
   }
 }

@@ -7,7 +7,9 @@ fp32 (kernels/lora_mlp/tests/test_lora_mlp.py:507-549, :1348-1456;
 kernels/lora_qkv/tests/test_v2_2_v2_3_v3.py) - where its big GEMMs are plain
 cuBLAS fp32 products.  This module is that path here: every product is
 forge_gemm_generic (fp32 accumulation, one rounding to the storage type, any
-strides, so transposed operands are read in place), the activation is the
+strides, so transposed operands are read in place; aligned fp16 products run
+on the MFMA core there, and those whose tiles leave CUs idle are split over K
+by `gmm`), the activation is the
 SwiGLU / GeGLU kernel and RoPE the RoPE kernel, all in the input's dtype.
 The math is the reference's PyTorch formulation
 (kernels/lora_mlp/reference/lora_mlp_pytorch.py:100-225,
@@ -23,6 +25,7 @@ from typing import Optional
 import torch
 
 from forge_hip import _lib as L
+from kernels._lora_ops import COL, ROW, skinny_split, split_for, split_gemm, split_k_for
 
 GENERIC_DTYPES = (torch.float32, torch.float16)
 
@@ -33,6 +36,76 @@ def check_dtypes(what: str, *ts) -> torch.dtype:
     if len(dts) != 1:
         raise TypeError(f"{what}: tensors must share one dtype, got {sorted(str(d) for d in dts)}")
     return dts.pop()
+
+
+_MAX_PITCH = (1 << 31) // 512 - 1
+
+
+def _mfma_layouts(a: torch.Tensor, b: torch.Tensor):
+    """(a_layout, lda, b_layout, ldb) of a @ b for the MFMA core, or None:
+    fp16 operands that it reads in 16-byte chunks along their unit-stride
+    dimension (the rule of forge_gemm_generic, csrc/gemm_generic.hip)."""
+    M, K = a.shape
+    N = b.shape[1]
+    if a.dtype != torch.float16 or K == 0 or a.data_ptr() % 16 or b.data_ptr() % 16:
+        return None
+    (am, ak), (bk, bn) = a.stride(), b.stride()
+    if ak == 1:
+        al, lda = ROW, am
+    elif am == 1:
+        al, lda = COL, ak
+    else:
+        return None
+    if bk == 1:
+        bl, ldb = COL, bn
+    elif bn == 1:
+        bl, ldb = ROW, bk
+    else:
+        return None
+    if lda % 8 or ldb % 8 or lda > _MAX_PITCH or ldb > _MAX_PITCH:
+        return None
+    if (al == ROW or bl == COL) and K % 8 or al == COL and M % 8 or bl == ROW and N % 8:
+        return None
+    return al, lda, bl, ldb
+
+
+def _split(M: int, N: int, K: int, al: int) -> int:
+    """Split-K factor of one MFMA product: by the rules of the bf16 paths for
+    skinny outputs (rank-r products and gradients) and for big tiles that do
+    not fill the chip."""
+    if al == COL:  # reduced over tokens: A^T B
+        big = M > 64 and N > 64
+        tiles = (-(-M // 256) if M > 64 else 1) * (-(-N // 256) if N > 64 else 1)
+        return split_k_for(K, tiles, target_wgs=256 if big else 512)
+    if N <= 64 and M > N:
+        return skinny_split(M, N, K)
+    if N > 256 and N % 8 == 0 and M > 64:
+        return split_for(M, N, -(-K // 64))
+    return 1
+
+
+def gmm_sum(pairs) -> torch.Tensor:
+    """sum of a @ b over pairs: one product over all of them (one rounding)
+    where the MFMA core takes each in the same layouts, else one product
+    after another, added in the storage type."""
+    lay = [_mfma_layouts(a, b) for a, b in pairs]
+    M, N = pairs[0][0].shape[0], pairs[0][1].shape[1]
+    if M > 0 and N > 0 and all(v is not None and v[0::2] == lay[0][0::2] for v in lay):
+        al, bl = lay[0][0::2]
+        segs = [(a, v[1], b, v[3], a.shape[1]) for (a, b), v in zip(pairs, lay)]
+        out = torch.empty(M, N, dtype=torch.float16, device=pairs[0][0].device)
+        split = _split(M, N, sum(-(-a.shape[1] // 64) * 64 for a, _ in pairs), al)
+        if split > 1:
+            return split_gemm(M, N, segs, al, bl, split, out)
+        arr = (L.GemmSegment * len(segs))(*(L.GemmSegment(a.data_ptr(), lda, b.data_ptr(), ldb, k, 0, 0)
+                                            for a, lda, b, ldb, k in segs))
+        L.check(L.forge_gemm_f16(M, N, arr, len(segs), al, bl, out.data_ptr(), N, L.DTYPE_F16, 1.0, 0.0,
+                                 L.EPI_STORE, 1, L.stream_of(out)), "forge_gemm_f16")
+        return out
+    out = None
+    for a, b in pairs:
+        out = gmm(a, b, out=out, beta=0.0 if out is None else 1.0)
+    return out
 
 
 def gmm(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None, alpha: float = 1.0,
@@ -52,6 +125,11 @@ def gmm(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None, al
             out.mul_(beta)
         return out
     assert out.stride(1) == 1 or N == 1
+    if beta == 0.0 and out.dtype == a.dtype:
+        lay = _mfma_layouts(a, b)
+        split = _split(M, N, K, lay[0]) if lay is not None else 1
+        if split > 1:
+            return split_gemm(M, N, [(a, lay[1], b, lay[3], K)], lay[0], lay[2], split, out, alpha)
     L.check(L.forge_gemm_generic(M, N, K, L.dtype_code(a.dtype), a.data_ptr(), a.stride(0), a.stride(1),
                                  b.data_ptr(), b.stride(0), b.stride(1), out.data_ptr(), out.stride(0),
                                  L.dtype_code(out.dtype), float(alpha), float(beta), None, L.GEMM_ACT_NONE,
@@ -139,8 +217,7 @@ def mlp_backward(dY2, X2, e, g, W_gate, A_gate, B_gate, s_gate, W_up, A_up, B_up
     else:
         xau, xag = gmm(X2, A_up.t()), gmm(X2, A_gate.t())
     dBu, dBg = gmm(df.t(), xau, alpha=s_up), gmm(de.t(), xag, alpha=s_gate)
-    dX = gmm(df, W_up)
-    gmm(de, W_gate, out=dX, beta=1.0)
+    dX = gmm_sum([(df, W_up), (de, W_gate)])
     gmm(vu, A_up, out=dX, alpha=s_up, beta=1.0)
     gmm(vg, A_gate, out=dX, alpha=s_gate, beta=1.0)
     return dX, dAg, dBg, dAu, dBu, dAd, dBd
@@ -178,13 +255,11 @@ def qkv_forward(X2, W_q, W_k, W_v, A_q, B_q, s_q, A_k, B_k, s_k, A_v, B_v, s_v, 
 def qkv_backward(dQ, dK, dV, X2, W_q, W_k, W_v, A_q, B_q, s_q, A_k, B_k, s_k, A_v, B_v, s_v, aux=None):
     """(dX, dA_q, dB_q, dA_k, dB_k, dA_v, dB_v): lora_qkv_pytorch.py:170-214."""
     X2 = _c(X2)
-    dX = None
+    dQ, dK, dV = _c(dQ), _c(dK), _c(dV)
+    dX = gmm_sum([(dQ, W_q), (dK, W_k), (dV, W_v)])
     grads = []
     xas = aux["xa"] if aux and aux.get("generic") else [None, None, None]
-    for dY, W, A, B, s, xa in ((dQ, W_q, A_q, B_q, s_q, xas[0]), (dK, W_k, A_k, B_k, s_k, xas[1]),
-                               (dV, W_v, A_v, B_v, s_v, xas[2])):
-        dY = _c(dY)
-        dX = gmm(dY, W, out=dX, beta=0.0 if dX is None else 1.0)
+    for dY, A, B, s, xa in ((dQ, A_q, B_q, s_q, xas[0]), (dK, A_k, B_k, s_k, xas[1]), (dV, A_v, B_v, s_v, xas[2])):
         dYB = gmm(dY, B)                                    # [M, r]
         gmm(dYB, A, out=dX, alpha=s, beta=1.0)
         xa = xa if xa is not None else gmm(X2, A.t())

@@ -18,6 +18,7 @@ to that check: call clear_caches() after them.
 from __future__ import annotations
 
 import ctypes
+import functools
 import weakref
 from typing import Optional, Sequence, Tuple
 
@@ -63,6 +64,37 @@ def skinny_split(M: int, N: int, K: int, k_contiguous: bool = True) -> int:
     return max(1, min(16, -(-512 // tiles), k_tiles // 4))
 
 
+@functools.lru_cache(maxsize=512)
+def split_for(M: int, N: int, k_tiles: int) -> int:
+    """Split-K factor of an output on 256 x 256 tiles (N > 256) over k_tiles
+    64-deep K tiles: the factor with the least modelled time, 1 unless that
+    saves 10%.
+
+    With fewer tiles than CUs the K loop is a serial chain on a part of the
+    chip; split s ways it is s times shorter on s times the CUs, for s fp32
+    partial outputs written and read once.  Model in us, fitted to MI355X
+    (within 10% of the points below): a K tile costs 1.05 with up to 64
+    workgroups running, 1.45 with 128 and 1.5 with 256 (the clock and the L2
+    traffic per CU), each round of 256 workgroups 8 (12 with an fp32 partial output),
+    the reduction 5 plus its bytes at 5.5 TB/s.  Measured, no split against
+    the factor chosen: [1003, 4096] K = 14336 238 -> 110 us (4), K = 28672 493
+    -> 207 (4); [512, 4096] K = 14336 233 -> 71 (8); [300, 4096] K = 128256
+    2176 -> 402 (8); [2048, 4096] K = 4096 102 -> 78 (2); left whole:
+    [2048, 8192] K = 2048 61 (99 at 2), [1003, 14336] K = 4096 94 (134)."""
+    tiles = -(-M // 256) * -(-N // 256)
+    out_us = M * N * 4 / 5.5e6
+
+    def cost(s: int) -> float:
+        wgs = tiles * s
+        per_tile = 1.05 + 0.4 * min(max((wgs - 64) / 64, 0.0), 1.0) + 0.05 * min(max((wgs - 128) / 128, 0.0), 1.0)
+        t = -(-wgs // 256) * (-(-k_tiles // s) * per_tile + (12 if s > 1 else 8))
+        return t if s == 1 else t + 5 + (s + 0.5) * out_us
+
+    # at least 4 K tiles a split; the partial outputs stay within two rounds of tiles (128 MB)
+    best = min((s for s in range(1, 17) if s == 1 or (k_tiles // s >= 4 and tiles * s <= 512)), key=cost)
+    return best if cost(best) < 0.9 * cost(1) else 1
+
+
 def _segments(segs) -> ctypes.Array:
     """forge_gemm_segment array from (A, lda, B, ldb, K) tuples, optionally
     extended by (n_lo, n_hi): the output columns the segment applies to."""
@@ -80,12 +112,17 @@ def gemm(M: int, N: int, segs: Sequence[Tuple[torch.Tensor, int, torch.Tensor, i
     """C[M, N] = alpha * sum_s A_s @ B_s (+ beta C).  segs: (A, lda, B, ldb, K),
     or (A, lda, B, ldb, K, n_lo, n_hi) for a segment that applies to output
     columns [n_lo, n_hi) only (B's first row is column n_lo).  atomic=True accumulates into a zero-initialised fp32 C over split_k
-    K partitions.  A skinny bf16 output (N <= 64, beta = 0) is split over K
-    into fp32 partial slices, then summed in a fixed order and rounded."""
+    K partitions.  A bf16 output (beta = 0) whose tiles leave CUs idle is
+    split over K into fp32 partial slices, then summed in a fixed order and
+    rounded once."""
     dev = device if device is not None else segs[0][0].device
     K = sum(int(sg[4]) for sg in segs)
-    if not atomic and beta == 0.0 and N <= 64 and M >= 1024 and (out is None or out.dtype == torch.bfloat16):
-        split = skinny_split(M, N, K, a_layout == ROW)
+    if not atomic and split_k == 1 and beta == 0.0 and (out.dtype if out is not None else out_dtype) == torch.bfloat16:
+        split = 1
+        if N <= 64 and M > N:
+            split = skinny_split(M, N, K, a_layout == ROW)
+        elif N > 256 and N % 8 == 0 and M > 64 and all(len(sg) == 5 for sg in segs):
+            split = split_for(M, N, sum(-(-int(sg[4]) // 64) for sg in segs))
         if split > 1:
             if out is None:
                 out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
@@ -111,13 +148,14 @@ def split_gemm(M: int, N: int, segs, a_layout: int, b_layout: int, split: int, o
     """out = alpha * sum_s A_s @ B_s with K split `split` ways: each split
     writes fp32 partials to its slice of a [split, M, N] workspace and
     forge_splitk_reduce sums them in a fixed order (deterministic) and rounds
-    once to out's dtype."""
+    once to out's dtype.  The operands are bf16 or fp16."""
     dev = device if device is not None else out.device
     parts = torch.empty(split, M, N, dtype=torch.float32, device=dev)
     arr = _segments(segs)
     st = L.stream_of(parts)
-    L.check(L.forge_gemm(M, N, arr, len(segs), a_layout, b_layout, parts.data_ptr(), N, L.DTYPE_F32, float(alpha),
-                         0.0, L.EPI_STORE, int(split), st), "forge_gemm")
+    fn = L.forge_gemm_f16 if segs[0][0].dtype == torch.float16 else L.forge_gemm
+    L.check(fn(M, N, arr, len(segs), a_layout, b_layout, parts.data_ptr(), N, L.DTYPE_F32, float(alpha),
+               0.0, L.EPI_STORE, int(split), st), "forge_gemm")
     L.check(L.forge_splitk_reduce(parts.data_ptr(), M * N, int(split), M, N, N, out.data_ptr(), ld(out),
                                   L.dtype_code(out.dtype), 1.0, st), "forge_splitk_reduce")
     return out
@@ -161,7 +199,7 @@ def lora_a(x: torch.Tensor, mats: Sequence[torch.Tensor], scales: Sequence[float
         out = torch.empty(M, n * r, dtype=torch.bfloat16, device=x.device)
     ptrs = (ctypes.c_void_p * n)(*addrs)
     sc = (ctypes.c_float * n)(*[float(s) for s in scales])
-    split = skinny_split(M, n * r, K) if M >= 1024 else 1
+    split = skinny_split(M, n * r, K) if M > n * r else 1
     work = torch.empty(split, M, n * r, dtype=torch.float32, device=x.device) if split > 1 else None
     L.check(
         L.forge_lora_a(M, K, r, n, x.data_ptr(), ld(x), ptrs, lda, sc, out.data_ptr(), ld(out),

@@ -1,0 +1,85 @@
+"""Outputs on 256 x 256 tiles that are split over K (kernels/_lora_ops.py
+split_for, kernels/_generic_lora.py gmm / gmm_sum) and the fp32 epilogue their
+partial slices are stored with.
+
+Oracle: the product in float64; bounds: one rounding to C's type and fp32
+accumulation in any order (K 2^-24 sum |a| |b|)."""
+import pytest
+import torch
+
+from forge_hip import _lib as L
+from kernels._generic_lora import gmm, gmm_sum
+from kernels._lora_ops import COL, ROW, gemm, split_for
+
+U = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}
+
+
+def _close(c, ref, mag, K):
+    bound = U[c.dtype] * ref.abs() * 1.01 + K * 2.0 ** -24 * mag + 1e-7
+    assert ((c.double() - ref).abs() <= bound).all(), ((c.double() - ref).abs() - bound).max().item()
+
+
+def test_split_rule():
+    assert split_for(8192, 4096, 224) == 1 and split_for(2048, 8192, 32) == 1  # the chip is full
+    assert split_for(1003, 4096, 224) == 4
+    for m in (65, 256, 300, 1003, 4096):
+        for n in (264, 4096, 128256):
+            for kt in (1, 3, 64, 2004):
+                s = split_for(m, n, kt)
+                tiles = -(-m // 256) * -(-n // 256)
+                assert s == 1 or (kt // s >= 4 and tiles * s <= 512)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(65, 264, 2048), (256, 512, 1024), (1003, 4096, 4096), (300, 776, 4104)])
+def test_split_products(M, N, K):
+    g = torch.Generator().manual_seed(0)
+    for dtype in (torch.bfloat16, torch.float16):
+        a = torch.randn(M, K, generator=g).to(dtype).cuda()
+        b = torch.randn(N, K, generator=g).to(dtype).cuda()
+        xa = torch.randn(M, 16, generator=g).to(dtype).cuda()
+        bb = torch.randn(N, 16, generator=g).to(dtype).cuda()
+        if dtype == torch.bfloat16:
+            assert split_for(M, N, -(-K // 64) + 1) > 1
+            c = gemm(M, N, [(a, K, b, K, K), (xa, 16, bb, 16, 16)], ROW, COL, alpha=0.5)
+            _close(c, 0.5 * (a.double() @ b.double().t() + xa.double() @ bb.double().t()),
+                   0.5 * (a.double().abs() @ b.double().abs().t() + xa.double().abs() @ bb.double().abs().t()), K + 16)
+        else:
+            _close(gmm(a, b.t(), alpha=0.5), 0.5 * (a.double() @ b.double().t()),
+                   0.5 * (a.double().abs() @ b.double().abs().t()), K)
+            _close(gmm_sum([(a, b.t()), (xa, bb.t())]), a.double() @ b.double().t() + xa.double() @ bb.double().t(),
+                   a.double().abs() @ b.double().abs().t() + xa.double().abs() @ bb.double().abs().t(), K + 16)
+            w, v = b.t().contiguous(), bb.t().contiguous()  # [K, N] as stored
+            _close(gmm_sum([(a, w), (xa, v)]), a.double() @ w.double() + xa.double() @ v.double(),
+                   a.double().abs() @ w.double().abs() + xa.double().abs() @ v.double().abs(), K + 16)
+
+
+@pytest.mark.gpu
+def test_gmm_sum_of_mixed_layouts_adds_products():
+    g = torch.Generator().manual_seed(1)
+    a, b = torch.randn(70, 40, generator=g).half().cuda(), torch.randn(40, 264, generator=g).half().cuda()
+    x, y = torch.randn(70, 12, generator=g).half().cuda(), torch.randn(12, 264, generator=g).half().cuda()  # K % 8 != 0
+    ref = a.double() @ b.double() + x.double() @ y.double()
+    # the first product is rounded to fp16 before the second is added
+    assert ((gmm_sum([(a, b), (x, y)]).double() - ref).abs()
+            <= 2.0 ** -10 * ((a.double() @ b.double()).abs() + ref.abs()) + 1e-4).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(256, 256, 64), (300, 264, 136), (65, 512, 72), (257, 1000, 64)])
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+@pytest.mark.parametrize("pitch", [0, 8, 1])
+def test_fp32_store(M, N, K, beta, pitch):
+    """Whole and ragged tiles, with and without C read, and a pitch that
+    rules out 16-byte stores."""
+    g = torch.Generator().manual_seed(2)
+    a = torch.randn(M, K, generator=g).bfloat16().cuda()
+    b = torch.randn(N, K, generator=g).bfloat16().cuda()
+    buf = torch.randn(M, N + pitch, generator=g).cuda()
+    before = buf.clone()
+    seg = (L.GemmSegment * 1)(L.GemmSegment(a.data_ptr(), K, b.data_ptr(), K, K, 0, 0))
+    L.check(L.forge_gemm(M, N, seg, 1, ROW, COL, buf.data_ptr(), N + pitch, L.DTYPE_F32, 2.0, beta, L.EPI_STORE, 1,
+                         L.stream_of(buf)), "forge_gemm")
+    _close(buf[:, :N], 2.0 * (a.double() @ b.double().t()) + beta * before[:, :N].double(),
+           2.0 * (a.double().abs() @ b.double().abs().t()) + beta * before[:, :N].double().abs(), K)
+    assert torch.equal(buf[:, N:], before[:, N:])
