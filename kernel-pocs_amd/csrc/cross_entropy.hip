@@ -17,9 +17,9 @@
 //     exp(x - m) and keeps p = exp(x - m) as fp16 in place of the input, pass
 //     C writes p/d.  Used for the common case (2-byte logits, no class
 //     weights / softcap / argmax) when the row fits in 512 * 32 * 8 elements.
-//   * ce_stream_kernel: any row length and every feature; the row is streamed
-//     twice (online max/sum, then gradient), the second read largely served by
-//     the L2 / Infinity Cache.
+//   * ce_stream_kernel: any row length, alignment and every feature; the row
+//     is streamed twice (online max/sum, then gradient), the second read
+//     largely served by the Infinity Cache.
 // exp is evaluated as exp2 on log2e-prescaled values (one FMA + v_exp_f32).
 #include <atomic>
 #include <mutex>
@@ -448,123 +448,275 @@ __device__ __forceinline__ bool ce_row_head(CeArgs& a, int64_t row, int64_t y, T
 }
 
 // ---------------------------------------------------------------------------
-// Streaming engine (every feature, any row length)
+// Streaming engine (every feature, any row length and alignment)
+//
+// Two passes over a row: an online max / sum, then the gradient in place (one
+// pass without gradients).  The row is peeled to its first 16-byte boundary,
+// so every length and pitch moves as 16-byte vectors; kStreamU of them are in
+// flight per thread.  Bound by the vector ALU as much as by memory: a softcap
+// row at 16-bit logits costs about 30 issue slots an element, so what the
+// flags switch is a template parameter or a branch per vector, never per
+// element, the divisions by the token count are folded into one scale and
+// shift, and the soft cap is a polynomial (cap_fast).  The second pass reads
+// the Infinity Cache (a bound on the workgroups per CU, so on the rows in
+// flight, measured equal).
+// Measured on MI355X, forward + backward, before -> after the vector ALU work
+// was cut and rows were peeled: bf16 [2048, 256000] softcap 30 1102 -> 490 us,
+// [4096, 151936] 869 -> 530, [8192, 50257] (rows off 16-byte alignment, which
+// went element by element) 1637 -> 372; fp32 [4096, 128256] 1262 -> 866; bf16
+// [8192, 128256] loss, accuracy and predictions 721 -> 412.
 // ---------------------------------------------------------------------------
-constexpr int kStreamBlock = 512;
-constexpr int kStreamWaves = kStreamBlock / 64;
+constexpr int kStreamU = 4;  // vectors in flight per thread
 
-template <class T, int VEC>
-__global__ __launch_bounds__(kStreamBlock) void ce_stream_kernel(CeArgs a) {
-  __shared__ float redf[2 * kStreamWaves];
-  __shared__ int64_t redi[kStreamWaves];
+// sc tanh(x / sc) for 16-bit logits, n values.  |x| <= sc / 2 throughout the
+// vector: x P((x / sc)^2), P the degree-4 Chebyshev fit of tanh(u) / u on
+// u^2 <= 1/4 (relative error 1.1e-7 evaluated in fp32, libm's tanhf 1e-7);
+// else 1 - 2 / (1 + e^2u), whose absolute error of 1.2e-7 sc is far below
+// the 16-bit spacing of such logits.  The choice is per wave.
+template <int N>
+__device__ __forceinline__ void cap_fast(float (&x)[N], float sc, float inv_sc) {
+  float big = 0.f;
+#pragma unroll
+  for (int j = 0; j < N; ++j) big = fmaxf(big, fabsf(x[j]));
+  bool ok = big <= 0.5f * sc;
+#pragma unroll
+  for (int j = 0; j < N; ++j) ok = ok && x[j] == x[j];  // (fmaxf drops NaN)
+  if (__all(ok)) {
+    const float q0 = inv_sc * inv_sc;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float q = x[j] * x[j] * q0;
+      float p = fmaf(q, 0.01714132f, -0.05298924f);
+      p = fmaf(q, p, 0.13324829f);
+      p = fmaf(q, p, -0.33333072f);
+      p = fmaf(q, p, 0.99999999f);
+      x[j] *= p;
+    }
+  } else {
+    const float k = 2.f * kLog2e * inv_sc;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      x[j] = fmaf(-2.f * sc, __builtin_amdgcn_rcpf(1.f + fast_exp2(x[j] * k)), sc);
+  }
+}
+
+// Soft cap of a vector (fp32 logits keep libm's tanhf).
+template <bool EXACT, int N>
+__device__ __forceinline__ void cap(float (&x)[N], float sc, float inv_sc) {
+  if constexpr (EXACT) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) x[j] = sc * tanhf(x[j] / sc);
+  } else {
+    cap_fast<N>(x, sc, inv_sc);
+  }
+}
+
+template <class T, int NT, bool SC, bool W, bool ARG>
+__global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
+  constexpr int VEC = 16 / sizeof(T), NW = NT / 64, U = kStreamU;
+  constexpr bool EXACT = sizeof(T) == 4;
+  __shared__ float redf[2 * NW];
+  __shared__ int64_t redi[NW];
   const int64_t row = blockIdx.x;
   const int64_t y = a.target[row * a.target_stride];
   T* xr = (T*)a.x + row * a.ld;
   const int64_t V = a.n_cols;
-  const bool vec = VEC > 1;
-  if (ce_row_head<T, kStreamBlock>(a, row, y, xr, vec, redf)) return;
+  const int tid = threadIdx.x;
+  // elements before the first 16-byte boundary and after the last one: one
+  // thread each (at most 2 VEC - 2 of them)
+  const int64_t pre = (int64_t)(((16 - (reinterpret_cast<uintptr_t>(xr) & 15)) & 15) / sizeof(T));
+  const int64_t head = pre < V ? pre : V;
+  const int64_t nvec = (V - head) / VEC;
+  const int edge = (int)(V - nvec * VEC);
+  const int64_t ecol = tid < head ? tid : nvec * VEC + tid;  // column of this thread's edge element (tid < edge)
+  T* xv = xr + head;
+  if (ce_row_head<T, NT>(a, row, y, xr, pre == 0 && V % VEC == 0, redf)) return;
 
-  const bool has_w = a.flags & FORGE_CE_HAS_WEIGHT;
-  const bool has_sc = a.flags & FORGE_CE_HAS_SOFTCAP;
-  const bool need_arg = a.flags & (FORGE_CE_RETURN_ACCURACY | FORGE_CE_RETURN_PREDICTED);
   const bool grads = a.flags & FORGE_CE_HAS_GRADIENTS;
-  const float sc = a.softcap;
+  const float sc = a.softcap, inv_sc = SC ? 1.f / sc : 0.f;
   const float ls = a.label_smoothing;
   const float eps = ls / (float)V;
-  const float wy = has_w ? a.weight[y] : 1.f;
-  float xy = to_f32(xr[y]);
-  if (has_sc) xy = sc * tanhf(xy / sc);
+  const float wy = W ? a.weight[y] : 1.f;
+  float xy1[1] = {to_f32(xr[y])};
+  if constexpr (SC) cap<EXACT, 1>(xy1, sc, inv_sc);
+  const float xy = xy1[0];
 
   // ---- pass 1: online max / sum (log2 domain), argmax, smoothing sum ----
-  float m = -INFINITY, d = 0.f, sxs = 0.f, amax_v = -INFINITY;
+  // A 16-bit softcap row needs no max: |v| <= sc, and for sc <= 40 every
+  // exp(v - sc) is a normal fp32 number.
+  const bool bounded = SC && !EXACT && sc <= 40.f;
+  float m = bounded ? sc * kLog2e : -INFINITY, d = 0.f, sxs = 0.f, amax_v = -INFINITY;
   int64_t amax_i = V;
-  for (int64_t c0 = (int64_t)threadIdx.x * VEC; c0 < V; c0 += (int64_t)kStreamBlock * VEC) {
-    float v[VEC];
-    if constexpr (VEC > 1) {
-      Vec16<T> raw = load16(xr + c0);
+  auto pass1 = [&](auto& v, int64_t c0) {
+    constexpr int N = sizeof(v) / sizeof(float);
+    if constexpr (ARG) {
+      // the first vector that holds this thread's largest logit (its place in
+      // the vector is looked up after the pass).  Logits are compared before a
+      // fast cap, whose order they share (see below), and after an exact one.
+      if constexpr (SC && EXACT) cap<EXACT, N>(v, sc, inv_sc);
+      float t = v[0];
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) v[j] = to_f32(raw.v[j]);
-    } else {
-      v[0] = to_f32(xr[c0]);
+      for (int j = 1; j < N; ++j) t = fmaxf(t, v[j]);
+      if (t > amax_v) { amax_v = t; amax_i = c0; }
     }
-    float vm = -INFINITY;
+    if constexpr (SC && !(ARG && EXACT)) cap<EXACT, N>(v, sc, inv_sc);
+    if (ls > 0.f) {
+      float t = 0.f;
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) {
-      if (has_sc) v[j] = sc * tanhf(v[j] / sc);
-      if (need_arg && v[j] > amax_v) { amax_v = v[j]; amax_i = c0 + j; }
-      if (ls > 0.f) sxs += has_w ? -eps * v[j] * a.weight[c0 + j] : -eps * v[j];
-      v[j] *= kLog2e;
-      vm = fmaxf(vm, v[j]);
+      for (int j = 0; j < N; ++j) t += W ? v[j] * a.weight[c0 + j] : v[j];
+      sxs += t;
     }
-    if (vm > m) {
-      d = (m == -INFINITY) ? 0.f : d * fast_exp2(m - vm);
-      m = vm;
+    if (!bounded) {
+      float vm = v[0];
+#pragma unroll
+      for (int j = 1; j < N; ++j) vm = fmaxf(vm, v[j]);
+      vm *= kLog2e;
+      if (vm > m) {
+        d = (m == -INFINITY) ? 0.f : d * fast_exp2(m - vm);
+        m = vm;
+      }
     }
     if (m != -INFINITY) {
+      float t = 0.f;
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) d += fast_exp2(v[j] - m);
+      for (int j = 0; j < N; ++j) t += fast_exp2(fmaf(v[j], kLog2e, -m));
+      d += t;
+    }
+  };
+  auto unpack = [&](const Vec16<T>& raw, float (&v)[VEC]) {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) v[j] = to_f32(raw.v[j]);
+  };
+  // f(vector, its index) over the row's vectors, U loads in flight
+  auto each = [&](auto load, auto f) {
+    int64_t i0 = 0;
+    for (; i0 + (int64_t)NT * U <= nvec; i0 += (int64_t)NT * U) {
+      Vec16<T> raw[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) raw[u] = load(xv + (i0 + u * NT + tid) * VEC);
+#pragma unroll
+      for (int u = 0; u < U; ++u) f(raw[u], i0 + u * NT + tid);
+    }
+    for (int64_t i = i0 + tid; i < nvec; i += NT) f(load(xv + i * VEC), i);
+  };
+  auto fwd = [&](const Vec16<T>& raw, int64_t i) {
+    float v[VEC];
+    unpack(raw, v);
+    pass1(v, head + i * VEC);
+  };
+  if (tid < edge && tid < head) {
+    float v[1] = {to_f32(xr[ecol])};
+    pass1(v, ecol);
+  }
+  if (grads) each([](const T* p) { return load16(p); }, fwd);  // read again below: kept cached
+  else each([](const T* p) { return load16_nt(p); }, fwd);
+  if (tid < edge && tid >= head) {
+    float v[1] = {to_f32(xr[ecol])};
+    pass1(v, ecol);
+  }
+  block_lse<NW>(m, d, redf);
+  float sxs_tot = 0.f;
+  if (ls > 0.f) sxs_tot = -eps * block_sum<NW>(sxs, redf);
+  int64_t amax = 0;
+  if constexpr (ARG) {
+    if (amax_i >= head && amax_i < head + nvec * VEC) {  // a vector: its first element with that value
+      float v[VEC];
+      unpack(load16(xr + amax_i), v);
+      if constexpr (SC && EXACT) cap<EXACT, VEC>(v, sc, inv_sc);
+      int j0 = 0;
+#pragma unroll
+      for (int j = VEC - 1; j >= 0; --j)
+        if (v[j] == amax_v) j0 = j;
+      amax_i += j0;
+    }
+    amax = block_argmax<NW>(amax_v, amax_i, redf, redi);
+    if constexpr (SC && !EXACT) {
+      // The argmax is the first of the largest CAPPED values.  Up to 4 sc the
+      // cap is strictly increasing over 16-bit logits (neighbours are 2^-11
+      // apart or more, 40 fp32 ulps after the cap), so the largest logit is
+      // the one; past it distinct logits may cap to one value, and the row is
+      // searched again with the exact cap.
+      const float top = block_max<NW>(amax_v, redf);
+      if (!(fabsf(top) <= 4.f * sc)) {
+        amax_v = -INFINITY;
+        amax_i = V;
+        for (int64_t c = tid; c < V; c += NT) {
+          const float v = sc * tanhf(to_f32(xr[c]) / sc);
+          if (v > amax_v) { amax_v = v; amax_i = c; }
+        }
+        amax = block_argmax<NW>(amax_v, amax_i, redf, redi);
+      }
     }
   }
-  block_lse<kStreamWaves>(m, d, redf);
-  float sxs_tot = 0.f;
-  if (ls > 0.f) sxs_tot = block_sum<kStreamWaves>(sxs, redf);
-  int64_t amax = 0;
-  if (need_arg) amax = block_argmax<kStreamWaves>(amax_v, amax_i, redf, redi);
   // natural-log lse: m is log2-scaled
-  const float lse = (m + __log2f(d)) * kLn2;
-  const bool ok = a.il.word ? il_stats<kStreamBlock>(a) : true;
-  if (threadIdx.x == 0) write_row_outputs(a, row, y, lse, xy, wy, sxs_tot, amax, ok);
+  const float m2 = m + __log2f(d);  // exp2(v*log2e - m2) = softmax
+  const float lse = m2 * kLn2;
+  const bool ok = a.il.word ? il_stats<NT>(a) : true;
+  if (tid == 0) write_row_outputs(a, row, y, lse, xy, wy, sxs_tot, amax, ok);
 
   // ---- pass 2: gradient in place ----
   if (grads && ok) {
     const bool mean = a.flags & FORGE_CE_REDUCTION_MEAN;
-    const float lss = a.lse_square_scale;
-    const float m2 = m + __log2f(d);  // exp2(v*log2e - m2) = softmax
-    const float inv_n = 1.f / a.n_non_ignore;
-    const float inv_snw = 1.f / a.sum_non_ignore_weight;
-    for (int64_t c0 = (int64_t)threadIdx.x * VEC; c0 < V; c0 += (int64_t)kStreamBlock * VEC) {
-      float v[VEC], th[VEC];
-      if constexpr (VEC > 1) {
-        Vec16<T> raw = load16(xr + c0);
+    const float inv_n = mean ? 1.f / a.n_non_ignore : 1.f;
+    const float inv_snw = mean ? 1.f / a.sum_non_ignore_weight : 1.f;
+    const float dz = 2.f * a.lse_square_scale * lse;
+    // without class weights: g = p scale - shift, less ydelta at the target
+    const float scale = (1.f + dz) * inv_n, shift = eps * inv_n, ydelta = (1.f - ls) * inv_n;
+    const float dy = W ? (1.f - ls) * wy * inv_snw : ydelta;
+    auto pass2 = [&](auto& v, int64_t c0) {
+      constexpr int N = sizeof(v) / sizeof(float);
+      float th[N];  // tanh(x / sc), for the cap's slope 1 - th^2
+      if constexpr (SC && EXACT) {
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) v[j] = to_f32(raw.v[j]);
-      } else {
-        v[0] = to_f32(xr[c0]);
-      }
-      float g[VEC];
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) {
-        if (has_sc) { th[j] = tanhf(v[j] / sc); v[j] = sc * th[j]; }
-        const float p = fast_exp2(fmaf(v[j], kLog2e, -m2));
-        const bool is_y = (c0 + j) == y;
-        if (!has_w) {
-          float t = p + 2.f * lss * lse * p;
-          t += -eps;
-          if (is_y) t -= (1.f - ls);
-          if (mean) t = t / a.n_non_ignore;
-          g[j] = t;
-        } else {
-          float ori = (1.f - ls) * p;
-          if (is_y) ori -= (1.f - ls);
-          ori *= wy;
-          float smooth = eps * (-a.weight[c0 + j] + p * a.weight_sum);
-          float dz = 2.f * lss * lse * p;
-          if (mean) { ori *= inv_snw; smooth *= inv_snw; dz *= inv_n; }
-          g[j] = ori + smooth + dz;
+        for (int j = 0; j < N; ++j) {
+          th[j] = tanhf(v[j] / sc);
+          v[j] = sc * th[j];
         }
-        if (has_sc) g[j] *= (1.f - th[j] * th[j]);
-      }
-      if constexpr (VEC > 1) {
-        Vec16<T> o;
+      } else if constexpr (SC) {
+        cap_fast<N>(v, sc, inv_sc);
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) o.v[j] = from_f32<T>(g[j]);
-        store16(xr + c0, o);
-      } else {
-        xr[c0] = from_f32<T>(g[0]);
+        for (int j = 0; j < N; ++j) th[j] = v[j] * inv_sc;
       }
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const float p = fast_exp2(fmaf(v[j], kLog2e, -m2));
+        float g;
+        if constexpr (!W) {
+          g = fmaf(p, scale, -shift);
+        } else {
+          const float ori = (1.f - ls) * p * wy;
+          const float smooth = eps * (-a.weight[c0 + j] + p * a.weight_sum);
+          g = ori * inv_snw + smooth * inv_snw + dz * p * inv_n;
+        }
+        if constexpr (SC) {
+          th[j] = 1.f - th[j] * th[j];
+          g *= th[j];
+        }
+        v[j] = g;
+      }
+      if (const int64_t at = y - c0; at >= 0 && at < N) {  // the vector that holds the target
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          if (j == (int)at) v[j] -= SC ? dy * th[j] : dy;
+      }
+    };
+    each([](const T* p) { return load16_nt(p); },
+         [&](const Vec16<T>& raw, int64_t i) {
+           float v[VEC];
+           unpack(raw, v);
+           pass2(v, head + i * VEC);
+           Vec16<T> o;
+#pragma unroll
+           for (int j = 0; j < VEC; ++j) o.v[j] = from_f32<T>(v[j]);
+           store16_nt(xv + i * VEC, o);
+         });
+    if (tid < edge) {
+      float v[1] = {to_f32(xr[ecol])};
+      pass2(v, ecol);
+      xr[ecol] = from_f32<T>(v[0]);
     }
   }
-  if (a.il.loss_sum) il_last_sum<kStreamWaves>(a, row, redf);
+  if (a.il.loss_sum) il_last_sum<NW>(a, row, redf);
 }
 
 // ---------------------------------------------------------------------------
@@ -782,6 +934,33 @@ void ce_resident_kernel(CeArgs a) {
   if (a.il.loss_sum) il_last_sum<kResWaves>(a, row, redf);
 }
 
+template <class T, bool SC, bool W>
+void launch_stream_sw(const CeArgs& a, dim3 grid, hipStream_t s) {
+  // Long rows take 1024 threads: half the rows in flight, which the second
+  // pass still finds in the Infinity Cache.  Measured on MI355X, 512 against
+  // 1024 threads: [2048, 256000] fp32 1040 / 898 us, [4096, 128256] fp32 890
+  // / 866, [4096, 151936] bf16 550 / 532, [8192, 50257] bf16 386 / 392.  With
+  // a softcap the arithmetic holds the kernel and the smaller workgroups'
+  // barriers cost less: [2048, 256000] bf16 494 / 519, [4096, 32000] 146 / 184.
+  const bool wide = !SC && a.n_cols * (int64_t)sizeof(T) >= 256 * 1024;
+  if (a.flags & (FORGE_CE_RETURN_ACCURACY | FORGE_CE_RETURN_PREDICTED)) {
+    if (wide) ce_stream_kernel<T, 1024, SC, W, true><<<grid, 1024, 0, s>>>(a);
+    else ce_stream_kernel<T, 512, SC, W, true><<<grid, 512, 0, s>>>(a);
+  } else {
+    if (wide) ce_stream_kernel<T, 1024, SC, W, false><<<grid, 1024, 0, s>>>(a);
+    else ce_stream_kernel<T, 512, SC, W, false><<<grid, 512, 0, s>>>(a);
+  }
+}
+
+template <class T>
+void launch_stream(const CeArgs& a, dim3 grid, hipStream_t s) {
+  const bool sc = a.flags & FORGE_CE_HAS_SOFTCAP, w = a.flags & FORGE_CE_HAS_WEIGHT;
+  if (sc && w) launch_stream_sw<T, true, true>(a, grid, s);
+  else if (sc) launch_stream_sw<T, true, false>(a, grid, s);
+  else if (w) launch_stream_sw<T, false, true>(a, grid, s);
+  else launch_stream_sw<T, false, false>(a, grid, s);
+}
+
 template <class T>
 int launch_ce(CeArgs a, hipStream_t s) {
   constexpr int V = 16 / sizeof(T);
@@ -804,12 +983,7 @@ int launch_ce(CeArgs a, hipStream_t s) {
         ce_resident_kernel<T, kResNRMax><<<grid, kResBlock, 0, s>>>(a);
     }
   }
-  if (resident) {
-  } else if (vec) {
-    ce_stream_kernel<T, V><<<grid, kStreamBlock, 0, s>>>(a);
-  } else {
-    ce_stream_kernel<T, 1><<<grid, kStreamBlock, 0, s>>>(a);
-  }
+  if (!resident) launch_stream<T>(a, grid, s);
   FORGE_CHECK_LAUNCH();
   return FORGE_OK;
 }

@@ -1,0 +1,125 @@
+"""The streaming cross-entropy engine where it can go wrong: rows that start
+and end off a 16-byte boundary, rows shorter than one vector or one pass of
+the workgroup, both workgroup sizes, the polynomial soft cap against its
+exponential form, argmax ties after saturation, and rows of infinities and
+NaN.
+
+Oracle: float64 torch.  Bounds: one rounding of the gradient to the logits'
+type (2^-8, 2^-11, 2^-24 of it) and an fp32 exponent error of a few 2^-24 of
+|x log2 e| <= 100, so 1e-5 of p."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from kernels.cross_entropy.experiments.v2 import forge_cross_entropy
+
+U = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}
+
+
+def _rows(n, V, dtype, pitch, offset, std, gen):
+    """[n, V] logits in a buffer of the given pitch, `offset` elements in."""
+    buf = torch.zeros(n * pitch + offset + 8, dtype=dtype, device="cuda")
+    x = buf[offset:offset + n * pitch].view(n, pitch)[:, :V]
+    x.copy_((torch.randn(n, V, generator=gen) * std).to(dtype))
+    return buf, x
+
+
+def _reference(x, t, softcap, smoothing, weight):
+    z = x.double().requires_grad_(True)
+    v = softcap * torch.tanh(z / softcap) if softcap else z
+    loss = F.cross_entropy(v, t, ignore_index=-100, label_smoothing=smoothing,
+                           weight=weight.double() if weight is not None else None)
+    return loss.detach(), torch.autograd.grad(loss, z)[0], v.detach()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("V,pitch,offset", [(1, 1, 0), (5, 5, 3), (13, 16, 1), (1003, 1003, 0), (4099, 4104, 5),
+                                            (8192, 8192, 1), (16391, 16391, 2)])
+@pytest.mark.parametrize("softcap,smoothing,weighted", [(None, 0.0, False), (30.0, 0.0, False), (None, 0.1, False),
+                                                        (30.0, 0.1, True), (3.0, 0.0, False), (50.0, 0.1, False)])
+def test_ragged_rows(dtype, V, pitch, offset, softcap, smoothing, weighted):
+    gen = torch.Generator().manual_seed(V + offset)
+    n = 7
+    buf, x = _rows(n, V, dtype, pitch, offset, 4.0, gen)
+    before = buf.clone()
+    t = torch.randint(0, V, (n,), generator=gen).cuda()
+    t[0], t[1] = 0, V - 1
+    t[3] = -100
+    w = torch.rand(V, generator=gen).cuda() + 0.5 if weighted else None
+    loss, grad, v = _reference(x, t, softcap, smoothing, w)
+    leaf = x.detach().requires_grad_(True)
+    got = forge_cross_entropy(leaf, t, weight=w, softcap=softcap, label_smoothing=smoothing)
+    assert abs(got.double() - loss) <= U[dtype] * abs(loss) + 2e-6 * (1 + v.abs().max())
+    p = torch.softmax(v, -1) / 6 * (1.5 if weighted else 1.0)
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 1e-9
+    # (2^-22 of p - onehot: the cap's slope 1 - tanh^2, with tanh good to 2^-23)
+    near = p.scatter(1, t.clamp(min=0)[:, None], 1.5 / 6 if weighted else 1 / 6)
+    bound = U[dtype] * grad.abs() * 1.01 + 2e-5 * p + 2.0 ** -22 * near + tiny
+    assert ((x.double() - grad).abs() <= bound).all()
+    outside = torch.ones_like(buf, dtype=torch.bool)
+    outside[offset:offset + n * pitch].view(n, pitch)[:, :V] = False
+    assert torch.equal(buf[outside], before[outside])  # neighbours of the rows untouched
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 140001), (torch.float32, 70003), (torch.bfloat16, 262144)])
+@pytest.mark.parametrize("evaluate", [False, True])
+def test_long_rows(dtype, V, evaluate):
+    gen = torch.Generator().manual_seed(V)
+    _, x = _rows(3, V, dtype, V, 0, 3.0, gen)
+    t = torch.randint(0, V, (3,), generator=gen).cuda()
+    loss, grad, v = _reference(x, t, None, 0.0, None)
+    if evaluate:
+        t[1] = v[1].argmax()
+        o = forge_cross_entropy(x.clone(), t, return_token_accuracy=True, return_predicted_tokens=True)
+        first = (x == x.amax(-1, keepdim=True)).int().argmax(-1)
+        assert torch.equal(o.predicted_tokens, first)
+        assert abs(o.token_accuracy.item() - (first == t).float().mean().item()) < 1e-6
+        return
+    got = forge_cross_entropy(x.requires_grad_(True), t)
+    assert abs(got.double() - loss) <= U[dtype] * abs(loss) + 1e-5
+    x = x.detach()
+    assert ((x.double() - grad).abs() <= U[dtype] * grad.abs() * 1.01 + 2e-5 * torch.softmax(v, -1) / 3 + 1e-12).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("level", [0.5, 3.9, 4.5, 40.0, -40.0])
+def test_softcap_argmax(dtype, level):
+    """The prediction is the first of the largest capped values in the
+    logits' fp32 cap, saturated ones included."""
+    gen = torch.Generator().manual_seed(5)
+    V, sc = 3001, 30.0
+    x = (torch.randn(4, V, generator=gen) + level * sc).to(dtype).cuda()
+    x[0, 7] = x[0, 100] = x[0].max()
+    t = torch.zeros(4, dtype=torch.int64, device="cuda")
+    o = forge_cross_entropy(x, t, softcap=sc, return_predicted_tokens=True)
+    capped = sc * torch.tanh(x.float() / sc)
+    best = capped.gather(1, o.predicted_tokens[:, None])[:, 0]
+    # torch's fp32 tanh may differ from the kernel's by an ulp
+    assert (best >= capped.amax(-1) * (1 - 2.0 ** -22 * (1 if level > 0 else -1))).all()
+    if abs(level) >= 40:  # every value caps to +-sc: the first column
+        assert (o.predicted_tokens == 0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("softcap", [None, 30.0])
+def test_infinities_and_nan(dtype, softcap):
+    V = 2053
+    gen = torch.Generator().manual_seed(6)
+    x = torch.randn(4, V, generator=gen).to(dtype).cuda()
+    x[1, 5:900] = -float("inf")  # masked columns
+    x[2, 11] = float("nan")
+    if softcap:
+        x[3, 17] = float("inf")  # caps to softcap
+    t = torch.tensor([1, 2, 3, 17], device="cuda")
+    ref = x.double()
+    v = softcap * torch.tanh(ref / softcap) if softcap else ref
+    logp = torch.log_softmax(v, -1)
+    o = forge_cross_entropy(x.clone().requires_grad_(True), t, softcap=softcap, reduction="none")
+    want = -logp.gather(1, t[:, None])[:, 0]
+    assert torch.isnan(o[2]) and torch.isnan(want[2])
+    keep = torch.tensor([0, 1, 3], device="cuda")
+    assert ((o[keep].double() - want[keep]).abs() <= U[dtype] * want[keep].abs() + 1e-5).all()
