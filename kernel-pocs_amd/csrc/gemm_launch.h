@@ -28,6 +28,18 @@ int launch_atomic_f32(int cfg, int al, int bl, const GemmArgs& a, hipStream_t s)
 int launch_glu_fwd(int epi, int al, int bl, const GemmArgs& a, hipStream_t s);
 int launch_glu_bwd(int epi, int al, int bl, const GemmArgs& a, hipStream_t s);
 int launch_rope(const GemmArgs& a, hipStream_t s);
+int launch_rows(int epi, const GemmArgs& a, hipStream_t s);  // few rows, K-contiguous operands
+
+// Few rows against K-contiguous weights: the row engine (gemm_rows.hip).  Up
+// to 32 rows of a plain product (43 us at 32 rows, K = 14336, N = 4096; 256 x
+// 256 tiles split over K take 45 at any row count up to 128, the row engine 77
+// at 64) and 64 of a gate/up product (80 us; 256 x 256 tiles 94, the row
+// engine 172 at 128).
+inline bool rows_engine(int epi, const GemmArgs& a) {
+  if (a.split_k != 1 || a.N <= a.M) return false;
+  if (epi == EPI_STORE_BF16) return a.M <= 32;
+  return glu_fwd_epi(epi) && a.M <= 64 && !a.ep.vpart && !a.f16;
+}
 int launch_f16(int epi, int cfg, int al, int bl, const GemmArgs& a, hipStream_t s);  // fp16 operands
 
 #ifndef SKINNY_NSTAGE

@@ -69,7 +69,7 @@ def _mfma_layouts(a: torch.Tensor, b: torch.Tensor):
     return al, lda, bl, ldb
 
 
-def _split(M: int, N: int, K: int, al: int) -> int:
+def _split(M: int, N: int, K: int, al: int, bl: int) -> int:
     """Split-K factor of one MFMA product: by the rules of the bf16 paths for
     skinny outputs (rank-r products and gradients) and for big tiles that do
     not fill the chip."""
@@ -79,7 +79,7 @@ def _split(M: int, N: int, K: int, al: int) -> int:
         return split_k_for(K, tiles, target_wgs=256 if big else 512)
     if N <= 64 and M > N:
         return skinny_split(M, N, K)
-    if N > 256 and N % 8 == 0 and M > 64:
+    if N > 256 and N % 8 == 0 and (M > 64 or M > 32 and bl == COL):
         return split_for(M, N, -(-K // 64))
     return 1
 
@@ -94,7 +94,7 @@ def gmm_sum(pairs) -> torch.Tensor:
         al, bl = lay[0][0::2]
         segs = [(a, v[1], b, v[3], a.shape[1]) for (a, b), v in zip(pairs, lay)]
         out = torch.empty(M, N, dtype=torch.float16, device=pairs[0][0].device)
-        split = _split(M, N, sum(-(-a.shape[1] // 64) * 64 for a, _ in pairs), al)
+        split = _split(M, N, sum(-(-a.shape[1] // 64) * 64 for a, _ in pairs), al, bl)
         if split > 1:
             return split_gemm(M, N, segs, al, bl, split, out)
         arr = (L.GemmSegment * len(segs))(*(L.GemmSegment(a.data_ptr(), lda, b.data_ptr(), ldb, k, 0, 0)
@@ -127,7 +127,7 @@ def gmm(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None, al
     assert out.stride(1) == 1 or N == 1
     if beta == 0.0 and out.dtype == a.dtype:
         lay = _mfma_layouts(a, b)
-        split = _split(M, N, K, lay[0]) if lay is not None else 1
+        split = _split(M, N, K, lay[0], lay[2]) if lay is not None else 1
         if split > 1:
             return split_gemm(M, N, [(a, lay[1], b, lay[3], K)], lay[0], lay[2], split, out, alpha)
     L.check(L.forge_gemm_generic(M, N, K, L.dtype_code(a.dtype), a.data_ptr(), a.stride(0), a.stride(1),

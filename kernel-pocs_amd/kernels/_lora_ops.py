@@ -121,7 +121,8 @@ def gemm(M: int, N: int, segs: Sequence[Tuple[torch.Tensor, int, torch.Tensor, i
         split = 1
         if N <= 64 and M > N:
             split = skinny_split(M, N, K, a_layout == ROW)
-        elif N > 256 and N % 8 == 0 and M > 64 and all(len(sg) == 5 for sg in segs):
+        elif N > 256 and N % 8 == 0 and (M > 64 or M > 32 and (a_layout, b_layout) == (ROW, COL)) and \
+                all(len(sg) == 5 for sg in segs):
             split = split_for(M, N, sum(-(-int(sg[4]) // 64) for sg in segs))
         if split > 1:
             if out is None:

@@ -1,0 +1,80 @@
+"""The few-rows GEMM engine (csrc/gemm_rows.hip) at its edges: 1 to 64 rows
+around each block of 16, columns and K that are not whole tiles, K shorter
+than one chunk and long enough that every wave has several, column-ranged
+segments, the gate/up product with LoRA segments that share one K range, and
+the row counts just past it.
+
+Oracle: the product in float64; bound: one rounding to C's type and fp32
+accumulation in any order (K 2^-24 sum |a| |b|); the gated activation carries
+the bound of its two factors."""
+import pytest
+import torch
+
+from forge_hip import _lib as L
+from kernels._lora_ops import COL, ROW, gemm
+
+U = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _mat(rows, cols, gen, dtype=torch.bfloat16, pad=0):
+    t = torch.randn(rows, cols + pad, generator=gen).to(dtype).cuda()
+    return t[:, :cols]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K,pad", [(72, 8, 0), (1000, 264, 8), (1040, 4104, 0), (2056, 72, 16)])
+def test_rows(dtype, M, N, K, pad):
+    gen = torch.Generator().manual_seed(M * N)
+    a, b = _mat(M, K, gen, dtype, pad), _mat(N, K, gen, dtype)
+    c = torch.randn(M, N, generator=gen).to(dtype).cuda()
+    ref = 0.5 * (a.double() @ b.double().t()) + 2.0 * c.double()
+    seg = (L.GemmSegment * 1)(L.GemmSegment(a.data_ptr(), a.stride(0), b.data_ptr(), K, K, 0, 0))
+    fn = L.forge_gemm_f16 if dtype == torch.float16 else L.forge_gemm
+    L.check(fn(M, N, seg, 1, ROW, COL, c.data_ptr(), N, L.dtype_code(dtype), 0.5, 2.0, L.EPI_STORE, 1,
+               L.stream_of(c)), "forge_gemm")
+    bound = U[dtype] * ref.abs() * 1.01 + K * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t()) + 1e-6
+    assert ((c.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [3, 20])
+def test_column_ranges(M):
+    """Segments that cover columns [0, 40), [40, 100) and all of them; ranges
+    that start and end inside a block of 16 columns."""
+    gen = torch.Generator().manual_seed(M)
+    N, K = 100, 320
+    a, x, y, z = _mat(M, K, gen), _mat(40, K, gen), _mat(60, K, gen), _mat(N, 16, gen)
+    t = _mat(M, 16, gen)
+    c = gemm(M, N, [(a, K, x, K, K, 0, 40), (a, K, y, K, K, 40, 100), (t, 16, z, 16, 16)], ROW, COL)
+    w = torch.cat([x, y]).double()
+    ref = a.double() @ w.t() + t.double() @ z.double().t()
+    mag = a.double().abs() @ w.abs().t() + t.double().abs() @ z.double().abs().t()
+    assert ((c.double() - ref).abs() <= 2.0 ** -8 * 1.01 * ref.abs() + K * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 16, 31, 48, 64, 65])
+@pytest.mark.parametrize("H,I,r", [(256, 264, 0), (264, 4136, 8), (2048, 4104, 24), (64, 512, 64)])
+@pytest.mark.parametrize("act", [L.ACT_SILU, L.ACT_GELU_TANH, L.ACT_GELU_ERF])
+def test_gate_up(M, H, I, r, act):
+    gen = torch.Generator().manual_seed(M + I)
+    x, wg, wu = _mat(M, H, gen), _mat(I, H, gen) * H ** -0.5, _mat(I, H, gen) * H ** -0.5
+    xa, bg, bu = _mat(M, 2 * max(r, 8), gen), _mat(I, max(r, 8), gen), _mat(I, max(r, 8), gen)
+    e, g, h = (torch.empty(M, I, dtype=torch.bfloat16, device="cuda") for _ in range(3))
+    args = (M, H, I, r, x.data_ptr(), H, wg.data_ptr(), wu.data_ptr(), H, xa.data_ptr() if r else None, 2 * r,
+            bg.data_ptr() if r else None, bu.data_ptr() if r else None, r)
+    L.check(L.forge_lora_mlp_gate_up(*args, e.data_ptr(), g.data_ptr(), h.data_ptr(), I, act, L.stream_of(x)), "gate_up")
+    re, rg = x.double() @ wg.double().t(), x.double() @ wu.double().t()
+    if r:
+        re, rg = re + xa[:, :r].double() @ bg.double().t(), rg + xa[:, r:].double() @ bu.double().t()
+    for got, ref in ((e, re), (g, rg)):
+        assert ((got.double() - ref).abs() <= 2.0 ** -8 * 1.01 * ref.abs() + 1e-4).all()
+    a = {L.ACT_SILU: torch.nn.functional.silu(re), L.ACT_GELU_TANH: torch.nn.functional.gelu(re, approximate="tanh"),
+         L.ACT_GELU_ERF: torch.nn.functional.gelu(re)}[act]
+    # GELU forms round e, g and the activation first: four roundings of at most 2^-8, slope of the activation <= 1.13
+    assert ((h.double() - a * rg).abs() <= 4.6 * 2.0 ** -8 * (a.abs() + re.abs() * 0.3) * rg.abs() + 1e-3).all()
+    h2 = torch.empty_like(h)  # inference: h alone
+    L.check(L.forge_lora_mlp_gate_up(*args, None, None, h2.data_ptr(), I, act, L.stream_of(x)), "gate_up")
+    assert torch.equal(h, h2)
