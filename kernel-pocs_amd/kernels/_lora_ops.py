@@ -232,7 +232,15 @@ def frozen_t(w: torch.Tensor, pitch_multiple: int = 1) -> torch.Tensor:
             return wt
     n_out = w.shape[0]
     pad = -(-n_out // pitch_multiple) * pitch_multiple
-    if pad == n_out:
+    if w.is_cuda and w.element_size() == 2 and w.stride(1) == 1 and w.stride(0) >= w.shape[1]:
+        # (torch's strided copy reads a [14336, 4096] bf16 weight at 0.95 TB/s:
+        # 246 us on MI355X against 47 here; a first pass makes one per weight)
+        wt = torch.empty(w.shape[1], pad, dtype=w.dtype, device=w.device)
+        if pad != n_out:
+            wt[:, n_out:].zero_()
+        L.check(L.forge_transpose_2b(w.data_ptr(), w.stride(0), n_out, w.shape[1], wt.data_ptr(), pad, L.stream_of(w)),
+                "forge_transpose_2b")
+    elif pad == n_out:
         wt = w.detach().t().contiguous()
     else:
         wt = torch.zeros(w.shape[1], pad, dtype=w.dtype, device=w.device)

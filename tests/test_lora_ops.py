@@ -92,3 +92,19 @@ def test_clear_caches_after_data_writes():
     Q1, K1, V1 = LoRAQKVv4Function.apply(x, *qp)
     Q2, K2, V2 = LoRAQKVv4Function.apply(x, *[t.clone() if isinstance(t, torch.Tensor) else t for t in qp])
     assert torch.equal(Q1, Q2) and torch.equal(K1, K2) and torch.equal(V1, V2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,cols,pitch,multiple", [(1, 1, 1, 8), (37, 24, 24, 1), (300, 520, 520, 8),
+                                                      (1003, 264, 272, 8), (513, 65, 67, 8), (512, 2048, 2048, 1)])
+def test_frozen_t_on_the_gpu(dtype, rows, cols, pitch, multiple):
+    from kernels._lora_ops import clear_caches, frozen_t
+
+    buf = torch.randn(rows, pitch, device="cuda").to(dtype)
+    for w in (buf[:, :cols], buf.t().contiguous().t()[:, :cols]):  # rows as stored; no unit stride along a row
+        clear_caches()
+        wt = frozen_t(w, multiple)
+        assert torch.equal(wt[:, :rows], w.t())
+        assert wt.shape == (cols, -(-rows // multiple) * multiple) and not wt[:, rows:].any()
+        assert frozen_t(w, multiple) is wt
