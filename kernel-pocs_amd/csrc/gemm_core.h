@@ -63,6 +63,15 @@ constexpr int LDS_PITCH = BK + 8;  // bf16 elements per LDS row
 
 enum Layout { ROW = 0, COL = 1 };
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <class T>
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
+  if constexpr (std::is_same_v<T, fp16_t>)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(fp16x8, a), __builtin_bit_cast(fp16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
 // Output-row mapping of B-tile rows in "dual" mode: the tile's B rows come
 // alternately (in groups of 32) from two weights, so that a wave's N tiles
 // t = 0,1,2,3 are (gate cols c..c+31, up cols c..c+31, gate c+32.., up c+32..)

@@ -20,16 +20,6 @@
 
 namespace fgemm {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <class T>
-__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
-  if constexpr (std::is_same_v<T, fp16_t>)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(fp16x8, a), __builtin_bit_cast(fp16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
 // MB: blocks of 16 rows; CB: blocks of 16 columns; ND: 2 for the dual gate / up B, else 1.
 // Lane l of a wave feeds weight row n0 + l % 16 and output row 16 b + l % 16
 // (two k-steps share 64 k: 16 (l / 16) .. + 7, then + 8 .. + 15, in both

@@ -2,25 +2,38 @@
 // 128 x 128, one wave per SIMD.
 //
 // Why 4 waves of 128 x 128: a wave's LDS fragment reads per MFMA fall with
-// the size of its output tile.  A 128 x 128 wave tile reads 4 A + 4 B
-// fragments per 16 MFMAs (0.5 per MFMA); the 64 x 128 wave tiles of 8 waves
-// read 2 + 4 per 8 (0.75), which with the LDS-DMA writes held the LDS port,
-// not the matrix cores, as the limit (MFMA busy 63% on MI355X).  The 256
-// fp32 accumulators per lane need the whole AGPR file, so each SIMD holds
-// exactly one wave (512 registers: 256 VGPRs + 256 AGPRs).
+// the size of its output tile.  A 128 x 128 wave tile reads 8 A + 8 B
+// fragments per 64 MFMAs; the 64 x 128 wave tiles of 8 waves half as many
+// again, which with the LDS-DMA writes held the LDS port, not the matrix
+// cores, as the limit (MFMA busy 63% on MI355X).  The 256 fp32 accumulators
+// per lane need the whole AGPR file, so each SIMD holds exactly one wave (512
+// registers: 256 VGPRs + 256 AGPRs).
+//
+// Why v_mfma_f32_16x16x32: under MFMA load the chip is held by its power, and
+// this shape does the same work for less.  Register-only loops on random bf16
+// data, back to back: 2100 TFLOP/s against 1820 with 32x32x16 (2460 both on
+// zeros).  The GEMMs, back to back, 32x32x16 -> 16x16x32: [8192, 4096] K =
+// 14336 838 -> 806 us, [4096, 4096] K = 128256 3137 -> 2900, [4096, 128256] K =
+// 4096 3423 -> 3330 (hipBLASLt on the same box: 650, 2740 and 3000).  With a
+// few tiles in flight, where power does not matter, a K tile takes 1.08 us
+// either way.
 //
 // With one wave per SIMD nothing else covers a stall, so the main loop keeps
 // the matrix core fed across K-tile boundaries:
-//   * fragments are double-buffered in registers: the reads of k-step ks+1
-//     are interleaved 1 : 2 with the MFMAs of k-step ks;
+//   * fragments are double-buffered in registers: the 16 reads of the next
+//     32-deep k-step are interleaved with the 64 MFMAs of this one;
 //   * the workgroup barrier of each K tile sits before the tile's LAST
 //     k-step (whose fragments are already in registers), so the barrier, the
 //     first fragment reads of the next tile and the DMA issue for the freed
 //     LDS slot all overlap that k-step's MFMAs instead of draining the pipe;
-//   * global -> LDS moves by LDS-DMA (buffer_load ... lds) into an NSTAGE ring
-//     of K tiles, NSTAGE - 1 tiles ahead of the MFMAs.  A DMA whose tile does
-//     not exist is still issued, with every offset out of range (the hardware
-//     returns zeros without a fetch), so the instruction stream has no branch.
+//   * global -> LDS moves by LDS-DMA (buffer_load ... lds) into a ring of
+//     half-tiles.  A DMA whose tile does not exist is still issued, with every
+//     offset out of range (the hardware returns zeros without a fetch);
+//   * the addresses of the next DMA are two scalar additions; segment
+//     switches, partial last tiles and the end of the list take a path out of
+//     the loop's way.  (Walking (segment, tile) cursors there, with 64-bit
+//     multiplies and two far branches between the last MFMA and the barrier,
+//     cost 1 to 3% of the whole product.)
 #pragma once
 
 #include "gemm_core.h"
@@ -98,16 +111,22 @@ struct W4Loader {
     }
   }
 
-  // Buffer resources and tail masks of one K-tile DMA at k0 (kvalid valid
-  // k; <= 0: every chunk reads zeros); load_one issues instruction j of it.
+  // Addresses and tail masks of one K-tile DMA at k0 (kvalid valid k; <= 0:
+  // every chunk reads zeros); load_one issues instruction j of it, next()
+  // moves to the following tile of the segment (the masks stay).
   struct Prep {
-    __amdgpu_buffer_rsrc_t r0, r1;
+    const char* p0;
+    const char* p1;
     bool kin[2][2];  // [gate / up rows][instruction parity]
+    __device__ __forceinline__ void next() {
+      p0 += BKT * 2;
+      if constexpr (DUAL) p1 += BKT * 2;
+    }
   };
   __device__ __forceinline__ Prep prep(int64_t k0, int64_t kvalid) const {
     Prep p;
-    p.r0 = make_rsrc(base[0] + k0 * 2);
-    p.r1 = make_rsrc(base[1] + k0 * 2);
+    p.p0 = base[0] + k0 * 2;
+    p.p1 = base[1] + k0 * 2;
     const int64_t ks = k_split - k0;  // the split in tile coordinates
 #pragma unroll
     for (int par = 0; par < 2; ++par) {
@@ -119,10 +138,7 @@ struct W4Loader {
   __device__ __forceinline__ void load_one(const Prep& p, int j, char* dst) const {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint32_t off = p.kin[sel_of(j)][j % 2] ? voff[j] : OOB;
-    // (the resource goes through a local: passed to the builtin as a
-    // conditional of two struct members, hipcc's host pass emitted the
-    // launch stub of the first instantiation of the kernel only)
-    const __amdgpu_buffer_rsrc_t r = sel_of(j) ? p.r1 : p.r0;
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(sel_of(j) ? p.p1 : p.p0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r,
                                              (__attribute__((address_space(3))) void*)(dst + (wave * IPW + j) * 1024),
                                              16, off, 0, 0, 0);
@@ -145,11 +161,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_w4_kernel(GemmArgs args) {
   constexpr int BM = 256, BN = 256, WAVES_M = 2, WAVES_N = 2, BKT = 64;
   constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N;  // 128 x 128 per wave
-  constexpr int FM = TM / 32, FN = TN / 32;
-  constexpr int KS = BKT / 16;                         // k-steps per K tile
+  constexpr int FM = TM / 16, FN = TN / 16;            // 16 x 16 blocks per wave
+  constexpr int KS = BKT / 32;                         // k-steps per K tile
   constexpr int RB = BKT * 2;                          // LDS bytes per row
   constexpr int NH = W4_NHALF;
-  static_assert(KS % 2 == 0, "an even number of k-steps per tile keeps the fragment slots static");
+  static_assert(KS == 2, "one fragment slot per k-step of a tile");
   constexpr int RING = NH * W4_HALF;
   static_assert(RING >= W4_STAGE_BYTES && RING >= W4_DUAL_BYTES, "the staged epilogue reuses the ring");
   constexpr int SMEM = RING;
@@ -164,7 +180,7 @@ void gemm_w4_kernel(GemmArgs args) {
   const int64_t m0 = (int64_t)tmi * BM;
   const int64_t n0 = (int64_t)tni * OUT_BN;
   const int lane = threadIdx.x % 64;
-  const int wave = threadIdx.x / 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int wm = wave % WAVES_M;
   const int wn = wave / WAVES_M;
 
@@ -180,13 +196,11 @@ void gemm_w4_kernel(GemmArgs args) {
   const int t_begin = blockIdx.z * per;
   const int t_end = min(total_tiles, t_begin + per);
 
-  f32x16 acc[FM][FN];
+  f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   using LoaderA = W4Loader<BKT, false>;
   using LoaderB = W4Loader<BKT, BMODE == B_DUAL>;
@@ -216,113 +230,90 @@ void gemm_w4_kernel(GemmArgs args) {
       });
     }
   };
-  // A and B walk the flat K-tile list [t_begin, t_end) with cursors of their
-  // own: A runs one tile ahead of B in the ring's issue order.
-  struct Cursor {
-    int s, t, n;    // segment, tile inside it, tiles in it
-    int64_t k;      // the segment's K
-  };
-  Cursor ca, cb;
-  {
-    int s = 0, t = t_begin, acc_t = 0;
-    while (s < args.n_segs && t >= acc_t + seg_tiles[s]) { acc_t += seg_tiles[s]; ++s; }
-    ca.s = cb.s = s;
-    ca.t = cb.t = t - acc_t;
-    ca.n = cb.n = 0;
-    ca.k = cb.k = 0;
-  }
-  // first = the cursor's current tile (set up its segment); else the next one
-  auto advance = [&](Cursor& c, bool first, bool is_a) {
-    if (!first) {
-      ++c.t;
-      if (c.t < c.n) return;
-      do { ++c.s; } while (seg_tiles[c.s] == 0);
-      c.t = 0;
+  // A and B walk the flat K-tile list [t_begin, t_end); `at` points a loader at
+  // tile t of it (past the end: nothing is read) and returns how many tiles
+  // after it next() alone reaches: whole ones of the same segment.
+  const int n_t = t_end - t_begin;
+  int seg_a = -1, seg_b = -1;  // segments that la and lb are set up for
+  constexpr int FOREVER = 1 << 30;
+  auto at = [&](int t, auto& loader, auto& setup, int& seg, auto& out) -> int {
+    if (t >= n_t) {
+      out = loader.prep(0, 0);
+      return FOREVER;
     }
-    c.n = seg_tiles[c.s];
-    c.k = args.segs[c.s].k;
-    if (is_a) setup_a(c.s);
-    else setup_b(c.s);
+    int s = 0, rel = t_begin + t;
+    while (rel >= seg_tiles[s]) rel -= seg_tiles[s++];
+    if (s != seg) setup(s);
+    seg = s;
+    const int64_t k = args.segs[s].k, k0 = (int64_t)rel * BKT;
+    out = loader.prep(k0, k - k0);
+    // (a k_split segment's masks change from tile to tile)
+    const int whole = (BMODE == B_DUAL && args.segs[s].k_split) ? 0 : (int)(k / BKT) - 1 - rel;
+    return whole < 0 ? 0 : (whole < n_t - 1 - t ? whole : n_t - 1 - t);
   };
+  auto at_a = [&](int t, PrepA& out) { return at(t, la, setup_a, seg_a, out); };
+  auto at_b = [&](int t, PrepB& out) { return at(t, lb, setup_b, seg_b, out); };
 
   constexpr int IPH = LoaderA::IPW;  // DMA instructions per wave per half-tile
   static_assert(IPH == LoaderB::IPW, "equal halves");
-  // DMA of one half (the cursor's K tile of A or B); valid = false issues
-  // the same instructions with every chunk out of range (zeros, no fetch),
-  // so the instruction stream has no branch
-  auto prep_a = [&](bool valid, PrepA& out) {
-    const int64_t k0 = (int64_t)ca.t * BKT;
-    out = la.prep(k0, valid ? ca.k - k0 : 0);
-  };
-  auto prep_b = [&](bool valid, PrepB& out) {
-    const int64_t k0 = (int64_t)cb.t * BKT;
-    out = lb.prep(k0, valid ? cb.k - k0 : 0);
-  };
   auto half_ptr = [&](int h) { return smem + h * W4_HALF; };
 
-  // per-lane fragment offsets: row (wave tile + lane % 32), chunk 2 ks + lane / 32, swizzled
-  const int g = swz<BKT>(lane % 32) ^ (lane / 32);  // chunk ^ swz = 2 ks ^ g
-  const int a_row = (wm * TM + lane % 32) * RB;
-  const int b_row = (wn * TN + lane % 32) * RB;
-  bf16x8 af[2][FM], bfr[2][FN];
-  // fragment read `idx` of k-step ks of the tile in half-slots (ha, hb) into
-  // register slot sl, in the order the MFMAs consume them: A0, B0 .. B3, A1 .. A3
-  auto frag_read = [&](const char* pa, const char* pb, int ks, int sl, int idx) {
-    const int ko = ((2 * ks) ^ g) << 4;
-    if (idx == 0) af[sl][0] = *reinterpret_cast<const bf16x8*>(pa + a_row + ko);
-    else if (idx <= FN) bfr[sl][idx - 1] = *reinterpret_cast<const bf16x8*>(pb + b_row + (idx - 1) * 32 * RB + ko);
-    else af[sl][idx - FN] = *reinterpret_cast<const bf16x8*>(pa + a_row + (idx - FN) * 32 * RB + ko);
+  // per-lane fragment offsets: row (wave tile + lane % 16), chunk 4 ks + lane / 16, swizzled
+  const int g = swz<BKT>(lane % 16) ^ (lane / 16);  // chunk ^ swz = 4 ks ^ g
+  const int a_row = (wm * TM + lane % 16) * RB;
+  const int b_row = (wn * TN + lane % 16) * RB;
+  bf16x8 af[KS][FM], bfr[KS][FN];
+  // fragment read `idx` of k-step ks of the tile in half-slots (pa, pb), in
+  // the order the MFMAs consume them: A0, B0 .. B7, A1 .. A7
+  auto frag_read = [&](const char* pa, const char* pb, int ks, int idx) {
+    const int ko = ((4 * ks) ^ g) << 4;
+    if (idx == 0) af[ks][0] = *reinterpret_cast<const bf16x8*>(pa + a_row + ko);
+    else if (idx <= FN) bfr[ks][idx - 1] = *reinterpret_cast<const bf16x8*>(pb + b_row + (idx - 1) * 16 * RB + ko);
+    else af[ks][idx - FN] = *reinterpret_cast<const bf16x8*>(pa + a_row + (idx - FN) * 16 * RB + ko);
   };
-  // MFMAs 2p and 2p+1 of a k-step, (i, j) row-major.  The operands are
+  // MFMAs 4p .. 4p + 3 of a k-step, (i, j) row-major.  The operands are
   // swapped (block (i, j) is computed as B_j A_i^T), so a lane accumulates
   // four consecutive output columns of one row (the layout gemm_w4_epi.h
   // stages with 8-byte writes).
-  auto mfma_pair = [&](int sl, int p) {
+  auto mfma_group = [&](int ks, int p) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int m = 2 * p + u, i = m / FN, j = m % FN;
-      acc[i][j] = mfma32<T>(bfr[sl][j], af[sl][i], acc[i][j]);
+    for (int u = 0; u < 4; ++u) {
+      const int m = 4 * p + u, i = m / FN, j = m % FN;
+      acc[i][j] = mfma16<T>(bfr[ks][j], af[ks][i], acc[i][j]);
     }
   };
-  constexpr int NPAIR = FM * FN / 2;  // 8 MFMA pairs per k-step ...
-  static_assert(NPAIR == FM + FN, "... and 8 fragment reads: one per pair");
+  constexpr int NGRP = FM * FN / 4;  // 16 groups of four MFMAs per k-step ...
+  static_assert(NGRP == FM + FN && NGRP == 2 * IPH, "... 16 fragment reads and 8 DMA instructions");
 
-  // DMA spread: every k-step issues 4 DMA instructions per wave (one after
-  // every other MFMA pair), so no k-step carries a burst (16 in one k-step
-  // held the in-order issue: loop time per K tile 3300 cycles against the
-  // MFMAs' 2048).  Per period (barrier(t-1) .. barrier(t)): last k-step of
-  // tile t-1 and k-step 0 of tile t: B of tile t+1 (its deadline is
-  // barrier(t)); k-steps 1 and 2 of tile t: A of tile t+2 (deadline
-  // barrier(t+1)).
-  static_assert(KS == 4 && IPH == 8 && NPAIR == 8, "4 DMA instructions per k-step");
-  const int n_t = t_end - t_begin;
+  // Per period (barrier(t-1) .. barrier(t)) the second k-step of tile t-1
+  // issues the DMA of B of tile t+1 (its deadline is barrier(t)) and the first
+  // of tile t that of A of tile t+2 (deadline barrier(t+1)), one instruction
+  // after every other group, so that no stretch carries a burst (16 in a
+  // quarter of a tile held the in-order issue: loop time per K tile 3300
+  // cycles against the MFMAs' 2048).
   if (n_t > 0) {
     // prologue: A0, B0, A1 whole and the first half of B1's instructions
     // into half-slots 0 .. 3; B1's rest and A2 follow in tile 0's k-steps
-    advance(ca, true, true);
-    advance(cb, true, false);
-    prep_a(true, pa_cur);
+    at_a(0, pa_cur);
 #pragma unroll
     for (int d = 0; d < IPH; ++d) la.load_one(pa_cur, d, half_ptr(0));
-    prep_b(true, pb_cur);
+    at_b(0, pb_cur);
 #pragma unroll
     for (int d = 0; d < IPH; ++d) lb.load_one(pb_cur, d, half_ptr(1));
-    if (1 < n_t) advance(ca, false, true);
-    prep_a(1 < n_t, pa_cur);
+    at_a(1, pa_cur);
 #pragma unroll
     for (int d = 0; d < IPH; ++d) la.load_one(pa_cur, d, half_ptr(2));
-    if (1 < n_t) advance(cb, false, false);
-    prep_b(1 < n_t, pb_cur);
+    int run_b = at_b(1, pb_cur);
 #pragma unroll
-    for (int d = 0; d < IPH / 2; ++d) lb.load_one(pb_cur, d, half_ptr(3));
-    if (2 < n_t) advance(ca, false, true);
-    prep_a(2 < n_t, pa_cur);
-    char* hb_dst = half_ptr(3);
+    for (int d = 0; d < IPH; ++d) lb.load_one(pb_cur, d, half_ptr(3));
+    // iterations that need no more than next(), for both operands
+    int run = at_a(2, pa_cur);
+    run = run < run_b ? run : run_b;
     char* ha_dst = half_ptr(4);
-    wait_vm_lgkm0<IPH + IPH / 2>();  // tile 0 (halves 0, 1) landed (this wave's part)
+    wait_vm_lgkm0<2 * IPH>();  // tile 0 (halves 0, 1) landed (this wave's part)
     bare_barrier();
 #pragma unroll
-    for (int p = 0; p < NPAIR; ++p) frag_read(half_ptr(0), half_ptr(1), 0, 0, p);
+    for (int p = 0; p < NGRP; ++p) frag_read(half_ptr(0), half_ptr(1), 0, p);
     // nothing but these reads outstanding at the loop entry, so the waits
     // inside the loop can count them precisely
     wait_vm_lgkm0<63>();
@@ -331,64 +322,68 @@ void gemm_w4_kernel(GemmArgs args) {
       const int hb = ha + 1 == NH ? 0 : ha + 1;
       const char* pa_t = half_ptr(ha);
       const char* pb_t = half_ptr(hb);
-      // Program order is pinned (sched_barrier): each MFMA pair is followed
-      // by one fragment read of the next k-step and, after every other pair,
-      // by one DMA instruction, all issued in the MFMAs' shadow.
+      // Program order is pinned (sched_barrier): the fragment reads of the
+      // other k-step and the DMA instructions are issued between groups of
+      // four MFMAs, in their shadow.  (The reads two a group at first, so that
+      // all have landed by the wait before the barrier, measured equal; the
+      // DMA in the first half of each k-step, or the barrier 2 or 4 groups into
+      // the second one, 1 to 3% slower.)
 #pragma unroll
-      for (int ks = 0; ks + 1 < KS; ++ks) {
-#pragma unroll
-        for (int p = 0; p < NPAIR; ++p) {
-          mfma_pair(ks & 1, p);
-          if (p % 2) {
-            const int q = p / 2;
-            if (ks == 0) lb.load_one(pb_cur, IPH / 2 + q, hb_dst);
-            else la.load_one(pa_cur, (ks - 1) * (IPH / 2) + q, ha_dst);
-          }
-          frag_read(pa_t, pb_t, ks + 1, (ks + 1) & 1, p);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+      for (int p = 0; p < NGRP; ++p) {
+        mfma_group(0, p);
+        if (p % 2) la.load_one(pa_cur, p / 2, ha_dst);
+        frag_read(pa_t, pb_t, 1, p);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      // Last k-step: its fragments are in registers.  Wait until this wave's
+      // Second k-step: its fragments are in registers.  Wait until this wave's
       // reads of tile t are done and its part of tile t+1 has landed (A of
       // tile t+2 may stay in flight), then one barrier: after it tile t+1 is
       // whole in LDS and tile t's half-slots (ha, hb) are free for B of tile
       // t+2 and A of tile t+3.
-      const bool b_more = t + 2 < n_t, a_more = t + 3 < n_t;
-      if (b_more) advance(cb, false, false);
-      if (a_more) advance(ca, false, true);
       wait_vm_lgkm0<IPH>();
       bare_barrier();
-      prep_b(b_more, pb_cur);
-      prep_a(a_more, pa_cur);
-      hb_dst = half_ptr(ha);
+      if (__builtin_expect(--run >= 0, 1)) {
+        pa_cur.next();
+        pb_cur.next();
+      } else {  // a segment's last, partial tile, the next segment, or the end
+        run_b = at_b(t + 2, pb_cur);
+        run = at_a(t + 3, pa_cur);
+        run = run < run_b ? run : run_b;
+      }
+      char* hb_dst = half_ptr(ha);
       ha_dst = half_ptr(hb);
       const int ha1 = hb + 1 == NH ? 0 : hb + 1;  // tile t+1's halves
       const int hb1 = ha1 + 1 == NH ? 0 : ha1 + 1;
       const char* pa_n = half_ptr(ha1);  // (after the last tile: slots nobody reads; in bounds)
       const char* pb_n = half_ptr(hb1);
 #pragma unroll
-      for (int p = 0; p < NPAIR; ++p) {
-        mfma_pair(1, p);
+      for (int p = 0; p < NGRP; ++p) {
+        mfma_group(1, p);
         if (p % 2) lb.load_one(pb_cur, p / 2, hb_dst);
-        frag_read(pa_n, pb_n, 0, 0, p);
+        frag_read(pa_n, pb_n, 0, p);
         __builtin_amdgcn_sched_barrier(0);
       }
       ha = ha1;
     }
     wait_vmcnt<0>();  // no zero-fill DMA may land in the staged epilogue's LDS
   }
+  // The epilogue's per-lane addresses are formed here: hoisted above the main
+  // loop (which holds 128 VGPRs of fragments), they spill inside it.
+  int elane = lane, ewave = wave;
+  asm volatile("" : "+v"(elane), "+s"(ewave));
+  const int ewm = ewave % WAVES_M, ewn = ewave / WAVES_M;
   if constexpr (STAGED) {
     static_assert(w4_staged_epi(EPI), "staged epilogue: 16-bit or fp32 outputs");
     static_assert(RING >= W4_F32_BYTES, "the fp32 epilogue's slabs reuse the ring");
     __bf16* lds = reinterpret_cast<__bf16*>(smem);
     if constexpr (EPI == EPI_STORE_F32)
-      w4_epilogue_f32(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
+      w4_epilogue_f32(args, acc, m0, n0, elane, ewm, ewn, reinterpret_cast<float*>(smem));
     else if constexpr (BMODE == B_DUAL)
-      w4_epilogue_staged_dual<EPI>(args, acc, m0, n0, lane, wm, wn, lds);
+      w4_epilogue_staged_dual<EPI>(args, acc, m0, n0, elane, ewm, ewn, lds);
     else  // (STORE_BF16 is launched staged at beta = 0 only)
-      w4_epilogue_staged<T, EPI>(args, acc, m0, n0, lane, wm, wn, lds);
+      w4_epilogue_staged<T, EPI>(args, acc, m0, n0, elane, ewm, ewn, lds);
   } else {
-    w4_epilogue_direct<T, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn);
+    w4_epilogue_direct<T, BMODE, EPI>(args, acc, m0, n0, elane, ewm, ewn);
   }
 }
 

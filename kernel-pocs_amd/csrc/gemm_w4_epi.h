@@ -1,13 +1,13 @@
 // Epilogues of the 4-wave GEMM engine (gemm_w4.h).
 //
-// The engine issues its MFMAs with the operands swapped (each 32 x 32 block
+// The engine issues its MFMAs with the operands swapped (each 16 x 16 block
 // is computed as B_tile A_tile^T, i.e. C^T), so that a lane's accumulators
 // hold runs of four consecutive output COLUMNS of one row:
-//   acc[i][j][r] of lane l = C[m][n],  m = m0 + 128 wm + 32 i + l % 32,
-//   n = colbase(j) + 8 (r / 4) + 4 (l / 32) + r % 4
-// with colbase(j) = n0 + 128 wn + 32 j for a single B, and for the dual
-// gate / up B (wave tile j = gate for even j, up for odd j) the output
-// columns n0 + 64 wn + 32 (j / 2) + ...
+//   acc[i][j][q] of lane l = C[m][n],  m = m0 + 128 wm + 16 i + l % 16,
+//   n = colbase(j) + 4 (l / 16) + q
+// with colbase(j) = n0 + 128 wn + 16 j for a single B, and for the dual
+// gate / up B (blocks 4c, 4c + 1 gate, 4c + 2, 4c + 3 up) the output columns
+// n0 + 64 wn + 32 c + 16 (j % 2).
 // (With A and B in the usual order a lane holds four consecutive ROWS of one
 // column, so staging a tile took 256 scattered 4-byte LDS writes per lane.)
 //
@@ -63,74 +63,69 @@ __device__ __forceinline__ float col_alpha(const EpiArgs& ep, int64_t n) {
 // Direct epilogue: every element from registers, bounds-checked.
 // ---------------------------------------------------------------------------
 template <class T, int BMODE, int EPI>
-__device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x16 (&acc)[4][4], int64_t m0, int64_t n0,
+__device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x4 (&acc)[8][8], int64_t m0, int64_t n0,
                                                    int lane, int wm, int wn) {
   const EpiArgs& ep = args.ep;
   const int64_t M = args.M, N = args.N;
-  const int cl = 4 * (lane / 32);
+  const int cl = 4 * (lane / 16);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int64_t m = m0 + wm * 128 + i * 32 + lane % 32;
+  for (int i = 0; i < 8; ++i) {
+    const int64_t m = m0 + wm * 128 + i * 16 + lane % 16;
     if (m >= M) continue;
     if constexpr (glu_fwd_epi(EPI)) {
 #pragma unroll
-      for (int jp = 0; jp < 2; ++jp)
+      for (int jp = 0; jp < 4; ++jp)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int64_t n = n0 + wn * 64 + 32 * jp + 8 * g + cl + q;
-            if (n >= N) continue;
-            const float e = acc[i][2 * jp][4 * g + q], gg = acc[i][2 * jp + 1][4 * g + q];
-            const int64_t off = m * ep.ld_eg + n;
-            if (ep.e) {
-              ep.e[off] = (__bf16)e;
-              ep.g[off] = (__bf16)gg;
-            }
-            ((__bf16*)ep.c)[m * ep.ldc + n] = (__bf16)glu_fwd_h<EPI>(e, gg);
+        for (int q = 0; q < 4; ++q) {
+          const int64_t n = n0 + wn * 64 + 16 * jp + cl + q;
+          if (n >= N) continue;
+          const int jg = 4 * (jp / 2) + jp % 2;  // gate block (up: two further)
+          const float e = acc[i][jg][q], gg = acc[i][jg + 2][q];
+          const int64_t off = m * ep.ld_eg + n;
+          if (ep.e) {
+            ep.e[off] = (__bf16)e;
+            ep.g[off] = (__bf16)gg;
           }
+          ((__bf16*)ep.c)[m * ep.ldc + n] = (__bf16)glu_fwd_h<EPI>(e, gg);
+        }
     } else if constexpr (EPI == EPI_ROPE) {
       const int64_t pos = ep.positions ? ep.positions[m] : m;
       const bool pos_ok = pos >= 0 && pos < ep.cs_rows;
-      const int half_tiles = ep.head_dim / 64;  // partner distance in 32-column tiles
+      const int half_blocks = ep.head_dim / 32;  // partner distance in 16-column blocks
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
+        for (int q = 0; q < 4; ++q) {
+          const int64_t n = n0 + wn * 128 + 16 * j + cl + q;
+          if (n >= N) continue;
+          float v = acc[i][j][q];
+          if (n < ep.rope_cols) {
+            const bool lo = (j % (2 * half_blocks)) < half_blocks;
+            const int partner = lo ? j + half_blocks : j - half_blocks;
+            float pv = 0.f;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int64_t n = n0 + wn * 128 + 32 * j + 8 * g + cl + q;
-            if (n >= N) continue;
-            float v = acc[i][j][4 * g + q];
-            if (n < ep.rope_cols) {
-              const bool lo = (j % (2 * half_tiles)) < half_tiles;
-              const int partner = lo ? j + half_tiles : j - half_tiles;
-              float pv = 0.f;
-#pragma unroll
-              for (int t = 0; t < 4; ++t)
-                if (t == partner) pv = acc[i][t][4 * g + q];
-              const int d = (int)(n % ep.head_dim) % (ep.head_dim / 2);
-              const float c = pos_ok ? (float)ep.cos[pos * ep.cs_ld + d] : __builtin_nanf("");
-              const float s = pos_ok ? (float)ep.sin[pos * ep.cs_ld + d] : __builtin_nanf("");
-              // the projection is rounded to bf16 first: RoPE is applied to the
-              // materialised Q/K in the unfused reference path
-              const float x = bf16r(v), xp = bf16r(pv);
-              v = lo ? x * c - xp * s : x * c + xp * s;
-            }
-            ((__bf16*)ep.c)[m * ep.ldc + n] = (__bf16)v;
+            for (int t = 0; t < 8; ++t)
+              if (t == partner) pv = acc[i][t][q];
+            const int d = (int)(n % ep.head_dim) % (ep.head_dim / 2);
+            const float c = pos_ok ? (float)ep.cos[pos * ep.cs_ld + d] : __builtin_nanf("");
+            const float s = pos_ok ? (float)ep.sin[pos * ep.cs_ld + d] : __builtin_nanf("");
+            // the projection is rounded to bf16 first: RoPE is applied to the
+            // materialised Q/K in the unfused reference path
+            const float x = bf16r(v), xp = bf16r(pv);
+            v = lo ? x * c - xp * s : x * c + xp * s;
           }
+          ((__bf16*)ep.c)[m * ep.ldc + n] = (__bf16)v;
+        }
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int64_t nb = n0 + wn * 128 + 32 * j + 8 * g + cl;
+      for (int j = 0; j < 8; ++j) {
+          const int64_t nb = n0 + wn * 128 + 16 * j + cl;
           if (nb >= N) continue;
           if constexpr (EPI == EPI_STORE_F32) {
             float* cp = (float*)ep.c + (int64_t)blockIdx.z * ep.split_stride + m * ep.ldc + nb;
             float v[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] = col_alpha(ep, nb + q) * acc[i][j][4 * g + q];
+            for (int q = 0; q < 4; ++q) v[q] = col_alpha(ep, nb + q) * acc[i][j][q];
             for (int q = 0; q < 4 && nb + q < N; ++q) {
               float o = v[q];
               if (ep.beta != 0.f) o += ep.beta * cp[q];
@@ -138,11 +133,11 @@ __device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x16 
             }
           } else if constexpr (EPI == EPI_ATOMIC_F32) {
             for (int q = 0; q < 4 && nb + q < N; ++q)
-              atomicAdd((float*)ep.c + m * ep.ldc + nb + q, col_alpha(ep, nb + q) * acc[i][j][4 * g + q]);
+              atomicAdd((float*)ep.c + m * ep.ldc + nb + q, col_alpha(ep, nb + q) * acc[i][j][q]);
           } else if constexpr (EPI == EPI_STORE_BF16) {
             T* cp = (T*)ep.c + m * ep.ldc + nb;
             for (int q = 0; q < 4 && nb + q < N; ++q) {
-              float o = col_alpha(ep, nb + q) * acc[i][j][4 * g + q];
+              float o = col_alpha(ep, nb + q) * acc[i][j][q];
               if (ep.beta != 0.f) o += ep.beta * (float)cp[q];
               if (ep.act) o = epi_act(ep.act, o);
               cp[q] = (T)o;
@@ -151,7 +146,7 @@ __device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x16 
             for (int q = 0; q < 4 && nb + q < N; ++q) {
               const int64_t off = m * ep.ld_eg + nb + q;
               float h, df, de;
-              glu_bwd_vals<EPI>(acc[i][j][4 * g + q], (float)ep.e[off], (float)ep.g[off], h, df, de);
+              glu_bwd_vals<EPI>(acc[i][j][q], (float)ep.e[off], (float)ep.g[off], h, df, de);
               ((__bf16*)ep.c)[m * ep.ldc + nb + q] = (__bf16)h;
               ep.e[off] = (__bf16)df;
               ep.g[off] = (__bf16)de;
@@ -177,26 +172,28 @@ __device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x16 
 constexpr int W4_FP = 128 + 4;                      // floats per staged row (4 banks apart)
 constexpr int W4_F32_BYTES = 4 * 2 * 32 * W4_FP * 4;  // 4 waves x 2 slabs of 32 rows
 
-__device__ __forceinline__ void w4_epilogue_f32(const GemmArgs& args, f32x16 (&acc)[4][4], int64_t m0, int64_t n0,
+__device__ __forceinline__ void w4_epilogue_f32(const GemmArgs& args, f32x4 (&acc)[8][8], int64_t m0, int64_t n0,
                                                 int lane, int wm, int wn, float* lds) {
   const EpiArgs& ep = args.ep;
   const int64_t M = args.M, N = args.N;
-  const int cl = 4 * (lane / 32);
+  const int cl = 4 * (lane / 16);
   lds_barrier();  // the main loop's LDS reads are done in every wave
   float* base = lds + (wn * 2 + wm) * 2 * 32 * W4_FP;
   const int c = (lane % 32) * 4;
   const int64_t n = n0 + wn * 128 + c;
   float* cbase = (float*)ep.c + (int64_t)blockIdx.z * ep.split_stride;
   const bool plain = ep.beta == 0.f && !ep.act && ep.alpha_group == 0 && n0 + 256 <= N;
+  const float alpha = ep.alpha_group == 0 ? ep.alpha : 1.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float* slab = base + (i & 1) * 32 * W4_FP;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<float4*>(slab + (lane % 32) * W4_FP + 32 * j + 8 * g + cl) =
-            make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+      for (int j = 0; j < 8; ++j)
+        // (scaled here: written as they are, the accumulators go to LDS from the
+        // AGPRs, and the register allocator then permuted them in the main loop)
+        *reinterpret_cast<f32x4*>(slab + (16 * h + lane % 16) * W4_FP + 16 * j + cl) = alpha * acc[2 * i + h][j];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's slab is written
     const int64_t mb = m0 + wm * 128 + i * 32;
     if (plain) {  // a store per row run, nothing read
@@ -205,8 +202,7 @@ __device__ __forceinline__ void w4_epilogue_f32(const GemmArgs& args, f32x16 (&a
         const int rr = it * 2 + lane / 32;
         const float4 v = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
         if (mb + rr < M)
-          *reinterpret_cast<float4*>(cbase + (mb + rr) * ep.ldc + n) =
-              make_float4(ep.alpha * v.x, ep.alpha * v.y, ep.alpha * v.z, ep.alpha * v.w);
+          *reinterpret_cast<float4*>(cbase + (mb + rr) * ep.ldc + n) = v;
       }
       continue;
     }
@@ -219,9 +215,8 @@ __device__ __forceinline__ void w4_epilogue_f32(const GemmArgs& args, f32x16 (&a
       float* cp = cbase + (mb + rr) * ep.ldc + n;
       if (mb + rr >= M) continue;
       if (n + 4 <= N && !ep.act && ep.alpha_group == 0) {  // 16-byte aligned: ldc % 8 == 0
-        const float4 a4 = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
         float4* c4 = reinterpret_cast<float4*>(cp);
-        float4 v = make_float4(ep.alpha * a4.x, ep.alpha * a4.y, ep.alpha * a4.z, ep.alpha * a4.w);
+        float4 v = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
         if (ep.beta != 0.f) {
           const float4 o = *c4;
           v.x += ep.beta * o.x; v.y += ep.beta * o.y; v.z += ep.beta * o.z; v.w += ep.beta * o.w;
@@ -231,7 +226,8 @@ __device__ __forceinline__ void w4_epilogue_f32(const GemmArgs& args, f32x16 (&a
       }
 #pragma unroll 1
       for (int q = 0; q < 4 && n + q < N; ++q) {
-        float o = col_alpha(ep, n + q) * slab[rr * W4_FP + c + q];
+        float o = slab[rr * W4_FP + c + q];
+        if (ep.alpha_group > 0) o *= col_alpha(ep, n + q);
         if (ep.beta != 0.f) o += ep.beta * cp[q];
         cp[q] = ep.act ? epi_act(ep.act, o) : o;
       }
@@ -470,28 +466,25 @@ __device__ __forceinline__ void w4_rank_partial_any(const __bf16* lds, const __b
 // c = 8 (tid % 32) and walks rows tid / 32 + 8 it.
 // ---------------------------------------------------------------------------
 template <class T, int EPI>
-__device__ __forceinline__ void w4_epilogue_staged(const GemmArgs& args, f32x16 (&acc)[4][4], int64_t m0, int64_t n0,
+__device__ __forceinline__ void w4_epilogue_staged(const GemmArgs& args, f32x4 (&acc)[8][8], int64_t m0, int64_t n0,
                                                    int lane, int wm, int wn, __bf16* lds) {
   const EpiArgs& ep = args.ep;
   const int64_t M = args.M, N = args.N;
   const int tid = threadIdx.x;
-  const int cl = 4 * (lane / 32);
+  const int cl = 4 * (lane / 16);
   lds_barrier();  // the main loop's LDS reads are done (its DMAs drained before)
   // STORE_BF16 scales by alpha (the host launches per-column alpha groups,
   // activations and beta != 0 on the direct epilogue)
   const float alpha = EPI == EPI_STORE_BF16 ? ep.alpha : 1.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 8; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 8; ++j) {
+      float v[4];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        float v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = alpha * acc[i][j][4 * g + q];
-        *reinterpret_cast<uint2*>(lds + (wm * 128 + i * 32 + lane % 32) * W4_SP + wn * 128 + 32 * j + 8 * g + cl) =
-            pack4<T>(v);
-      }
+      for (int q = 0; q < 4; ++q) v[q] = alpha * acc[i][j][q];
+      *reinterpret_cast<uint2*>(lds + (wm * 128 + i * 16 + lane % 16) * W4_SP + wn * 128 + 16 * j + cl) = pack4<T>(v);
+    }
   lds_barrier();
   constexpr int IT = 256 / 8, GRP = 4;  // rows per thread; side inputs of 4 rows in flight
   const int c = (tid % 32) * 8;
@@ -659,12 +652,12 @@ __device__ __forceinline__ void w4_epilogue_staged(const GemmArgs& args, f32x16 
 // registers from the fp32 accumulators before anything is rounded.
 // ---------------------------------------------------------------------------
 template <int EPI>
-__device__ __forceinline__ void w4_epilogue_staged_dual(const GemmArgs& args, f32x16 (&acc)[4][4], int64_t m0,
+__device__ __forceinline__ void w4_epilogue_staged_dual(const GemmArgs& args, f32x4 (&acc)[8][8], int64_t m0,
                                                         int64_t n0, int lane, int wm, int wn, __bf16* lds) {
   const EpiArgs& ep = args.ep;
   const int64_t M = args.M, N = args.N;
   const int tid = threadIdx.x;
-  const int cl = 4 * (lane / 32);
+  const int cl = 4 * (lane / 16);
   __bf16* le = lds;
   __bf16* lg = lds + 128 * W4_DP;
   __bf16* lh = lds + 2 * 128 * W4_DP;
@@ -674,24 +667,23 @@ __device__ __forceinline__ void w4_epilogue_staged_dual(const GemmArgs& args, f3
     if (pass) lds_barrier();  // pass 0's readers are done with the buffers
     if (wm == pass) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = i * 32 + lane % 32;
+      for (int i = 0; i < 8; ++i) {
+        const int row = i * 16 + lane % 16;
 #pragma unroll
-        for (int jp = 0; jp < 2; ++jp)
+        for (int jp = 0; jp < 4; ++jp) {
+          const int jg = 4 * (jp / 2) + jp % 2;  // gate block (up: two further)
+          const int col = wn * 64 + 16 * jp + cl;
+          float e[4], gg[4], h[4];
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int col = wn * 64 + 32 * jp + 8 * g + cl;
-            float e[4], gg[4], h[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              e[q] = acc[i][2 * jp][4 * g + q];
-              gg[q] = acc[i][2 * jp + 1][4 * g + q];
-              h[q] = glu_fwd_h<EPI>(e[q], gg[q]);
-            }
-            *reinterpret_cast<uint2*>(le + row * W4_DP + col) = pack4(e);
-            *reinterpret_cast<uint2*>(lg + row * W4_DP + col) = pack4(gg);
-            *reinterpret_cast<uint2*>(lh + row * W4_DP + col) = pack4(h);
+          for (int q = 0; q < 4; ++q) {
+            e[q] = acc[i][jg][q];
+            gg[q] = acc[i][jg + 2][q];
+            h[q] = glu_fwd_h<EPI>(e[q], gg[q]);
           }
+          *reinterpret_cast<uint2*>(le + row * W4_DP + col) = pack4(e);
+          *reinterpret_cast<uint2*>(lg + row * W4_DP + col) = pack4(gg);
+          *reinterpret_cast<uint2*>(lh + row * W4_DP + col) = pack4(h);
+        }
       }
     }
     lds_barrier();
