@@ -84,28 +84,52 @@ def _split(M: int, N: int, K: int, al: int, bl: int) -> int:
     return 1
 
 
-def gmm_sum(pairs) -> torch.Tensor:
-    """sum of a @ b over pairs: one product over all of them (one rounding)
-    where the MFMA core takes each in the same layouts, else one product
-    after another, added in the storage type."""
-    lay = [_mfma_layouts(a, b) for a, b in pairs]
-    M, N = pairs[0][0].shape[0], pairs[0][1].shape[1]
-    if M > 0 and N > 0 and all(v is not None and v[0::2] == lay[0][0::2] for v in lay):
-        al, bl = lay[0][0::2]
-        segs = [(a, v[1], b, v[3], a.shape[1]) for (a, b), v in zip(pairs, lay)]
-        out = torch.empty(M, N, dtype=torch.float16, device=pairs[0][0].device)
-        split = _split(M, N, sum(-(-a.shape[1] // 64) * 64 for a, _ in pairs), al, bl)
-        if split > 1:
-            return split_gemm(M, N, segs, al, bl, split, out)
-        arr = (L.GemmSegment * len(segs))(*(L.GemmSegment(a.data_ptr(), lda, b.data_ptr(), ldb, k, 0, 0)
-                                            for a, lda, b, ldb, k in segs))
-        L.check(L.forge_gemm_f16(M, N, arr, len(segs), al, bl, out.data_ptr(), N, L.DTYPE_F16, 1.0, 0.0,
-                                 L.EPI_STORE, 1, L.stream_of(out)), "forge_gemm_f16")
-        return out
-    out = None
-    for a, b in pairs:
-        out = gmm(a, b, out=out, beta=0.0 if out is None else 1.0)
+_MAX_SEGS = 6  # K segments of one product (csrc/gemm_core.h)
+
+
+def _one_product(terms, out: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """sum of a @ b over terms as one fp16 product of as many K segments, or
+    None where the MFMA core does not take them all in the same layouts."""
+    M, N = terms[0][0].shape[0], terms[0][1].shape[1]
+    lay = [_mfma_layouts(a, b) for a, b in terms]
+    if M == 0 or N == 0 or len(terms) > _MAX_SEGS or any(v is None or v[0::2] != lay[0][0::2] for v in lay):
+        return None
+    al, bl = lay[0][0::2]
+    segs = [(a, v[1], b, v[3], a.shape[1]) for (a, b), v in zip(terms, lay)]
+    if out is None:
+        out = torch.empty(M, N, dtype=torch.float16, device=terms[0][0].device)
+    split = _split(M, N, sum(-(-a.shape[1] // 64) * 64 for a, _ in terms), al, bl)
+    if split > 1:
+        return split_gemm(M, N, segs, al, bl, split, out)
+    arr = (L.GemmSegment * len(segs))(*(L.GemmSegment(a.data_ptr(), lda, b.data_ptr(), ldb, k, 0, 0)
+                                        for a, lda, b, ldb, k in segs))
+    L.check(L.forge_gemm_f16(M, N, arr, len(segs), al, bl, out.data_ptr(), out.stride(0), L.DTYPE_F16, 1.0, 0.0,
+                             L.EPI_STORE, 1, L.stream_of(out)), "forge_gemm_f16")
     return out
+
+
+def gmm_sum(pairs, lora=(), out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """sum of a @ b over pairs + sum of s * a @ b over lora's (a, b, s): one
+    product over all of them (one rounding) where the MFMA core takes them,
+    else one product after another, added in the storage type.
+
+    A LoRA term joins with s = 1 as a K segment and with s = 2 as that segment
+    twice: the sum is exact in the fp32 accumulators, and no operand is scaled
+    in fp16 (where it could overflow or lose bits).  The 64-deep K tile that a
+    segment costs is 1 us, the read-modify-write product that it replaces 33 us
+    at [2048, 8192] (MI355X).  Other scales keep that product and its alpha."""
+    if lora and all(s in (1, 2) for _, _, s in lora):
+        joined = _one_product([*pairs, *((a, b) for a, b, s in lora for _ in range(int(s)))], out)
+        if joined is not None:
+            return joined
+    total = _one_product(pairs, out)
+    if total is None:
+        total = out
+        for i, (a, b) in enumerate(pairs):
+            total = gmm(a, b, out=total, beta=1.0 if i else 0.0)
+    for a, b, s in lora:
+        gmm(a, b, out=total, alpha=s, beta=1.0)
+    return total
 
 
 def gmm(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None, alpha: float = 1.0,
@@ -140,12 +164,10 @@ def gmm(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None, al
 
 def _proj(X, W, A, B, s, out=None):
     """X W^T + s (X A^T) B^T -> (out, xa = X A^T or None)."""
-    out = gmm(X, W.t(), out=out)
-    xa = None
-    if A is not None and B is not None:
-        xa = gmm(X, A.t())
-        gmm(xa, B.t(), out=out, alpha=s, beta=1.0)
-    return out, xa
+    if A is None or B is None:
+        return gmm(X, W.t(), out=out), None
+    xa = gmm(X, A.t())
+    return gmm_sum([(X, W.t())], [(xa, B.t(), s)], out=out), xa
 
 
 def _act_fwd(e, g, activation):
@@ -202,9 +224,8 @@ def mlp_backward(dY2, X2, e, g, W_gate, A_gate, B_gate, s_gate, W_up, A_up, B_up
     """(dX, dAg, dBg, dAu, dBu, dAd, dBd): lora_mlp_pytorch.py:153-225 with
     the activation's backward from the SwiGLU / GeGLU kernel."""
     dY2, X2, e, g = _c(dY2), _c(X2), _c(e), _c(g)
-    DW = gmm(dY2, W_down)                                   # [M, I]
     td = gmm(dY2, B_down)                                   # dY Bd [M, r]
-    gmm(td, A_down, out=DW, alpha=s_down, beta=1.0)
+    DW = gmm_sum([(dY2, W_down)], [(td, A_down, s_down)])   # [M, I]
     h = _act_fwd(e, g, activation)
     df, de = _act_bwd(DW, e, g, activation)                 # d up, d gate
     dAd = gmm(td.t(), h, alpha=s_down)                      # [r, I]
@@ -217,9 +238,7 @@ def mlp_backward(dY2, X2, e, g, W_gate, A_gate, B_gate, s_gate, W_up, A_up, B_up
     else:
         xau, xag = gmm(X2, A_up.t()), gmm(X2, A_gate.t())
     dBu, dBg = gmm(df.t(), xau, alpha=s_up), gmm(de.t(), xag, alpha=s_gate)
-    dX = gmm_sum([(df, W_up), (de, W_gate)])
-    gmm(vu, A_up, out=dX, alpha=s_up, beta=1.0)
-    gmm(vg, A_gate, out=dX, alpha=s_gate, beta=1.0)
+    dX = gmm_sum([(df, W_up), (de, W_gate)], [(vu, A_up, s_up), (vg, A_gate, s_gate)])
     return dX, dAg, dBg, dAu, dBu, dAd, dBd
 
 
@@ -256,12 +275,12 @@ def qkv_backward(dQ, dK, dV, X2, W_q, W_k, W_v, A_q, B_q, s_q, A_k, B_k, s_k, A_
     """(dX, dA_q, dB_q, dA_k, dB_k, dA_v, dB_v): lora_qkv_pytorch.py:170-214."""
     X2 = _c(X2)
     dQ, dK, dV = _c(dQ), _c(dK), _c(dV)
-    dX = gmm_sum([(dQ, W_q), (dK, W_k), (dV, W_v)])
+    dYBs = [gmm(dQ, B_q), gmm(dK, B_k), gmm(dV, B_v)]       # [M, r]
+    dX = gmm_sum([(dQ, W_q), (dK, W_k), (dV, W_v)],
+                 [(dYB, A, s) for dYB, A, s in zip(dYBs, (A_q, A_k, A_v), (s_q, s_k, s_v))])
     grads = []
     xas = aux["xa"] if aux and aux.get("generic") else [None, None, None]
-    for dY, A, B, s, xa in ((dQ, A_q, B_q, s_q, xas[0]), (dK, A_k, B_k, s_k, xas[1]), (dV, A_v, B_v, s_v, xas[2])):
-        dYB = gmm(dY, B)                                    # [M, r]
-        gmm(dYB, A, out=dX, alpha=s, beta=1.0)
+    for dY, dYB, A, s, xa in zip((dQ, dK, dV), dYBs, (A_q, A_k, A_v), (s_q, s_k, s_v), xas):
         xa = xa if xa is not None else gmm(X2, A.t())
         grads += [gmm(dYB.t(), X2, alpha=s), gmm(dY.t(), xa, alpha=s)]
     return (dX, *grads)

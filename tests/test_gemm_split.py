@@ -83,3 +83,34 @@ def test_fp32_store(M, N, K, beta, pitch):
     _close(buf[:, :N], 2.0 * (a.double() @ b.double().t()) + beta * before[:, :N].double(),
            2.0 * (a.double().abs() @ b.double().abs().t()) + beta * before[:, :N].double().abs(), K)
     assert torch.equal(buf[:, N:], before[:, N:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scales", [(1.0, 2.0), (2.0, 2.0), (0.5, 2.0), (2.0, 3.0), (-1.0, 1.0)])
+@pytest.mark.parametrize("M,N,K", [(1, 264, 512), (31, 72, 136), (72, 264, 520), (300, 776, 4104), (264, 8, 64)])
+@pytest.mark.parametrize("rank", [8, 64, 72, 12])
+def test_lora_terms_of_a_sum(scales, M, N, K, rank):
+    """Two base products and two LoRA terms in both weight layouts, into a
+    column slice.  Scales of 1 and 2 join the product where the rank lets
+    them (one rounding, also where s * B alone would overflow fp16); the
+    others are added to the rounded base (two roundings more)."""
+    g = torch.Generator().manual_seed(4)
+    draw = lambda *shape: torch.randn(*shape, generator=g).half().cuda()
+    a, x = draw(M, K), [draw(M, rank) for _ in scales]
+    x[1] *= 2.0 ** -10
+    for nt in (True, False):
+        w = draw(N, K).t() if nt else draw(K, N)
+        b = [draw(N, rank).t() if nt else draw(rank, N) for _ in scales]
+        b[1] = (b[1] * 4096).clamp(-40000, 40000)
+        buf = torch.full((M, N + 16), 7.0, dtype=torch.float16, device="cuda")
+        c = gmm_sum([(a, w), (a, w)], [(p, q, s) for p, q, s in zip(x, b, scales)], out=buf[:, 8:8 + N])
+        base = 2 * (a.double() @ w.double())
+        terms = [s * (p.double() @ q.double()) for p, q, s in zip(x, b, scales)]
+        ref = base + sum(terms)
+        mag = 2 * (a.double().abs() @ w.double().abs())
+        mag += sum(abs(s) * (p.double().abs() @ q.double().abs()) for p, q, s in zip(x, b, scales))
+        one = rank % 8 == 0 and all(s in (1.0, 2.0) for s in scales)
+        seen = ref.abs() if one else base.abs() + (base + terms[0]).abs() + ref.abs() + base.abs() / 2
+        bound = 2.0 ** -11 * 1.02 * seen + (2 * K + 4 * rank) * 2.0 ** -24 * mag + 1e-6
+        assert ((c.double() - ref).abs() <= bound).all(), (nt, ((c.double() - ref).abs() - bound).max().item())
+        assert (buf[:, :8] == 7).all() and (buf[:, 8 + N:] == 7).all()
