@@ -1225,11 +1225,22 @@ __device__ __forceinline__ int tr_lane_offset(int r0, int lane) {
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef short i16x8 __attribute__((ext_vector_type(8)));
 
+// One transposing read.  The restrict parameter gives the read an alias scope
+// of its own; without one the compiler takes it to read what any LDS-DMA in
+// flight writes and waits for all of them (vmcnt(0)) before it, which drained
+// the engines' rings on every K tile.  (Plain loads carry their type for that.)
+// What orders a read after its tile's DMA is the engine's own wait and barrier.
+// Measured on MI355X, 8 waves: [8192, 4096] K = 14336 with B as [K][N] 980 -> 850
+// us, A^T B [32768, 4096] K = 4096 1098 -> 1000.
+__device__ __forceinline__ i16x4 tr_read(__attribute__((address_space(3))) const i16x4* __restrict__ p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)p);
+}
+
 // one 32x32x16 operand fragment from a token-major stage: k 0..3 from p0 and
 // k 4..7 from p1 = p0 + 4 RB (lanes 32-63: k 8..15)
 __device__ __forceinline__ bf16x8 tr_frag(const char* p0, const char* p1) {
-  const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)p0);
-  const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)p1);
+  const i16x4 lo = tr_read((__attribute__((address_space(3))) const i16x4*)p0);
+  const i16x4 hi = tr_read((__attribute__((address_space(3))) const i16x4*)p1);
   const i16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   return __builtin_bit_cast(bf16x8, v);
 }
