@@ -84,6 +84,14 @@ static void order_columns(GemmArgs& a, int64_t out_bn, int64_t tn) {
   for (int j = 0; j < tn; ++j) a.col_order[j] = (uint8_t)idx[j];
 }
 
+// The 4-wave engine's epilogue through LDS: 16-byte vectors, and of the 16-bit
+// stores the plain one (alpha alone).
+template <int EPI>
+static bool w4_staged_launch(const GemmArgs& a) {
+  const bool plain = a.ep.beta == 0.f && a.ep.act == ACT_NONE && a.ep.alpha_group == 0;
+  return w4_staged_epi(EPI) && a.ep.vec_ok && (EPI != EPI_STORE_BF16 || plain);
+}
+
 template <class T, int BM, int BN, int WM, int WN, int AL, int BL, int BMODE, int EPI>
 static int launch_cfg(GemmArgs a, hipStream_t s) {
   constexpr int OUT_BN = (BMODE == B_DUAL) ? BN / 2 : BN;
@@ -98,8 +106,7 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
     // both operands K-contiguous: the 4-wave engine (128 x 128 per wave,
     // accumulators in AGPRs, a ring of five LDS half-slots fed by LDS-DMA)
     constexpr bool W4_STAGE = w4_staged_epi(EPI);
-    const bool plain = a.ep.beta == 0.f && a.ep.act == ACT_NONE && a.ep.alpha_group == 0;
-    if (W4_STAGE && a.ep.vec_ok && (EPI != EPI_STORE_BF16 || plain))
+    if (w4_staged_launch<EPI>(a))
       gemm_w4_kernel<T, BMODE, EPI, W4_STAGE><<<grid, 256, 0, s>>>(a);
     else if (EPI == EPI_STORE_BF16 && a.ep.vec_ok && a.ep.beta != 0.f)
       // beta reads C before the single rounding: the fp32-staged epilogue of
@@ -133,18 +140,27 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
     gemm_dma_kernel<T, 96, 192, 3, 2, BMODE, EPI, 64, 3, false, 2><<<grid, 384, 0, s>>>(a);
   } else if constexpr (AL == ROW && BL == ROW && BMODE == B_SINGLE && BM == 256 && BN == 256 &&
                        (EPI == EPI_STORE_BF16 || EPI == EPI_STORE_F32)) {
-    // B as stored [K][N]: the 8-wave LDS-DMA engine with transposing fragment
-    // reads of B
+    // B as stored [K][N]: the 4-wave engine with transposing fragment reads of
+    // B; C read (beta) or stored by elements: the 8-wave LDS-DMA engine
     constexpr bool DMA_STAGE = staged_ok(BM, BN, 4, 2, EPI);
-    if (DMA_STAGE && a.ep.vec_ok)
+    if (w4_staged_launch<EPI>(a))
+      gemm_w4_kernel<T, BMODE, EPI, true, false, true><<<grid, 256, 0, s>>>(a);
+    else if (DMA_STAGE && a.ep.vec_ok)
       gemm_dma_kernel<T, BM, BN, 4, 2, BMODE, EPI, 64, 2, DMA_STAGE, 2, false, true><<<grid, 512, 0, s>>>(a);
     else
       gemm_dma_kernel<T, BM, BN, 4, 2, BMODE, EPI, 64, 2, false, 2, false, true><<<grid, 512, 0, s>>>(a);
   } else if constexpr (AL == COL && BL == ROW && BMODE == B_SINGLE && BM == 256 && BN == 256) {
-    // both operands token-major (A^T B reduced over tokens): the LDS-DMA
-    // engine with transposing fragment reads, 8 waves as above
+    // both operands token-major (A^T B reduced over tokens): as above, with
+    // transposing fragment reads of both
     constexpr int DWM = 4, DWN = 2;
     constexpr bool DMA_STAGE = staged_ok(BM, BN, DWM, DWN, EPI);
+    if constexpr (w4_staged_epi(EPI)) {
+      if (w4_staged_launch<EPI>(a)) {
+        gemm_w4_kernel<T, BMODE, EPI, true, true, true><<<grid, 256, 0, s>>>(a);
+        FORGE_CHECK_LAUNCH();
+        return FORGE_OK;
+      }
+    }
     if (DMA_STAGE && a.ep.vec_ok)
       gemm_dma_kernel<T, BM, BN, DWM, DWN, BMODE, EPI, 64, 2, DMA_STAGE, 2, true, true><<<grid, DWM * DWN * 64, 0, s>>>(a);
     else

@@ -145,6 +145,73 @@ struct W4Loader {
   }
 };
 
+// The same for a token-major operand (A stored [K][M], B stored [K][N]): the
+// half-tile is 64 k-rows of 256 elements as they lie in memory, and the
+// fragments are read with ds_read_b64_tr_b16 (the lane layout stands with
+// tr_frag).  A 16x16x32 fragment's 16-lane group g takes k 8 g .. 8 g + 7 of 16
+// rows: 32 bytes of each of four k-rows a read.  k-rows are 512 bytes, so the
+// XOR of a k-row's 16-byte chunks puts those four in different 64-byte
+// windows of the 256-byte bank cycle, and the two groups of a half-wave (k-rows
+// 8 apart) in different halves of them.
+// Against 8 waves of 32x32x16 (gemm_dma_kernel), MI355X: [8192, 4096] K = 14336 with
+// B as [K][N] 850 -> 743 us (733 with both K-contiguous), A^T B [32768, 4096] K =
+// 4096 1000 -> 945.
+__device__ __forceinline__ int swz_w4t(int q) { return 4 * (q & 3) + 2 * ((q >> 3) & 1); }
+
+template <int BKT>
+struct W4LoaderT {
+  static constexpr int RB = 512;               // LDS bytes per k-row
+  static constexpr int CPR = RB / 16;          // 16-byte chunks per k-row
+  static constexpr int RPI = 64 / CPR;         // k-rows per wave instruction
+  static constexpr int IPW = BKT / RPI / 4;    // instructions per wave per tile
+  uint32_t voff[IPW];  // byte offset of this lane's chunk from the tile's first k-row (OOB = zero-fill)
+  const char* base;
+  int64_t ld_bytes;
+  int q0;              // this lane's k-row of instruction 0
+
+  // row_ok(r): row panel_off + r exists (extents are multiples of 8, so a
+  // chunk's 8 rows exist or not together)
+  template <class RowOk>
+  __device__ __forceinline__ void setup(const void* p, int64_t ld, int64_t panel_off, RowOk row_ok) {
+    ld_bytes = ld * 2;
+    base = p ? (const char*)p + panel_off * 2 : nullptr;
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    q0 = wave * IPW * RPI + lane / CPR;
+#pragma unroll
+    for (int j = 0; j < IPW; ++j) {
+      const int q = q0 + j * RPI;
+      const int chunk = (lane % CPR) ^ swz_w4t(q);  // source chunk of LDS slot lane % CPR
+      voff[j] = (base && row_ok(chunk * 8)) ? (uint32_t)(q * ld_bytes + chunk * 16) : OOB;
+    }
+  }
+
+  struct Prep {
+    const char* p0;
+    int64_t step;  // bytes of a K tile
+    int kvalid;    // k-rows of the tile that exist
+    __device__ __forceinline__ void next() { p0 += step; }
+  };
+  __device__ __forceinline__ Prep prep(int64_t k0, int64_t kvalid) const {
+    return {base + k0 * ld_bytes, BKT * ld_bytes, (int)(kvalid < BKT ? kvalid : BKT)};
+  }
+  __device__ __forceinline__ void load_one(const Prep& p, int j, char* dst) const {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint32_t off = q0 + j * RPI < p.kvalid ? voff[j] : OOB;
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(p.p0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r,
+                                             (__attribute__((address_space(3))) void*)(dst + (wave * IPW + j) * 1024),
+                                             16, off, 0, 0, 0);
+  }
+};
+
+// Byte offset, in a token-major half-tile, of what this lane supplies to the
+// fragment of rows r0 .. r0 + 15 (r0 a multiple of 128) at k 0..3; rows 16 i
+// further: ^ (i << 5); k-row q further: + q * 512 (q = 4, or a multiple of 32).
+__device__ __forceinline__ int w4t_lane_offset(int r0, int lane) {
+  const int l = lane % 16, q = 8 * (lane / 16) + l / 4, r = r0 + 4 * (l % 4);
+  return q * 512 + (((r / 8) ^ swz_w4t(q)) * 16) + (r % 8) * 2;
+}
+
 // Ring of NHALF half-slots of 32 KB (256 rows x 64 k of one operand).  K
 // tile x keeps A in half-slot (2x) % NHALF and B in (2x + 1) % NHALF.  With
 // NHALF = 5 (160 KB) the barrier of iteration t frees tile t's two halves,
@@ -156,7 +223,7 @@ struct W4Loader {
 constexpr int W4_NHALF = 5;
 constexpr int W4_HALF = 256 * 64 * 2;  // bytes per half-slot
 
-template <class T, int BMODE, int EPI, bool STAGED>
+template <class T, int BMODE, int EPI, bool STAGED, bool AT = false, bool BT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_w4_kernel(GemmArgs args) {
   constexpr int BM = 256, BN = 256, WAVES_M = 2, WAVES_N = 2, BKT = 64;
@@ -202,8 +269,9 @@ void gemm_w4_kernel(GemmArgs args) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  using LoaderA = W4Loader<BKT, false>;
-  using LoaderB = W4Loader<BKT, BMODE == B_DUAL>;
+  static_assert(!(BT && BMODE == B_DUAL), "dual B operands are K-contiguous");
+  using LoaderA = std::conditional_t<AT, W4LoaderT<BKT>, W4Loader<BKT, false>>;
+  using LoaderB = std::conditional_t<BT, W4LoaderT<BKT>, W4Loader<BKT, BMODE == B_DUAL>>;
   using PrepA = typename LoaderA::Prep;
   using PrepB = typename LoaderB::Prep;
   LoaderA la;
@@ -212,11 +280,17 @@ void gemm_w4_kernel(GemmArgs args) {
   PrepB pb_cur;  // B of tile t+1 (dst half-slot hb_dst)
   auto setup_a = [&](int s) {
     const Seg& sg = args.segs[s];
-    la.setup(sg.a, sg.a, sg.lda, m0, [&](int q, int) -> int64_t { return m0 + q < M ? q : -1; });
+    if constexpr (AT) la.setup(sg.a, sg.lda, m0, [&](int r) { return m0 + r < M; });
+    else la.setup(sg.a, sg.a, sg.lda, m0, [&](int q, int) -> int64_t { return m0 + q < M ? q : -1; });
   };
   auto setup_b = [&](int s) {
     const Seg& sg = args.segs[s];
-    if constexpr (BMODE == B_DUAL) {
+    if constexpr (BT) {
+      lb.setup(sg.b, sg.ldb, n0 - sg.n_lo, [&](int r) {
+        const int64_t n = n0 + r;
+        return n < args.N && n >= sg.n_lo && n < sg.n_hi;
+      });
+    } else if constexpr (BMODE == B_DUAL) {
       lb.setup(sg.b, sg.b2, sg.ldb, n0, [&](int q, int) -> int64_t {
         const int t4 = (q % 128) / 32;
         const int rel = (q / 128) * 64 + (t4 / 2) * 32 + q % 32;
@@ -262,14 +336,27 @@ void gemm_w4_kernel(GemmArgs args) {
   const int g = swz<BKT>(lane % 16) ^ (lane / 16);  // chunk ^ swz = 4 ks ^ g
   const int a_row = (wm * TM + lane % 16) * RB;
   const int b_row = (wn * TN + lane % 16) * RB;
+  const int a_tr = AT ? w4t_lane_offset(wm * TM, lane) : 0;
+  const int b_tr = BT ? w4t_lane_offset(wn * TN, lane) : 0;
   bf16x8 af[KS][FM], bfr[KS][FN];
+  auto read_tr = [&](const char* half, int off, int ks, int i) {
+    const char* p = smem + (((int)(half - smem) + off) ^ (i << 5)) + ks * 32 * 512;
+    return tr_frag(p, p + 4 * 512);
+  };
+  auto read_a = [&](const char* pa, int ks, int i) {
+    if constexpr (AT) return read_tr(pa, a_tr, ks, i);
+    else return *reinterpret_cast<const bf16x8*>(pa + a_row + i * 16 * RB + (((4 * ks) ^ g) << 4));
+  };
+  auto read_b = [&](const char* pb, int ks, int j) {
+    if constexpr (BT) return read_tr(pb, b_tr, ks, j);
+    else return *reinterpret_cast<const bf16x8*>(pb + b_row + j * 16 * RB + (((4 * ks) ^ g) << 4));
+  };
   // fragment read `idx` of k-step ks of the tile in half-slots (pa, pb), in
   // the order the MFMAs consume them: A0, B0 .. B7, A1 .. A7
   auto frag_read = [&](const char* pa, const char* pb, int ks, int idx) {
-    const int ko = ((4 * ks) ^ g) << 4;
-    if (idx == 0) af[ks][0] = *reinterpret_cast<const bf16x8*>(pa + a_row + ko);
-    else if (idx <= FN) bfr[ks][idx - 1] = *reinterpret_cast<const bf16x8*>(pb + b_row + (idx - 1) * 16 * RB + ko);
-    else af[ks][idx - FN] = *reinterpret_cast<const bf16x8*>(pa + a_row + (idx - FN) * 16 * RB + ko);
+    if (idx == 0) af[ks][0] = read_a(pa, ks, 0);
+    else if (idx <= FN) bfr[ks][idx - 1] = read_b(pb, ks, idx - 1);
+    else af[ks][idx - FN] = read_a(pa, ks, idx - FN);
   };
   // MFMAs 4p .. 4p + 3 of a k-step, (i, j) row-major.  The operands are
   // swapped (block (i, j) is computed as B_j A_i^T), so a lane accumulates

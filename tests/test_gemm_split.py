@@ -114,3 +114,35 @@ def test_lora_terms_of_a_sum(scales, M, N, K, rank):
         bound = 2.0 ** -11 * 1.02 * seen + (2 * K + 4 * rank) * 2.0 ** -24 * mag + 1e-6
         assert ((c.double() - ref).abs() <= bound).all(), (nt, ((c.double() - ref).abs() - bound).max().item())
         assert (buf[:, :8] == 7).all() and (buf[:, 8 + N:] == 7).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(264, 272, 8), (256, 512, 64), (264, 520, 200), (512, 264, 1096), (776, 1000, 328)])
+@pytest.mark.parametrize("a_layout", [ROW, COL])
+@pytest.mark.parametrize("split", [1, 3])
+def test_token_major_big_tiles(dtype, M, N, K, a_layout, split):
+    """256 x 256 tiles with B stored [K][N] and A either way: two segments of
+    unequal K (with A^T not a multiple of 8), padded pitches and partial tiles."""
+    g = torch.Generator().manual_seed(5)
+    ks = (K, 72) if a_layout == ROW else (K - 3, 65)
+    segs, ref, mag = [], 0, 0
+    for k in ks:
+        a, b = torch.randn(M, k, generator=g).to(dtype), torch.randn(k, N, generator=g).to(dtype)
+        ref, mag = ref + a.double() @ b.double(), mag + a.double().abs() @ b.double().abs()
+        b = torch.nn.functional.pad(b, (0, 8)).cuda()
+        if a_layout == ROW:
+            a, lda = torch.nn.functional.pad(a, (0, -k % 8)).cuda(), k + -k % 8
+        else:
+            a, lda = torch.nn.functional.pad(a.t(), (0, 16)).cuda(), M + 16
+        segs.append((a, lda, b, N + 8, k))
+    ref, mag = ref.cuda(), mag.cuda()
+    arr = (L.GemmSegment * 2)(*(L.GemmSegment(a.data_ptr(), la, b.data_ptr(), lb, k, 0, 0) for a, la, b, lb, k in segs))
+    fn = L.forge_gemm_f16 if dtype == torch.float16 else L.forge_gemm
+    for out_dtype in (dtype, torch.float32):
+        if out_dtype == dtype and split > 1:
+            continue
+        c = torch.full((split, M, N), float("nan"), dtype=out_dtype, device="cuda")
+        L.check(fn(M, N, arr, 2, a_layout, ROW, c.data_ptr(), N, L.dtype_code(out_dtype), 0.5, 0.0, L.EPI_STORE, split,
+                   L.stream_of(c)), "forge_gemm")
+        _close(c[0] if split == 1 else c.sum(0), 0.5 * ref, mag, sum(ks))
