@@ -36,12 +36,21 @@ def as_operand(t: torch.Tensor) -> torch.Tensor:
         raise TypeError(f"LoRA kernels compute in bf16, got {t.dtype}")
     if t.dim() != 2:
         t = t.reshape(-1, t.shape[-1])
-    ok = t.stride(-1) == 1 and (t.shape[0] <= 1 or t.stride(0) % 8 == 0) and t.data_ptr() % 16 == 0
+    s0, s1 = t.stride()
+    ok = s1 == 1 and (s0 % 8 == 0 or t.shape[0] <= 1) and t.data_ptr() % 16 == 0
     return t if ok else t.contiguous()
 
 
 def ld(t: torch.Tensor) -> int:
-    return t.stride(0) if t.dim() == 2 and t.shape[0] > 1 else t.shape[-1]
+    n = t.shape
+    return t.stride(0) if len(n) == 2 and n[0] > 1 else n[-1]
+
+
+# (ctypes makes an array type per length on a slower path than this lookup: a
+# LoRA training step on few tokens is bound by the host, 300 us of it here)
+@functools.lru_cache(maxsize=64)
+def _array(ctype, n: int):
+    return ctype * n
 
 
 def skinny_split(M: int, N: int, K: int, k_contiguous: bool = True) -> int:
@@ -98,12 +107,8 @@ def split_for(M: int, N: int, k_tiles: int) -> int:
 def _segments(segs) -> ctypes.Array:
     """forge_gemm_segment array from (A, lda, B, ldb, K) tuples, optionally
     extended by (n_lo, n_hi): the output columns the segment applies to."""
-    arr = (L.GemmSegment * len(segs))()
-    for i, sg in enumerate(segs):
-        a, lda, b, ldb, k = sg[:5]
-        n_lo, n_hi = (int(sg[5]), int(sg[6])) if len(sg) > 5 else (0, 0)
-        arr[i] = L.GemmSegment(a.data_ptr(), int(lda), b.data_ptr(), int(ldb), int(k), n_lo, n_hi)
-    return arr
+    return _array(L.GemmSegment, len(segs))(
+        *[(sg[0].data_ptr(), sg[1], sg[2].data_ptr(), sg[3], sg[4], *(sg[5:7] if len(sg) > 5 else (0, 0))) for sg in segs])
 
 
 def gemm(M: int, N: int, segs: Sequence[Tuple[torch.Tensor, int, torch.Tensor, int, int]], a_layout: int,
@@ -198,8 +203,8 @@ def lora_a(x: torch.Tensor, mats: Sequence[torch.Tensor], scales: Sequence[float
         addrs = [a.data_ptr() for a in mats]
     if out is None:
         out = torch.empty(M, n * r, dtype=torch.bfloat16, device=x.device)
-    ptrs = (ctypes.c_void_p * n)(*addrs)
-    sc = (ctypes.c_float * n)(*[float(s) for s in scales])
+    ptrs = _array(ctypes.c_void_p, n)(*addrs)
+    sc = _array(ctypes.c_float, n)(*[float(s) for s in scales])
     split = skinny_split(M, n * r, K) if M > n * r else 1
     work = torch.empty(split, M, n * r, dtype=torch.float32, device=x.device) if split > 1 else None
     L.check(
@@ -296,21 +301,21 @@ def small_t_batch(mats: Sequence[torch.Tensor]) -> list:
     if len(mats) > L.TRANSPOSE_BATCH_MAX or any(m.dtype != torch.bfloat16 or m.dim() != 2 for m in mats):
         return [small_t(m) for m in mats]
     mats = [as_operand(m.detach()) for m in mats]
-    sizes = [m.numel() for m in mats]
+    rows, cols = [m.shape[0] for m in mats], [m.shape[1] for m in mats]
     # each transposed matrix starts on a 16-byte boundary of the shared buffer
     offs, o = [], 0
-    for n in sizes:
+    for r, c in zip(rows, cols):
         offs.append(o)
-        o += -(-n // 8) * 8
+        o += -(-r * c // 8) * 8
     buf = torch.empty(o, dtype=mats[0].dtype, device=mats[0].device)
-    outs = [buf[off:off + n].view(m.shape[1], m.shape[0]) for off, n, m in zip(offs, sizes, mats)]
+    outs = [buf.as_strided((c, r), (r, 1), off) for r, c, off in zip(rows, cols, offs)]
     k = len(mats)
-    src = (ctypes.c_void_p * k)(*[m.data_ptr() for m in mats])
-    dst = (ctypes.c_void_p * k)(*[t.data_ptr() for t in outs])
-    ld_src = (ctypes.c_int64 * k)(*[ld(m) for m in mats])
-    rows = (ctypes.c_int64 * k)(*[m.shape[0] for m in mats])
-    cols = (ctypes.c_int64 * k)(*[m.shape[1] for m in mats])
-    ld_dst = (ctypes.c_int64 * k)(*[m.shape[0] for m in mats])
+    ptrs, ints = _array(ctypes.c_void_p, k), _array(ctypes.c_int64, k)
+    base, size = buf.data_ptr(), buf.element_size()
+    src = ptrs(*[m.data_ptr() for m in mats])
+    dst = ptrs(*[base + off * size for off in offs])
+    ld_src, ld_dst = ints(*[ld(m) for m in mats]), ints(*rows)
+    rows, cols = ld_dst, ints(*cols)
     L.check(L.forge_transpose_2b_batch(k, src, ld_src, rows, cols, dst, ld_dst, L.stream_of(buf)),
             "forge_transpose_2b_batch")
     return outs
