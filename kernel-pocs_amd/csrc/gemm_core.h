@@ -7,17 +7,15 @@
 // separate kernel and another pass over the output.
 //
 // Tiling: BM x BN x 64 block tile, WAVES_M x WAVES_N waves, each wave owns a
-// (BM/WAVES_M) x (BN/WAVES_N) sub-tile computed with v_mfma_f32_32x32x16_bf16.
-// Two main loops feed the same MFMA core:
-//   * gemm_dma_kernel (256 x 256 tiles, both operands K-contiguous: X W^T and
-//     its LoRA segments, the SwiGLU-dual and RoPE GEMMs): global -> LDS by
-//     LDS-DMA (buffer_load ... lds, no VGPR staging, no ds_write), XOR-swizzled
-//     unpadded LDS rows, a 2-stage ring (measured on MI355X: 918 -> 1018
-//     TFLOP/s on the 8192 x 28672 x 4096 gate/up GEMM; a 4-stage ring of
-//     32-deep tiles and an interleaved DMA issue were no faster).  It runs
-//     8 waves (4 x 2, 64 x 128 per wave) so that each SIMD holds two waves
-//     whose MFMA chains cover each other's LDS reads and barriers (measured:
-//     the 8192 x 4096 x 14336 down-projection 1075 -> 1213 TFLOP/s);
+// (BM/WAVES_M) x (BN/WAVES_N) sub-tile.  256 x 256 tiles run on the 4-wave
+// engine (gemm_w4.h, v_mfma_f32_16x16x32) and a few rows on the row engine
+// (gemm_rows.hip); here are the others, on v_mfma_f32_32x32x16:
+//   * gemm_dma_kernel (narrow and skinny tiles; 256 x 256 tiles whose C is read
+//     or whose stores cannot be vectors): global -> LDS by LDS-DMA
+//     (buffer_load ... lds, no VGPR staging, no ds_write), XOR-swizzled
+//     unpadded LDS rows, a 2- or 3-stage ring.  At 256 x 256 it runs 8 waves
+//     (4 x 2, 64 x 128 per wave) so that each SIMD holds two waves whose MFMA
+//     chains cover each other's LDS reads and barriers;
 //   * gemm_kernel (every layout): loads through registers into padded LDS
 //     rows ([rows][64 + 8 pad] bf16, 144-byte pitch, conflict-free fragment
 //     reads), double-buffered.  Operands whose K dimension is not contiguous

@@ -7,10 +7,11 @@ fp32 (kernels/lora_mlp/tests/test_lora_mlp.py:507-549, :1348-1456;
 kernels/lora_qkv/tests/test_v2_2_v2_3_v3.py) - where its big GEMMs are plain
 cuBLAS fp32 products.  This module is that path here: every product is
 forge_gemm_generic (fp32 accumulation, one rounding to the storage type, any
-strides, so transposed operands are read in place; aligned fp16 products run
-on the MFMA core there, and those whose tiles leave CUs idle are split over K
-by `gmm`), the activation is the
-SwiGLU / GeGLU kernel and RoPE the RoPE kernel, all in the input's dtype.
+strides, so transposed operands are read in place).  Aligned fp16 products run
+on the MFMA core: those whose tiles leave CUs idle are split over K (`gmm`),
+and the LoRA terms of a base product join it as K segments (`gmm_sum`).  The
+activation is the SwiGLU / GeGLU kernel and RoPE the RoPE kernel, all in the
+input's dtype.
 The math is the reference's PyTorch formulation
 (kernels/lora_mlp/reference/lora_mlp_pytorch.py:100-225,
 kernels/lora_qkv/reference/lora_qkv_pytorch.py:34-214):
