@@ -60,6 +60,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(GemmArgs args) {
     // up rows of a k_split segment start at column k - k_split
     const int64_t ks1 = ND == 2 ? sg.k_split : 0;
     const __amdgpu_buffer_rsrc_t rb1 = make_rsrc(ND == 2 ? sg.b2 + brow * sg.ldb - ks1 : sg.b);
+    // (a null operand reads as zeros, as in the other engines' loaders)
+    const bool has_a = sg.a, has_b0 = sg.b, has_b1 = ND == 1 || sg.b2;
     const int n_chunk = (int)((sg.k + 32 * U - 1) / (32 * U));
     const int first = ((wave - turn) % NW + NW) % NW;
     turn += n_chunk;
@@ -73,14 +75,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(GemmArgs args) {
         const int k = k0 + 64 * (u / 2) + 8 * (u % 2);
         const bool in = whole || k + kg < sg.k;
         // (a k_split segment: gate rows read k < k_split, up rows the rest)
-        const bool in0 = whole || (in && (ks1 == 0 || k + kg < ks1)), in1 = whole || (in && k + kg >= ks1);
+        const bool in0 = whole || (in && has_b0 && (ks1 == 0 || k + kg < ks1));
+        const bool in1 = whole || (in && has_b1 && k + kg >= ks1);
 #pragma unroll
         for (int c = 0; c < CB; ++c) {
           bf[u][c * ND] = load(rb0, in0 ? boff[c] : OOB, k);
           if constexpr (ND == 2) bf[u][c * ND + 1] = load(rb1, in1 ? boff[c] : OOB, k);
         }
 #pragma unroll
-        for (int b = 0; b < MB; ++b) af[u][b] = load(ra, in ? aoff[b] : OOB, k);
+        for (int b = 0; b < MB; ++b) af[u][b] = load(ra, whole || (in && has_a) ? aoff[b] : OOB, k);
       }
       // every load of the chunk is issued before the first wait (left to the
       // scheduler, half of them were)
@@ -94,7 +97,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(GemmArgs args) {
     };
     for (int c = first; c < n_chunk; c += NW) {
       const int k0 = c * 32 * U;
-      if (ks1 == 0 && k0 + 32 * U <= sg.k) chunk(k0, true);
+      if (ks1 == 0 && has_a && has_b0 && has_b1 && k0 + 32 * U <= sg.k) chunk(k0, true);
       else chunk(k0, false);
     }
   }

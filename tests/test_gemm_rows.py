@@ -78,3 +78,36 @@ def test_gate_up(M, H, I, r, act):
     h2 = torch.empty_like(h)  # inference: h alone
     L.check(L.forge_lora_mlp_gate_up(*args, None, None, h2.data_ptr(), I, act, L.stream_of(x)), "gate_up")
     assert torch.equal(h, h2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 20, 40, 64, 65])
+def test_null_operands_read_as_zeros(M):
+    """A missing operand contributes nothing, whatever the row count (the row
+    engine up to 64 rows, 256 x 256 tiles past them); K of one partial chunk
+    and of several whole ones."""
+    gen = torch.Generator().manual_seed(M)
+    H, I, r = 2056, 520, 16
+    x, wg, wu = _mat(M, H, gen), _mat(I, H, gen) * H ** -0.5, _mat(I, H, gen) * H ** -0.5
+    xa, b = _mat(M, 2 * r, gen), _mat(I, r, gen)
+    zero = torch.zeros_like(b)
+
+    def gate_up(wgate, wup, bg, bu, rank=r):
+        e, g, h = (torch.empty(M, I, dtype=torch.bfloat16, device="cuda") for _ in range(3))
+        L.check(L.forge_lora_mlp_gate_up(M, H, I, rank, x.data_ptr(), H, L.ptr(wgate), L.ptr(wup), H,
+                                         xa.data_ptr() if rank else None, 2 * r, L.ptr(bg), L.ptr(bu), r, e.data_ptr(),
+                                         g.data_ptr(), h.data_ptr(), I, L.ACT_SILU, L.stream_of(x)), "gate_up")
+        return e, g, h
+
+    for got, want in ((gate_up(wg, wu, None, b), gate_up(wg, wu, zero, b)),
+                      (gate_up(wg, wu, b, None), gate_up(wg, wu, b, zero)),
+                      (gate_up(wg, None, None, None, 0), gate_up(wg, torch.zeros_like(wu), None, None, 0))):
+        for a, c in zip(got, want):
+            assert torch.equal(a, c)
+    c = torch.full((M, I), 7.0, dtype=torch.bfloat16, device="cuda")
+    for a, w in ((None, wg), (x, None)):
+        seg = (L.GemmSegment * 1)(L.GemmSegment(L.ptr(a), H, L.ptr(w), H, H, 0, 0))
+        L.check(L.forge_gemm(M, I, seg, 1, ROW, COL, c.data_ptr(), I, L.DTYPE_BF16, 1.0, 0.0, L.EPI_STORE, 1,
+                             L.stream_of(c)), "forge_gemm")
+        assert not c.any()
+        c.fill_(7.0)
