@@ -533,7 +533,7 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
   if (ce_row_head<T, NT>(a, row, y, xr, pre == 0 && V % VEC == 0, redf)) return;
 
   const bool grads = a.flags & FORGE_CE_HAS_GRADIENTS;
-  const float sc = a.softcap, inv_sc = SC ? 1.f / sc : 0.f;
+  const float sc = fabsf(a.softcap), inv_sc = SC ? 1.f / sc : 0.f;  // (sc tanh(x / sc) is even in sc)
   const float ls = a.label_smoothing;
   const float eps = ls / (float)V;
   const float wy = W ? a.weight[y] : 1.f;

@@ -123,3 +123,23 @@ def test_infinities_and_nan(dtype, softcap):
     assert torch.isnan(o[2]) and torch.isnan(want[2])
     keep = torch.tensor([0, 1, 3], device="cuda")
     assert ((o[keep].double() - want[keep]).abs() <= U[dtype] * want[keep].abs() + 1e-5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("softcap", [3.0, 40.0, 100.0, 1000.0])
+def test_negative_softcap(dtype, softcap):
+    """softcap * tanh(x / softcap) is even in softcap: the functional entry
+    takes a negative value for its magnitude, argmax included."""
+    gen = torch.Generator().manual_seed(8)
+    x = (torch.randn(3, 4099, generator=gen) * 30).to(dtype).cuda()
+    t = torch.tensor([1, 4098, 2000], device="cuda")
+    out = []
+    for sc in (softcap, -softcap):
+        leaf = x.clone().requires_grad_(True)
+        o = forge_cross_entropy(leaf, t, softcap=sc, return_predicted_tokens=True)
+        o.loss.backward()
+        assert torch.isfinite(o.loss)
+        out.append((o.loss.detach(), leaf.grad, o.predicted_tokens))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
