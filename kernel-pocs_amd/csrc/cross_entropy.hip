@@ -468,47 +468,64 @@ __device__ __forceinline__ bool ce_row_head(CeArgs& a, int64_t row, int64_t y, T
 // ---------------------------------------------------------------------------
 constexpr int kStreamU = 4;  // vectors in flight per thread
 
-// sc tanh(x / sc) for 16-bit logits, n values.  |x| <= sc / 2 throughout the
-// vector: x P((x / sc)^2), P the degree-4 Chebyshev fit of tanh(u) / u on
-// u^2 <= 1/4 (relative error 1.1e-7 evaluated in fp32, libm's tanhf 1e-7);
-// else 1 - 2 / (1 + e^2u), whose absolute error of 1.2e-7 sc is far below
-// the 16-bit spacing of such logits.  The choice is per wave.
-template <int N>
-__device__ __forceinline__ void cap_fast(float (&x)[N], float sc, float inv_sc) {
+// Soft cap of 16-bit logits: x <- sc tanh(x / sc), and its slope 1 - tanh^2
+// where asked for.  |x| <= sc / 2 throughout the vector: x P((x / sc)^2), P the
+// degree-4 Chebyshev fit of tanh(u) / u on u^2 <= 1/4 (relative error 1.1e-7
+// evaluated in fp32, libm's tanhf 1e-7), and 1 - (u P)^2; else, with t = e^-2|u|
+// and r = 1 / (1 + t), tanh|u| = 1 - 2 t r, whose absolute error of 1.2e-7 sc is
+// far below the 16-bit spacing of such logits, and the slope 4 t r^2, which
+// stays a product where 1 - tanh^2 cancels (relative error 2e-6 up to |x| = 8
+// sc; of 1 - tanh^2 in fp32 1e-3 at 5 sc, 5e-2 at 7 sc).  The choice is per wave.
+template <int N, bool SLOPE>
+__device__ __forceinline__ void cap_fast(float (&x)[N], float (&slope)[N], float sc, float inv_sc) {
+  const float half = 0.5f * sc, k = -2.f * kLog2e * inv_sc;
+  auto small = [&](float& v, float& sl) {
+    const float u = v * inv_sc, q = u * u;
+    float p = fmaf(q, 0.01714132f, -0.05298924f);
+    p = fmaf(q, p, 0.13324829f);
+    p = fmaf(q, p, -0.33333072f);
+    p = fmaf(q, p, 0.99999999f);
+    v *= p;
+    if constexpr (SLOPE) {
+      const float th = u * p;
+      sl = fmaf(-th, th, 1.f);
+    }
+  };
   float big = 0.f;
 #pragma unroll
-  for (int j = 0; j < N; ++j) big = fmaxf(big, fabsf(x[j]));
-  bool ok = big <= 0.5f * sc;
+  for (int j = 0; j < N; ++j) big = fmaxf(big, fabsf(x[j]));  // (drops NaN, which either form keeps)
+  if (__all(big <= half)) {
 #pragma unroll
-  for (int j = 0; j < N; ++j) ok = ok && x[j] == x[j];  // (fmaxf drops NaN)
-  if (__all(ok)) {
-    const float q0 = inv_sc * inv_sc;
+    for (int j = 0; j < N; ++j) small(x[j], slope[j]);
+  } else {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      const float q = x[j] * x[j] * q0;
-      float p = fmaf(q, 0.01714132f, -0.05298924f);
-      p = fmaf(q, p, 0.13324829f);
-      p = fmaf(q, p, -0.33333072f);
-      p = fmaf(q, p, 0.99999999f);
-      x[j] *= p;
+      const float t = fast_exp2(fabsf(x[j]) * k), r = __builtin_amdgcn_rcpf(1.f + t), tr = t * r;
+      x[j] = copysignf(fmaf(-2.f * sc, tr, sc), x[j]);
+      if constexpr (SLOPE) slope[j] = 4.f * tr * r;
     }
-  } else {
-    const float k = 2.f * kLog2e * inv_sc;
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-      x[j] = fmaf(-2.f * sc, __builtin_amdgcn_rcpf(1.f + fast_exp2(x[j] * k)), sc);
   }
 }
 
-// Soft cap of a vector (fp32 logits keep libm's tanhf).
-template <bool EXACT, int N>
-__device__ __forceinline__ void cap(float (&x)[N], float sc, float inv_sc) {
+// Soft cap of a vector (fp32 logits keep libm's tanhf), with its slope or without.
+template <bool EXACT, bool SLOPE, int N>
+__device__ __forceinline__ void cap(float (&x)[N], float (&slope)[N], float sc, float inv_sc) {
   if constexpr (EXACT) {
 #pragma unroll
-    for (int j = 0; j < N; ++j) x[j] = sc * tanhf(x[j] / sc);
+    for (int j = 0; j < N; ++j) {
+      const float th = tanhf(x[j] / sc);
+      x[j] = sc * th;
+      if constexpr (SLOPE) slope[j] = 1.f - th * th;
+    }
   } else {
-    cap_fast<N>(x, sc, inv_sc);
+    cap_fast<N, SLOPE>(x, slope, sc, inv_sc);
   }
+}
+
+template <bool EXACT, int N>
+__device__ __forceinline__ void cap(float (&x)[N], float sc, float inv_sc) {
+  float none[N];
+  cap<EXACT, false, N>(x, none, sc, inv_sc);
 }
 
 template <class T, int NT, bool SC, bool W, bool ARG>
@@ -665,18 +682,8 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
     const float dy = W ? (1.f - ls) * wy * inv_snw : ydelta;
     auto pass2 = [&](auto& v, int64_t c0) {
       constexpr int N = sizeof(v) / sizeof(float);
-      float th[N];  // tanh(x / sc), for the cap's slope 1 - th^2
-      if constexpr (SC && EXACT) {
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-          th[j] = tanhf(v[j] / sc);
-          v[j] = sc * th[j];
-        }
-      } else if constexpr (SC) {
-        cap_fast<N>(v, sc, inv_sc);
-#pragma unroll
-        for (int j = 0; j < N; ++j) th[j] = v[j] * inv_sc;
-      }
+      float slope[N];  // of the cap
+      if constexpr (SC) cap<EXACT, true, N>(v, slope, sc, inv_sc);
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         const float p = fast_exp2(fmaf(v[j], kLog2e, -m2));
@@ -688,16 +695,13 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
           const float smooth = eps * (-a.weight[c0 + j] + p * a.weight_sum);
           g = ori * inv_snw + smooth * inv_snw + dz * p * inv_n;
         }
-        if constexpr (SC) {
-          th[j] = 1.f - th[j] * th[j];
-          g *= th[j];
-        }
+        if constexpr (SC) g *= slope[j];
         v[j] = g;
       }
       if (const int64_t at = y - c0; at >= 0 && at < N) {  // the vector that holds the target
 #pragma unroll
         for (int j = 0; j < N; ++j)
-          if (j == (int)at) v[j] -= SC ? dy * th[j] : dy;
+          if (j == (int)at) v[j] -= SC ? dy * slope[j] : dy;
       }
     };
     each([](const T* p) { return load16_nt(p); },

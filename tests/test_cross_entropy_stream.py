@@ -143,3 +143,27 @@ def test_negative_softcap(dtype, softcap):
         out.append((o.loss.detach(), leaf.grad, o.predicted_tokens))
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("softcap", [3.0, 30.0, 50.0])
+def test_softcap_slope(dtype, softcap):
+    """Gradients of logits of up to 8 times the cap, where its slope 1 - tanh^2
+    falls to 5e-7: relative to the slope itself (2e-6 from its own evaluation
+    and 1e-5 of p), not to 1."""
+    V = 2048
+    level = torch.linspace(0.0, 8.0, V)
+    x = torch.stack([level, -level, level.flip(0)]).mul(softcap).to(dtype).cuda()
+    t = torch.tensor([V - 1, V - 1, 700], device="cuda")  # 8 sc, -8 sc and 5.3 sc
+    z = x.double().requires_grad_(True)
+    v = softcap * torch.tanh(z / softcap)
+    F.cross_entropy(v, t, reduction="sum").backward()
+    leaf = x.clone().requires_grad_(True)
+    forge_cross_entropy(leaf, t, softcap=softcap, reduction="sum").backward()
+    p = torch.softmax(v.detach(), -1)
+    slope = 1.0 / torch.cosh(x.double() / softcap) ** 2
+    # (exponent errors of 2^-22 of |v| log2 e <= 72 in p and its normalisation)
+    error = slope * (4e-5 * p + 4e-6 * F.one_hot(t, V))
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 1e-30
+    assert ((leaf.grad.double() - z.grad).abs() <= U[dtype] * z.grad.abs() * 1.01 + error + tiny).all()
