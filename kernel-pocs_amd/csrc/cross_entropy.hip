@@ -456,8 +456,8 @@ __device__ __forceinline__ bool ce_row_head(CeArgs& a, int64_t row, int64_t y, T
 // flight per thread.  Bound by the vector ALU as much as by memory: a softcap
 // row at 16-bit logits costs about 30 issue slots an element, so what the
 // flags switch is a template parameter or a branch per vector, never per
-// element, the divisions by the token count are folded into one scale and
-// shift, and the soft cap is a polynomial (cap_fast).  The second pass reads
+// element, the divisions of 16-bit gradients by the token count are folded into
+// one scale and shift, and the soft cap is a polynomial (cap_fast).  The second pass reads
 // the Infinity Cache (a bound on the workgroups per CU, so on the rows in
 // flight, measured equal).
 // Measured on MI355X, forward + backward, before -> after the vector ALU work
@@ -560,8 +560,8 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
   const float ls = a.label_smoothing;
   const float eps = ls / (float)V;
   const float wy = W ? a.weight[y] : 1.f;
-  float xy1[1] = {to_f32(xr[y])};
-  if constexpr (SC) cap<EXACT, 1>(xy1, sc, inv_sc);
+  float xy1[1] = {to_f32(xr[y])}, slope_y[1] = {1.f};
+  if constexpr (SC) cap<EXACT, true, 1>(xy1, slope_y, sc, inv_sc);
   const float xy = xy1[0];
 
   // ---- pass 1: online max / sum (log2 domain), argmax, smoothing sum ----
@@ -680,12 +680,27 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
   // ---- pass 2: gradient in place ----
   if (grads && ok) {
     const bool mean = a.flags & FORGE_CE_REDUCTION_MEAN;
-    const float inv_n = mean ? 1.f / a.n_non_ignore : 1.f;
+    const float n = mean ? a.n_non_ignore : 1.f, inv_n = 1.f / n;
     const float inv_snw = mean ? 1.f / a.sum_non_ignore_weight : 1.f;
     const float dz = 2.f * a.lse_square_scale * lse;
-    // without class weights: g = p scale - shift, less ydelta at the target
-    const float scale = (1.f + dz) * inv_n, shift = eps * inv_n, ydelta = (1.f - ls) * inv_n;
-    const float dy = W ? (1.f - ls) * wy * inv_snw : ydelta;
+    // p -> gradient, hit = 1 - smoothing at the target and 0 elsewhere.  Without
+    // class weights a 16-bit gradient away from the target is one fma, p scale -
+    // shift (within 2 fp32 ulps, far below its rounding); fp32 ones, and the
+    // target's, where p - 1 cancels, subtract first and divide.  The division is
+    // a product with the rounded reciprocal and one residual step (Markstein's:
+    // correctly rounded; a / costs fp32 rows 5 to 10%).
+    const float scale = (1.f + dz) * inv_n, shift = eps * inv_n;
+    auto grad = [&](float p, float w, float hit) {
+      if constexpr (!W) {
+        const float t = fmaf(dz, p, p) - eps - hit, q = t * inv_n;
+        return fmaf(fmaf(-q, n, t), inv_n, q);
+      } else {
+        const float ori = ((1.f - ls) * p - hit) * wy;
+        const float smooth = eps * (-w + p * a.weight_sum);
+        return ori * inv_snw + smooth * inv_snw + dz * p * inv_n;
+      }
+    };
+    const float gy = grad(fast_exp2(fmaf(xy, kLog2e, -m2)), wy, 1.f - ls) * slope_y[0];
     auto pass2 = [&](auto& v, int64_t c0) {
       constexpr int N = sizeof(v) / sizeof(float);
       float slope[N];  // of the cap
@@ -694,20 +709,15 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
       for (int j = 0; j < N; ++j) {
         const float p = fast_exp2(fmaf(v[j], kLog2e, -m2));
         float g;
-        if constexpr (!W) {
-          g = fmaf(p, scale, -shift);
-        } else {
-          const float ori = (1.f - ls) * p * wy;
-          const float smooth = eps * (-a.weight[c0 + j] + p * a.weight_sum);
-          g = ori * inv_snw + smooth * inv_snw + dz * p * inv_n;
-        }
+        if constexpr (!W && !EXACT) g = fmaf(p, scale, -shift);
+        else g = grad(p, W ? a.weight[c0 + j] : 1.f, 0.f);
         if constexpr (SC) g *= slope[j];
         v[j] = g;
       }
       if (const int64_t at = y - c0; at >= 0 && at < N) {  // the vector that holds the target
 #pragma unroll
         for (int j = 0; j < N; ++j)
-          if (j == (int)at) v[j] -= SC ? dy * slope[j] : dy;
+          if (j == (int)at) v[j] = gy;
       }
     };
     each([](const T* p) { return load16_nt(p); },

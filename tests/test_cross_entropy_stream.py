@@ -190,3 +190,25 @@ def test_softcap_of_mixed_sizes(dtype, softcap):
     p = torch.softmax(v.detach(), -1)
     error = 1e-5 * p + 4e-6 * F.one_hot(t, V) + (2.0 ** -24 if dtype == torch.float16 else 1e-30)
     assert ((leaf.grad.double() - z.grad).abs() <= U[dtype] * z.grad.abs() * 1.01 + error).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("softcap,smoothing", [(None, 0.0), (None, 0.1), (30.0, 0.0)])
+def test_fp32_mean_is_the_sum_divided(softcap, smoothing):
+    """fp32 gradients of the mean are those of the sum divided by the token
+    count with one rounding, the target's too, where p - 1 cancels."""
+    gen = torch.Generator().manual_seed(10)
+    n, V = 7, 4099
+    x = (torch.randn(n, V, generator=gen) * 2).cuda()
+    t = torch.randint(0, V, (n,), generator=gen).cuda()
+    x[torch.arange(4), t[:4]] += 20.0  # confident rows: p within 1e-5 of 1
+    grads = []
+    for reduction in ("mean", "sum"):
+        leaf = x.clone().requires_grad_(True)
+        forge_cross_entropy(leaf, t, softcap=softcap, label_smoothing=smoothing, reduction=reduction).backward()
+        grads.append(leaf.grad.cpu())
+    want = grads[1] / torch.full_like(grads[1], n)  # (a scalar divisor may become a product with its reciprocal)
+    if softcap is None:
+        assert torch.equal(grads[0], want)
+    else:  # the cap's slope comes after the division in one and before it in the other: four roundings of 2^-24
+        assert ((grads[0] - want).abs() <= 2.0 ** -22 * want.abs() + 1e-44).all()
