@@ -134,9 +134,9 @@ __device__ __forceinline__ void block_lse(float& m, float& d, float* red) {
   for (int i = 1; i < NW; ++i) lse_merge(m, d, red[2 * i], red[2 * i + 1]);
 }
 
-// (max value, first index) reduction for argmax.
+// (max value, first index) reduction for argmax; v becomes the largest value.
 template <int NW>
-__device__ __forceinline__ int64_t block_argmax(float v, int64_t idx, float* redf, int64_t* redi) {
+__device__ __forceinline__ int64_t block_argmax(float& v, int64_t idx, float* redf, int64_t* redi) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     float v2 = __shfl_xor(v, off, 64);
@@ -570,17 +570,18 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
   const bool bounded = SC && !EXACT && sc <= 40.f;
   float m = bounded ? sc * kLog2e : -INFINITY, d = 0.f, sxs = 0.f, amax_v = -INFINITY;
   int64_t amax_i = V;
-  auto pass1 = [&](auto& v, int64_t c0) {
+  Vec16<T> amax_x;  // the vector at amax_i
+  auto pass1 = [&](auto& v, int64_t c0, const Vec16<T>& raw) {
     constexpr int N = sizeof(v) / sizeof(float);
     if constexpr (ARG) {
-      // the first vector that holds this thread's largest logit (its place in
-      // the vector is looked up after the pass).  Logits are compared before a
+      // the first vector that holds this thread's largest logit, kept: its place
+      // in the vector is looked up after the pass.  Logits are compared before a
       // fast cap, whose order they share (see below), and after an exact one.
       if constexpr (SC && EXACT) cap<EXACT, N>(v, sc, inv_sc);
       float t = v[0];
 #pragma unroll
       for (int j = 1; j < N; ++j) t = fmaxf(t, v[j]);
-      if (t > amax_v) { amax_v = t; amax_i = c0; }
+      if (t > amax_v) { amax_v = t; amax_i = c0; amax_x = raw; }
     }
     if constexpr (SC && !(ARG && EXACT)) cap<EXACT, N>(v, sc, inv_sc);
     if (ls > 0.f) {
@@ -625,17 +626,17 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
   auto fwd = [&](const Vec16<T>& raw, int64_t i) {
     float v[VEC];
     unpack(raw, v);
-    pass1(v, head + i * VEC);
+    pass1(v, head + i * VEC, raw);
   };
   if (tid < edge && tid < head) {
     float v[1] = {to_f32(xr[ecol])};
-    pass1(v, ecol);
+    pass1(v, ecol, Vec16<T>{});
   }
   if (grads) each([](const T* p) { return load16(p); }, fwd);  // read again below: kept cached
   else each([](const T* p) { return load16_nt(p); }, fwd);
   if (tid < edge && tid >= head) {
     float v[1] = {to_f32(xr[ecol])};
-    pass1(v, ecol);
+    pass1(v, ecol, Vec16<T>{});
   }
   block_lse<NW>(m, d, redf);
   float sxs_tot = 0.f;
@@ -644,7 +645,7 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
   if constexpr (ARG) {
     if (amax_i >= head && amax_i < head + nvec * VEC) {  // a vector: its first element with that value
       float v[VEC];
-      unpack(load16(xr + amax_i), v);
+      unpack(amax_x, v);
       if constexpr (SC && EXACT) cap<EXACT, VEC>(v, sc, inv_sc);
       int j0 = 0;
 #pragma unroll
@@ -659,8 +660,7 @@ __global__ __launch_bounds__(NT) void ce_stream_kernel(CeArgs a) {
       // apart or more, 40 fp32 ulps after the cap), so the largest logit is
       // the one; past it distinct logits may cap to one value, and the row is
       // searched again with the exact cap.
-      const float top = block_max<NW>(amax_v, redf);
-      if (!(fabsf(top) <= 4.f * sc)) {
+      if (!(fabsf(amax_v) <= 4.f * sc)) {
         amax_v = -INFINITY;
         amax_i = V;
         for (int64_t c = tid; c < V; c += NT) {
