@@ -956,18 +956,26 @@ void ce_resident_kernel(CeArgs a) {
 
 template <class T, bool SC, bool W>
 void launch_stream_sw(const CeArgs& a, dim3 grid, hipStream_t s) {
-  // Long rows take 1024 threads: half the rows in flight, which the second
-  // pass still finds in the Infinity Cache.  Measured on MI355X, 512 against
+  // Rows of up to 32 KB take 256 threads: a row's time there is its workgroup's
+  // barriers and reductions, and more threads than vectors only add to them.
+  // Measured on MI355X, 8192 rows, 512 against 256 threads: bf16 257 columns 59
+  // / 24 us, 4096 with accuracy and predictions 75 / 32, 16384 with softcap 150
+  // / 118; fp32 4096 73 / 47, 8192 115 / 102; 16384 213 / 230.
+  // Long rows take 1024: half the rows in flight, which the second
+  // pass still finds in the Infinity Cache.  512 against
   // 1024 threads: [2048, 256000] fp32 1040 / 898 us, [4096, 128256] fp32 890
   // / 866, [4096, 151936] bf16 550 / 532, [8192, 50257] bf16 386 / 392.  With
   // a softcap the arithmetic holds the kernel and the smaller workgroups'
   // barriers cost less: [2048, 256000] bf16 494 / 519, [4096, 32000] 146 / 184.
-  const bool wide = !SC && a.n_cols * (int64_t)sizeof(T) >= 256 * 1024;
+  const int64_t bytes = a.n_cols * (int64_t)sizeof(T);
+  const bool wide = !SC && bytes >= 256 * 1024;
   if (a.flags & (FORGE_CE_RETURN_ACCURACY | FORGE_CE_RETURN_PREDICTED)) {
-    if (wide) ce_stream_kernel<T, 1024, SC, W, true><<<grid, 1024, 0, s>>>(a);
+    if (bytes <= 32 * 1024) ce_stream_kernel<T, 256, SC, W, true><<<grid, 256, 0, s>>>(a);
+    else if (wide) ce_stream_kernel<T, 1024, SC, W, true><<<grid, 1024, 0, s>>>(a);
     else ce_stream_kernel<T, 512, SC, W, true><<<grid, 512, 0, s>>>(a);
   } else {
-    if (wide) ce_stream_kernel<T, 1024, SC, W, false><<<grid, 1024, 0, s>>>(a);
+    if (bytes <= 32 * 1024) ce_stream_kernel<T, 256, SC, W, false><<<grid, 256, 0, s>>>(a);
+    else if (wide) ce_stream_kernel<T, 1024, SC, W, false><<<grid, 1024, 0, s>>>(a);
     else ce_stream_kernel<T, 512, SC, W, false><<<grid, 512, 0, s>>>(a);
   }
 }

@@ -212,3 +212,25 @@ def test_fp32_mean_is_the_sum_divided(softcap, smoothing):
         assert torch.equal(grads[0], want)
     else:  # the cap's slope comes after the division in one and before it in the other: four roundings of 2^-24
         assert ((grads[0] - want).abs() <= 2.0 ** -22 * want.abs() + 1e-44).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,V,n", [(torch.bfloat16, 16384, 3), (torch.bfloat16, 16385, 3), (torch.float32, 8192, 3),
+                                       (torch.float32, 8193, 3), (torch.bfloat16, 17, 3001), (torch.float32, 2, 600)])
+@pytest.mark.parametrize("softcap", [None, 30.0])
+def test_workgroup_sizes(dtype, V, n, softcap):
+    """Either side of the row size that changes the workgroup, and more rows
+    than threads for the workgroup that sums the losses."""
+    gen = torch.Generator().manual_seed(V)
+    x = (torch.randn(n, V, generator=gen) * 3).to(dtype).cuda()
+    t = torch.randint(0, V, (n,), generator=gen).cuda()
+    loss, grad, v = _reference(x, t, softcap, 0.0, None)
+    leaf = x.clone().requires_grad_(True)
+    o = forge_cross_entropy(leaf, t, softcap=softcap, return_predicted_tokens=True, return_token_accuracy=True)
+    o.loss.backward()
+    assert abs(o.loss.double() - loss) <= U[dtype] * abs(loss) + 1e-5
+    error = 2e-5 * torch.softmax(v, -1) / n + 2.0 ** -22 * F.one_hot(t, V) / n
+    assert ((leaf.grad.double() - grad).abs() <= U[dtype] * grad.abs() * 1.01 + error + 1e-12).all()
+    first = (x == x.amax(-1, keepdim=True)).int().argmax(-1)
+    assert torch.equal(o.predicted_tokens, first)
+    assert abs(o.token_accuracy.item() - (first == t).float().mean().item()) < 1e-6
