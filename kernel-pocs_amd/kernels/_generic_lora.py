@@ -90,8 +90,11 @@ _MAX_SEGS = 6  # K segments of one product (csrc/gemm_core.h)
 
 def _one_product(terms, out: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """sum of a @ b over terms as one fp16 product of as many K segments, or
-    None where the MFMA core does not take them all in the same layouts."""
+    None where the MFMA core does not take them all in the same layouts, or an
+    `out` that is not fp16 with unit stride along its rows (left to gmm)."""
     M, N = terms[0][0].shape[0], terms[0][1].shape[1]
+    if out is not None and (out.dtype != torch.float16 or out.stride(1) != 1 and N != 1):
+        return None
     lay = [_mfma_layouts(a, b) for a, b in terms]
     if M == 0 or N == 0 or len(terms) > _MAX_SEGS or any(v is None or v[0::2] != lay[0][0::2] for v in lay):
         return None

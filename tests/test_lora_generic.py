@@ -201,3 +201,23 @@ def test_lora_qkv_rope_fp32_matches_oracle(head_dim):
     got = [x.grad] + [p[i].grad for i in (3, 4, 6, 7, 9, 10)]
     for n, a, b in zip(QKV_NAMES, got, ref_grads):
         close(a, b, n, torch.float32)
+
+
+def test_joined_products_write_only_the_output_they_can(monkeypatch):
+    """Products joined as K segments store fp16 rows of unit stride: another
+    kind of `out` goes to the general product, which converts or refuses it
+    (CPU: nothing is launched)."""
+    from kernels import _generic_lora as gl
+
+    launched = []
+    monkeypatch.setattr(gl.L, "forge_gemm_f16", lambda *a: launched.append(a) or 0)
+    monkeypatch.setattr(gl.L, "stream_of", lambda t: None)
+    a, w = torch.zeros(16, 64, dtype=torch.float16), torch.zeros(24, 64, dtype=torch.float16)
+    terms = [(a, w.t()), (a, w.t())]
+    good = torch.empty(16, 24, dtype=torch.float16)
+    assert gl._one_product(terms, good) is good and len(launched) == 1
+    assert gl._one_product(terms, torch.empty(16, 24)) is None                               # fp32
+    assert gl._one_product(terms, torch.empty(24, 16, dtype=torch.float16).t()) is None      # columns of unit stride
+    assert gl._one_product(terms, torch.empty(16, 48, dtype=torch.float16)[:, ::2]) is None  # every other column
+    assert len(launched) == 1
+    pytest.raises(AssertionError, gl.gmm_sum, [(a, w.t())], out=torch.empty(24, 16, dtype=torch.float16).t())
