@@ -5,16 +5,34 @@
 
 namespace fgemm {
 
+// 33 .. 64 rows of K-contiguous operands take the big tiles instead of two rows
+// of 32-row ones (a register engine) where the caller split them over K, and,
+// of the products whose big-tile epilogue moves vectors, where the 32-row tiles
+// no longer fit on 256 CUs at once and where a short product is added to a
+// 16-bit C (whose traffic is the cost).  Measured on MI355X, 64 rows, 32-row
+// against big tiles: [4096], K = 14336 240 / 45 us split 16 ways, 260 unsplit;
+// unsplit, K = 4096: [4096] 61 / 76, with SiLU 62 / 140, fp32 atomics 68 / 182,
+// [32000] 92 / 93, [40960] 152 / 98, [128256] 341 / 228; added to C, K = 64:
+// [4096] 13 / 10, K = 256 [14336] 15 / 14, K = 1024 [1024] 23 / 28.
+static bool few_rows_big(int64_t N, int epi, const GemmArgs& a) {
+  if (a.split_k > 1) return epi == EPI_STORE_F32;
+  const bool linear = a.ep.act == ACT_NONE && a.ep.alpha_group == 0;
+  if (!a.ep.vec_ok || (epi != EPI_STORE_F32 && !(epi == EPI_STORE_BF16 && linear))) return false;
+  int64_t k = 0;
+  for (int i = 0; i < a.n_segs; ++i) k += a.segs[i].k;
+  return 2 * ((N + 255) / 256) > 256 || (epi == EPI_STORE_BF16 && a.ep.beta != 0.f && k <= 256);
+}
+
 // Picks a tile shape from the output shape (a K-contiguous A takes the
-// 64-row narrow tiles up to N = 256).  33 .. 64 rows of K-contiguous
-// operands take the big tiles, which the caller splits over K: [64, 4096], K =
-// 14336 240 -> 45 us on MI355X (the 32-row tiles' register engine before).
-static int pick_cfg(int64_t M, int64_t N, int al, int bl) {
+// 64-row narrow tiles up to N = 256).
+static int pick_cfg(int64_t N, int al, int bl, int epi, const GemmArgs& a) {
+  const int64_t M = a.M;
   if (al == ROW && (bl == COL || bl == ROW) && N <= 256 && M > N)
     return N <= 64 ? CFG_SKINNY_N64 : N <= 128 ? CFG_NARROW_128 : (N <= 192 && bl == COL) ? CFG_NARROW_192 : CFG_NARROW_256;
   if (N <= 32 && M > N) return CFG_SKINNY_N;
   if (N <= 64 && M > N) return CFG_SKINNY_N64;
-  if (M <= 64 && N > M && !(M > 32 && N > 256 && al == ROW && bl == COL)) return CFG_SKINNY_M;
+  if (M > 32 && M <= 64 && N > 256 && al == ROW && bl == COL && few_rows_big(N, epi, a)) return CFG_BIG;
+  if (M <= 64 && N > M) return CFG_SKINNY_M;
   return CFG_BIG;
 }
 
@@ -46,7 +64,7 @@ static int check_segs(const GemmArgs& a, int al, int bl) {
   return FORGE_OK;
 }
 
-int run(int cfg, int al, int bl, int epi, const GemmArgs& args, hipStream_t s) {
+int run(int64_t width, int al, int bl, int epi, const GemmArgs& args, hipStream_t s) {
   if (int e = check_segs(args, al, bl)) return e;
   // 16-byte vector epilogue when every buffer it touches allows it
   GemmArgs a = args;
@@ -65,7 +83,7 @@ int run(int cfg, int al, int bl, int epi, const GemmArgs& args, hipStream_t s) {
     return forge_set_error(FORGE_ERR_INVALID, "gemm: [K][N] B layout needs N %% 8 == 0 (N=%lld)", (long long)a.N);
   if (a.M == 0 || a.N == 0) return FORGE_OK;
   if (al == ROW && bl == COL && rows_engine(epi, a)) return launch_rows(epi, a, s);
-  if (cfg < 0) cfg = pick_cfg(a.M, a.N, al, bl);
+  const int cfg = pick_cfg(width > 0 ? width : a.N, al, bl, epi, a);
   if (a.f16) return launch_f16(epi, cfg, al, bl, a, s);
   switch (epi) {
     case EPI_STORE_BF16: return launch_store_bf16(cfg, al, bl, a, s);
@@ -119,9 +137,6 @@ static int gemm_entry(int dtype, int64_t M, int64_t N, const forge_gemm_segment*
     }
     if (a.segs[i].n_hi - a.segs[i].n_lo > width) width = a.segs[i].n_hi - a.segs[i].n_lo;
   }
-  // column-ranged segments: tiles sized for the widest range, so that
-  // independent products side by side get tiles of their own
-  const int cfg = ranged ? pick_cfg(M, width, a_layout, b_layout) : -1;
   a.split_k = split_k;
   a.ep.c = c;
   a.ep.ldc = ldc;
@@ -155,7 +170,9 @@ static int gemm_entry(int dtype, int64_t M, int64_t N, const forge_gemm_segment*
   } else {
     return forge_set_error(FORGE_ERR_INVALID, "gemm: epilogue %d", epilogue);
   }
-  return run(cfg, a_layout, b_layout, epi, a, (hipStream_t)stream);
+  // column-ranged segments: tiles sized for the widest range, so that
+  // independent products side by side get tiles of their own
+  return run(ranged ? width : 0, a_layout, b_layout, epi, a, (hipStream_t)stream);
 }
 
 extern "C" int forge_gemm(int64_t M, int64_t N, const forge_gemm_segment* segs, int n_segs,

@@ -1460,7 +1460,8 @@ void gemm_dma_kernel(GemmArgs args) {
   }
 }
 
-// Launches one GEMM with tile config `cfg` (-1 = pick from the shape).
-int run(int cfg, int a_layout, int b_layout, int epi, const GemmArgs& a, hipStream_t s);
+// Launches one GEMM on tiles picked from its shape; width: the columns to size
+// them for (0: N).
+int run(int64_t width, int a_layout, int b_layout, int epi, const GemmArgs& a, hipStream_t s);
 
 }  // namespace fgemm

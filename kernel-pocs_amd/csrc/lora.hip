@@ -301,7 +301,7 @@ static int gate_up(int64_t M, int64_t H, int64_t I, int64_t r, const void* x, in
     a.ep.vbt_ld = ld_ad;
     a.ep.vr = (int)rd;
   }
-  return run(-1, ROW, COL, epi, a, (hipStream_t)stream);
+  return run(0, ROW, COL, epi, a, (hipStream_t)stream);
 }
 
 extern "C" int forge_lora_mlp_gate_up(int64_t M, int64_t H, int64_t I, int64_t r,
@@ -381,7 +381,7 @@ static int down_bwd(int64_t M, int64_t H, int64_t I, int64_t r, const void* dy, 
       a.ep.wxt_ld = ld_xat;
     }
   }
-  return run(-1, ROW, w_layout, epi, a, (hipStream_t)stream);
+  return run(0, ROW, w_layout, epi, a, (hipStream_t)stream);
 }
 
 extern "C" int forge_lora_mlp_down_bwd(int64_t M, int64_t H, int64_t I, int64_t r,
@@ -484,8 +484,8 @@ extern "C" int forge_lora_qkv_rope(int64_t M, int64_t K, int64_t hq, int64_t hkv
   a.ep.positions = positions;
   a.ep.rope_cols = apply_rope ? k1 : 0;
   a.ep.head_dim = (int)(head_dim > 0 ? head_dim : 128);
-  if (!apply_rope) return run(-1, ROW, COL, EPI_STORE_BF16, a, (hipStream_t)stream);
-  return run(-1, ROW, COL, EPI_ROPE, a, (hipStream_t)stream);
+  if (!apply_rope) return run(0, ROW, COL, EPI_STORE_BF16, a, (hipStream_t)stream);
+  return run(0, ROW, COL, EPI_ROPE, a, (hipStream_t)stream);
 }
 
 
@@ -599,16 +599,15 @@ extern "C" int forge_lora_a(int64_t M, int64_t K, int64_t r, int n_proj, const v
   // fill the chip): split z writes fp32 partial sums to work[z]
   // ([split_k][M][N]), which one reduction pass sums in a fixed order
   // (deterministic) and rounds to bf16.
-  const int cfg = -1;  // the narrow K-contiguous tiles (64 x N, N up to 256) picked from the shape
   if (split_k <= 1) {
     a.ep.c = out;
     a.ep.ldc = ld_out;
-    return run(cfg, ROW, COL, EPI_STORE_BF16, a, s);
+    return run(0, ROW, COL, EPI_STORE_BF16, a, s);
   }
   a.ep.c = work;
   a.ep.ldc = N;
   a.ep.split_stride = M * N;
-  if (int e = run(cfg, ROW, COL, EPI_STORE_F32, a, s)) return e;
+  if (int e = run(0, ROW, COL, EPI_STORE_F32, a, s)) return e;
   return forge_splitk_reduce(work, M * N, split_k, M, N, N, out, ld_out, FORGE_DTYPE_BF16, 1.0f, stream);
 }
 

@@ -111,3 +111,31 @@ def test_null_operands_read_as_zeros(M):
                              L.stream_of(c)), "forge_gemm")
         assert not c.any()
         c.fill_(7.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [33, 64])
+@pytest.mark.parametrize("N,K", [(264, 64), (1000, 512), (32768, 72), (32776, 72)])
+@pytest.mark.parametrize("c_dtype,epi", [(torch.bfloat16, L.EPI_STORE), (torch.bfloat16, L.EPI_SILU),
+                                         (torch.float32, L.EPI_STORE), (torch.float32, L.EPI_SILU),
+                                         (torch.float32, L.EPI_ATOMIC_F32)])
+def test_unsplit_33_to_64_rows(M, N, K, c_dtype, epi):
+    """Either side of the lines of the rule that picks 32-row or 256-row
+    tiles: column counts, K, epilogues, a C that is added to, and a pitch
+    that rules out vectors."""
+    gen = torch.Generator().manual_seed(N)
+    a, b = _mat(M, K, gen), _mat(N, K, gen) * K ** -0.5
+    prod, mag = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    seg = (L.GemmSegment * 1)(L.GemmSegment(a.data_ptr(), K, b.data_ptr(), K, K, 0, 0))
+    for beta, pad in ((0.0, 0), (1.0, 0), (0.0, 3)):
+        c = torch.randn(M, N + pad, generator=gen).to(c_dtype).cuda()
+        c0 = c.double()[:, :N]
+        L.check(L.forge_gemm(M, N, seg, 1, ROW, COL, c.data_ptr(), N + pad, L.dtype_code(c_dtype), 1.0, beta, epi, 1,
+                             L.stream_of(c)), "forge_gemm")
+        ref = prod + (c0 if epi == L.EPI_ATOMIC_F32 else beta * c0)
+        if epi == L.EPI_SILU:
+            ref = torch.nn.functional.silu(ref)
+        ulp = U.get(c_dtype, 2.0 ** -24)
+        # (1.1: the activation's slope; 1e-6: its own fp32 evaluation)
+        bound = ulp * ref.abs() * 1.01 + 1.1 * (K + 2) * 2.0 ** -24 * (mag + c0.abs()) + 1e-6
+        assert ((c.double()[:, :N] - ref).abs() <= bound).all(), (beta, pad)
