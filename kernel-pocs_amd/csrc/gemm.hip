@@ -18,9 +18,9 @@ static bool few_rows_big(int64_t N, int epi, const GemmArgs& a) {
   if (a.split_k > 1) return epi == EPI_STORE_F32;
   const bool linear = a.ep.act == ACT_NONE && a.ep.alpha_group == 0;
   if (!a.ep.vec_ok || (epi != EPI_STORE_F32 && !(epi == EPI_STORE_BF16 && linear))) return false;
-  int64_t k = 0;
-  for (int i = 0; i < a.n_segs; ++i) k += a.segs[i].k;
-  return 2 * ((N + 255) / 256) > 256 || (epi == EPI_STORE_BF16 && a.ep.beta != 0.f && k <= 256);
+  const bool short_k = total_k(a) <= 256;
+  if (2 * ((N + 255) / 256) > 256) return linear || !short_k;
+  return epi == EPI_STORE_BF16 && a.ep.beta != 0.f && short_k;
 }
 
 // Picks a tile shape from the output shape (a K-contiguous A takes the

@@ -84,12 +84,37 @@ static void order_columns(GemmArgs& a, int64_t out_bn, int64_t tn) {
   for (int j = 0; j < tn; ++j) a.col_order[j] = (uint8_t)idx[j];
 }
 
-// The 4-wave engine's epilogue through LDS: 16-byte vectors, and of the 16-bit
-// stores the plain one (alpha alone).
-template <int EPI>
-static bool w4_staged_launch(const GemmArgs& a) {
-  const bool plain = a.ep.beta == 0.f && a.ep.act == ACT_NONE && a.ep.alpha_group == 0;
-  return w4_staged_epi(EPI) && a.ep.vec_ok && (EPI != EPI_STORE_BF16 || plain);
+static bool plain_store(const GemmArgs& a) { return a.ep.beta == 0.f && a.ep.act == ACT_NONE && a.ep.alpha_group == 0; }
+
+static int64_t total_k(const GemmArgs& a) {
+  int64_t k = 0;
+  for (int i = 0; i < a.n_segs; ++i) k += a.segs[i].k;
+  return k;
+}
+
+// Launches the 4-wave engine with its epilogue through LDS, or returns false:
+// it needs 16-byte vectors, and of the 16-bit stores takes the plain one.  A^T B
+// added to an fp32 C stays on 8 waves, whose two waves a SIMD cover each other's
+// reads of C, where the reduction is short or an activation follows.  Measured
+// on MI355X, 8 against 4 waves: [8192, 4096] K = 64 71 / 76 us, with GELU 71 /
+// 90, [512, 4096] K = 64 19 / 23, [1024, 1024] K = 1024 39 / 45, [4096, 4096] K
+// = 4096 152 / 131.
+template <class T, int BMODE, int EPI, bool AT, bool BT>
+static bool launch_w4_staged(const GemmArgs& a, dim3 grid, hipStream_t s) {
+  if constexpr (w4_staged_epi(EPI)) {
+    if (!a.ep.vec_ok) return false;
+    if constexpr (EPI == EPI_STORE_F32) {
+      if (!plain_store(a)) {
+        if (AT && a.ep.beta != 0.f && (a.ep.act != ACT_NONE || total_k(a) <= 1024)) return false;
+        gemm_w4_kernel<T, BMODE, EPI, true, AT, BT, false><<<grid, 256, 0, s>>>(a);
+        return true;
+      }
+    }
+    if (EPI == EPI_STORE_BF16 && !plain_store(a)) return false;
+    gemm_w4_kernel<T, BMODE, EPI, true, AT, BT><<<grid, 256, 0, s>>>(a);
+    return true;
+  }
+  return false;
 }
 
 template <class T, int BM, int BN, int WM, int WN, int AL, int BL, int BMODE, int EPI>
@@ -105,10 +130,8 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
   if constexpr (BM == 256 && BN == 256 && AL == ROW && BL == COL) {
     // both operands K-contiguous: the 4-wave engine (128 x 128 per wave,
     // accumulators in AGPRs, a ring of five LDS half-slots fed by LDS-DMA)
-    constexpr bool W4_STAGE = w4_staged_epi(EPI);
-    if (w4_staged_launch<EPI>(a))
-      gemm_w4_kernel<T, BMODE, EPI, W4_STAGE><<<grid, 256, 0, s>>>(a);
-    else if (EPI == EPI_STORE_BF16 && a.ep.vec_ok && a.ep.beta != 0.f)
+    if (launch_w4_staged<T, BMODE, EPI, false, false>(a, grid, s)) {
+    } else if (EPI == EPI_STORE_BF16 && a.ep.vec_ok && a.ep.beta != 0.f)
       // beta reads C before the single rounding: the fp32-staged epilogue of
       // the 8-wave engine moves it as 16-byte vectors (rank-r products added
       // to a base product: K is short and C's traffic is the cost)
@@ -143,9 +166,8 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
     // B as stored [K][N]: the 4-wave engine with transposing fragment reads of
     // B; C read (beta) or stored by elements: the 8-wave LDS-DMA engine
     constexpr bool DMA_STAGE = staged_ok(BM, BN, 4, 2, EPI);
-    if (w4_staged_launch<EPI>(a))
-      gemm_w4_kernel<T, BMODE, EPI, true, false, true><<<grid, 256, 0, s>>>(a);
-    else if (DMA_STAGE && a.ep.vec_ok)
+    if (launch_w4_staged<T, BMODE, EPI, false, true>(a, grid, s)) {
+    } else if (DMA_STAGE && a.ep.vec_ok)
       gemm_dma_kernel<T, BM, BN, 4, 2, BMODE, EPI, 64, 2, DMA_STAGE, 2, false, true><<<grid, 512, 0, s>>>(a);
     else
       gemm_dma_kernel<T, BM, BN, 4, 2, BMODE, EPI, 64, 2, false, 2, false, true><<<grid, 512, 0, s>>>(a);
@@ -154,14 +176,8 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
     // transposing fragment reads of both
     constexpr int DWM = 4, DWN = 2;
     constexpr bool DMA_STAGE = staged_ok(BM, BN, DWM, DWN, EPI);
-    if constexpr (w4_staged_epi(EPI)) {
-      if (w4_staged_launch<EPI>(a)) {
-        gemm_w4_kernel<T, BMODE, EPI, true, true, true><<<grid, 256, 0, s>>>(a);
-        FORGE_CHECK_LAUNCH();
-        return FORGE_OK;
-      }
-    }
-    if (DMA_STAGE && a.ep.vec_ok)
+    if (launch_w4_staged<T, BMODE, EPI, true, true>(a, grid, s)) {
+    } else if (DMA_STAGE && a.ep.vec_ok)
       gemm_dma_kernel<T, BM, BN, DWM, DWN, BMODE, EPI, 64, 2, DMA_STAGE, 2, true, true><<<grid, DWM * DWN * 64, 0, s>>>(a);
     else
       gemm_dma_kernel<T, BM, BN, DWM, DWN, BMODE, EPI, 64, 2, false, 2, true, true><<<grid, DWM * DWN * 64, 0, s>>>(a);

@@ -223,7 +223,7 @@ __device__ __forceinline__ int w4t_lane_offset(int r0, int lane) {
 constexpr int W4_NHALF = 5;
 constexpr int W4_HALF = 256 * 64 * 2;  // bytes per half-slot
 
-template <class T, int BMODE, int EPI, bool STAGED, bool AT = false, bool BT = false>
+template <class T, int BMODE, int EPI, bool STAGED, bool AT = false, bool BT = false, bool PLAIN = true>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_w4_kernel(GemmArgs args) {
   constexpr int BM = 256, BN = 256, WAVES_M = 2, WAVES_N = 2, BKT = 64;
@@ -464,7 +464,7 @@ void gemm_w4_kernel(GemmArgs args) {
     static_assert(RING >= W4_F32_BYTES, "the fp32 epilogue's slabs reuse the ring");
     __bf16* lds = reinterpret_cast<__bf16*>(smem);
     if constexpr (EPI == EPI_STORE_F32)
-      w4_epilogue_f32(args, acc, m0, n0, elane, ewm, ewn, reinterpret_cast<float*>(smem));
+      w4_epilogue_f32<PLAIN>(args, acc, m0, n0, elane, ewm, ewn, reinterpret_cast<float*>(smem));
     else if constexpr (BMODE == B_DUAL)
       w4_epilogue_staged_dual<EPI>(args, acc, m0, n0, elane, ewm, ewn, lds);
     else  // (STORE_BF16 is launched staged at beta = 0 only)

@@ -167,11 +167,16 @@ __device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x4 (
 // [2048, 8192], K = 2048 split 8 ways 829 -> 304 us; [1003, 4096], K = 14336
 // split 4 ways 176 -> 110 us; [256, 4096], K = 4096 split 8 ways 87 -> 33 us
 // (with every case unrolled in one loop the last two took 130 and 52 us: the
-// code outgrew the instruction cache).
+// code outgrew the instruction cache); [4096, 4096], K = 64 added to C 40 -> 32
+// us, with SiLU 65 -> 25 (a row at a time and an element at a time before).
 // ---------------------------------------------------------------------------
 constexpr int W4_FP = 128 + 4;                      // floats per staged row (4 banks apart)
 constexpr int W4_F32_BYTES = 4 * 2 * 32 * W4_FP * 4;  // 4 waves x 2 slabs of 32 rows
 
+// PLAIN: alpha alone, whole rows (the other forms have a kernel of their own:
+// with their code between the plain stores every launch fetches it too, 5 us of
+// 16 at [2048, 4096], K = 16).
+template <bool PLAIN>
 __device__ __forceinline__ void w4_epilogue_f32(const GemmArgs& args, f32x4 (&acc)[8][8], int64_t m0, int64_t n0,
                                                 int lane, int wm, int wn, float* lds) {
   const EpiArgs& ep = args.ep;
@@ -182,8 +187,12 @@ __device__ __forceinline__ void w4_epilogue_f32(const GemmArgs& args, f32x4 (&ac
   const int c = (lane % 32) * 4;
   const int64_t n = n0 + wn * 128 + c;
   float* cbase = (float*)ep.c + (int64_t)blockIdx.z * ep.split_stride;
-  const bool plain = ep.beta == 0.f && !ep.act && ep.alpha_group == 0 && n0 + 256 <= N;
-  const float alpha = ep.alpha_group == 0 ? ep.alpha : 1.f;
+  const bool whole = n0 + 256 <= N, full = n + 4 <= N;
+  const float alpha = PLAIN || ep.alpha_group == 0 ? ep.alpha : 1.f;
+  float al[4];  // per-column alphas, where the accumulators were not scaled on their way to LDS
+  if constexpr (!PLAIN)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) al[q] = ep.alpha_group > 0 ? col_alpha(ep, n + q) : 1.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float* slab = base + (i & 1) * 32 * W4_FP;
@@ -196,40 +205,94 @@ __device__ __forceinline__ void w4_epilogue_f32(const GemmArgs& args, f32x4 (&ac
         *reinterpret_cast<f32x4*>(slab + (16 * h + lane % 16) * W4_FP + 16 * j + cl) = alpha * acc[2 * i + h][j];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's slab is written
     const int64_t mb = m0 + wm * 128 + i * 32;
-    if (plain) {  // a store per row run, nothing read
+    if constexpr (PLAIN) {  // a store per row run, nothing read
+      if (whole) {
 #pragma unroll
-      for (int it = 0; it < 16; ++it) {
-        const int rr = it * 2 + lane / 32;
-        const float4 v = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
-        if (mb + rr < M)
-          *reinterpret_cast<float4*>(cbase + (mb + rr) * ep.ldc + n) = v;
+        for (int it = 0; it < 16; ++it) {
+          const int rr = it * 2 + lane / 32;
+          const float4 v = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
+          if (mb + rr < M)
+            *reinterpret_cast<float4*>(cbase + (mb + rr) * ep.ldc + n) = v;
+        }
+      } else {  // the last columns of a ragged N
+#pragma unroll 1
+        for (int it = 0; it < 16; ++it) {
+          const int rr = it * 2 + lane / 32;
+          float* cp = cbase + (mb + rr) * ep.ldc + n;
+          if (mb + rr >= M) continue;
+          if (full) {
+            *reinterpret_cast<float4*>(cp) = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
+          } else {
+#pragma unroll 1
+            for (int q = 0; q < 4 && n + q < N; ++q) cp[q] = slab[rr * W4_FP + c + q];
+          }
+        }
       }
       continue;
     }
-    // beta, activations, per-column alphas and the last columns of a ragged N
-    // (loops kept rolled: unrolled, this code is fetched from memory by every
-    // launch and costs more than the stores)
+    // beta, per-column alphas, activations and the last columns of a ragged N.
+    // The eight reads of C in a batch are in flight together; activations come
+    // after, in a rolled loop (unrolled, their code is fetched from memory by
+    // every launch and costs more than the stores).
+    if (full) {
+      if (ep.beta != 0.f || ep.alpha_group > 0 || !ep.act) {
 #pragma unroll 1
-    for (int it = 0; it < 16; ++it) {
-      const int rr = it * 2 + lane / 32;
-      float* cp = cbase + (mb + rr) * ep.ldc + n;
-      if (mb + rr >= M) continue;
-      if (n + 4 <= N && !ep.act && ep.alpha_group == 0) {  // 16-byte aligned: ldc % 8 == 0
-        float4* c4 = reinterpret_cast<float4*>(cp);
-        float4 v = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
-        if (ep.beta != 0.f) {
-          const float4 o = *c4;
-          v.x += ep.beta * o.x; v.y += ep.beta * o.y; v.z += ep.beta * o.z; v.w += ep.beta * o.w;
+        for (int it0 = 0; it0 < 16; it0 += 8) {
+          float4 o[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const int rr = (it0 + u) * 2 + lane / 32;
+            o[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (ep.beta != 0.f && mb + rr < M)
+              o[u] = *reinterpret_cast<const float4*>(cbase + (mb + rr) * ep.ldc + n);
+          }
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const int rr = (it0 + u) * 2 + lane / 32;
+            float4* sp = reinterpret_cast<float4*>(slab + rr * W4_FP + c);
+            float4 v = *sp;
+            if (ep.alpha_group > 0) { v.x *= al[0]; v.y *= al[1]; v.z *= al[2]; v.w *= al[3]; }
+            if (ep.beta != 0.f) {
+              v.x += ep.beta * o[u].x; v.y += ep.beta * o[u].y; v.z += ep.beta * o[u].z; v.w += ep.beta * o[u].w;
+            }
+            if (ep.act) *sp = v;
+            else if (mb + rr < M) *reinterpret_cast<float4*>(cbase + (mb + rr) * ep.ldc + n) = v;
+          }
         }
-        *c4 = v;
-        continue;
       }
+      if (ep.act) {
 #pragma unroll 1
-      for (int q = 0; q < 4 && n + q < N; ++q) {
-        float o = slab[rr * W4_FP + c + q];
-        if (ep.alpha_group > 0) o *= col_alpha(ep, n + q);
-        if (ep.beta != 0.f) o += ep.beta * cp[q];
-        cp[q] = ep.act ? epi_act(ep.act, o) : o;
+        for (int it = 0; it < 16; ++it) {
+          const int rr = it * 2 + lane / 32;
+          const float4 v = *reinterpret_cast<const float4*>(slab + rr * W4_FP + c);
+          float r[4] = {v.x, v.y, v.z, v.w};
+          if (ep.act == ACT_SILU) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r[q] = epi_act(ACT_SILU, r[q]);
+          } else if (ep.act == ACT_RELU) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r[q] = epi_act(ACT_RELU, r[q]);
+          } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r[q] = epi_act(ACT_GELU, r[q]);
+          }
+          if (mb + rr < M)
+            *reinterpret_cast<float4*>(cbase + (mb + rr) * ep.ldc + n) = make_float4(r[0], r[1], r[2], r[3]);
+        }
+      }
+    } else if (n < N) {  // fewer than four columns left
+#pragma unroll 1
+      for (int it = 0; it < 16; ++it) {
+        const int rr = it * 2 + lane / 32;
+        if (mb + rr >= M) continue;
+        float* cp = cbase + (mb + rr) * ep.ldc + n;
+#pragma unroll 1
+        for (int q = 0; q < (int)(N - n); ++q) {
+          float o = slab[rr * W4_FP + c + q];
+          if (ep.alpha_group > 0) o *= col_alpha(ep, n + q);
+          if (ep.beta != 0.f) o += ep.beta * cp[q];
+          cp[q] = ep.act ? epi_act(ep.act, o) : o;
+        }
       }
     }
   }

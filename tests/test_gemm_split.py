@@ -146,3 +146,52 @@ def test_token_major_big_tiles(dtype, M, N, K, a_layout, split):
         L.check(fn(M, N, arr, 2, a_layout, ROW, c.data_ptr(), N, L.dtype_code(out_dtype), 0.5, 0.0, L.EPI_STORE, split,
                    L.stream_of(c)), "forge_gemm")
         _close(c[0] if split == 1 else c.sum(0), 0.5 * ref, mag, sum(ks))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("al,bl,N", [(ROW, COL, 518), (ROW, COL, 512), (ROW, ROW, 520), (COL, ROW, 520)])
+@pytest.mark.parametrize("K", [64, 264, 1032])
+def test_fp32_forms(al, bl, N, K):
+    """An fp32 C that is added to, activated and both, whole tiles and ragged
+    ones (N that is not a multiple of 4 included), short and long reductions."""
+    M = 264
+    gen = torch.Generator().manual_seed(K)
+    a = torch.randn(M, K, generator=gen).to(torch.bfloat16)
+    b = (torch.randn(K, N, generator=gen) * K ** -0.5).to(torch.bfloat16)
+    prod, mag = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    ad, bd = (a if al == ROW else a.t().contiguous()).cuda(), (b if bl == ROW else b.t().contiguous()).cuda()
+    seg = (L.GemmSegment * 1)(L.GemmSegment(ad.data_ptr(), ad.stride(0), bd.data_ptr(), bd.stride(0), K, 0, 0))
+    acts = ((L.EPI_STORE, lambda v: v), (L.EPI_SILU, torch.nn.functional.silu), (L.EPI_RELU, torch.relu),
+            (L.EPI_GELU, lambda v: torch.nn.functional.gelu(v, approximate="tanh")))
+    for epi, act in acts:
+        for alpha, beta in ((0.5, 0.0), (1.0, 2.0)):
+            c0 = torch.randn(M, 520, generator=gen)
+            c = c0.cuda()
+            L.check(L.forge_gemm(M, N, seg, 1, al, bl, c.data_ptr(), 520, L.DTYPE_F32, alpha, beta, epi, 1,
+                                 L.stream_of(c)), "forge_gemm")
+            ref = act(alpha * prod + beta * c0.double()[:, :N])
+            # (1.13: the activations' largest slope; 2e-6: their own fp32 evaluation)
+            bound = 1.13 * ((K + 2) * 2.0 ** -24 * (abs(alpha) * mag + abs(beta) * c0.abs()[:, :N])) + 2e-6 + \
+                2.0 ** -22 * ref.abs()
+            got = c.cpu()
+            assert ((got.double()[:, :N] - ref).abs() <= bound).all(), (epi, beta)
+            assert torch.equal(got[:, N:], c0[:, N:])  # past the last column
+
+
+@pytest.mark.gpu
+def test_fp32_partials_with_column_alphas():
+    """Stacked LoRA-A products wider than the narrow tiles, split over K: each
+    projection's scale is applied to its own columns."""
+    M, K, r, n = 300, 1024, 96, 4
+    gen = torch.Generator().manual_seed(3)
+    x = torch.randn(M, K, generator=gen).to(torch.bfloat16).cuda()
+    stack = torch.randn(n * r, K, generator=gen).to(torch.bfloat16).cuda()
+    scales = [0.5, 1.0, 2.0, -3.0]
+    out = torch.empty(M, n * r, dtype=torch.bfloat16, device="cuda")
+    work = torch.empty(4, M, n * r, device="cuda")
+    import ctypes
+    ptrs = (ctypes.c_void_p * n)(*[stack[p * r:].data_ptr() for p in range(n)])
+    L.check(L.forge_lora_a(M, K, r, n, x.data_ptr(), K, ptrs, K, (ctypes.c_float * n)(*scales), out.data_ptr(), n * r,
+                           work.data_ptr(), 4, L.stream_of(x)), "forge_lora_a")
+    s = torch.tensor(scales, device="cuda", dtype=torch.float64).repeat_interleave(r)
+    _close(out, x.double() @ stack.double().t() * s, x.double().abs() @ stack.double().abs().t() * s.abs(), K)
