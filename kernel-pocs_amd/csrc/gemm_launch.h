@@ -98,7 +98,9 @@ static int64_t total_k(const GemmArgs& a) {
 // reads of C, where the reduction is short or an activation follows.  Measured
 // on MI355X, 8 against 4 waves: [8192, 4096] K = 64 71 / 76 us, with GELU 71 /
 // 90, [512, 4096] K = 64 19 / 23, [1024, 1024] K = 1024 39 / 45, [4096, 4096] K
-// = 4096 152 / 131.
+// = 4096 152 / 131.  So does a short A^T B in 16 bits of more than one round of
+// tiles: [8192, 4096] K = 64 27 / 31, K = 256 35 / 42; [4096, 4096] K = 512 28 /
+// 28, [2048, 4096] K = 16 14.2 / 13.5.
 template <class T, int BMODE, int EPI, bool AT, bool BT>
 static bool launch_w4_staged(const GemmArgs& a, dim3 grid, hipStream_t s) {
   if constexpr (w4_staged_epi(EPI)) {
@@ -110,7 +112,7 @@ static bool launch_w4_staged(const GemmArgs& a, dim3 grid, hipStream_t s) {
         return true;
       }
     }
-    if (EPI == EPI_STORE_BF16 && !plain_store(a)) return false;
+    if (EPI == EPI_STORE_BF16 && (!plain_store(a) || (AT && total_k(a) <= 256 && grid.x > 256))) return false;
     gemm_w4_kernel<T, BMODE, EPI, true, AT, BT><<<grid, 256, 0, s>>>(a);
     return true;
   }

@@ -195,3 +195,20 @@ def test_fp32_partials_with_column_alphas():
                            work.data_ptr(), 4, L.stream_of(x)), "forge_lora_a")
     s = torch.tensor(scales, device="cuda", dtype=torch.float64).repeat_interleave(r)
     _close(out, x.double() @ stack.double().t() * s, x.double().abs() @ stack.double().abs().t() * s.abs(), K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [256, 264])
+def test_token_major_to_16_bits(K):
+    """Either side of the reduction length that changes the engine of A^T B
+    (289 tiles)."""
+    M, N = 4104, 4112
+    g = torch.Generator().manual_seed(K)
+    for dtype in (torch.bfloat16, torch.float16):
+        a, b = torch.randn(K, M, generator=g).to(dtype).cuda(), torch.randn(K, N, generator=g).to(dtype).cuda()
+        c = torch.empty(M, N, dtype=dtype, device="cuda")
+        seg = (L.GemmSegment * 1)(L.GemmSegment(a.data_ptr(), M, b.data_ptr(), N, K, 0, 0))
+        fn = L.forge_gemm if dtype == torch.bfloat16 else L.forge_gemm_f16
+        L.check(fn(M, N, seg, 1, COL, ROW, c.data_ptr(), N, L.dtype_code(dtype), 0.5, 0.0, L.EPI_STORE, 1,
+                   L.stream_of(c)), "forge_gemm")
+        _close(c, 0.5 * (a.double().t() @ b.double()), 0.5 * (a.double().abs().t() @ b.double().abs()), K)
