@@ -30,14 +30,38 @@ int launch_glu_bwd(int epi, int al, int bl, const GemmArgs& a, hipStream_t s);
 int launch_rope(const GemmArgs& a, hipStream_t s);
 int launch_rows(int epi, const GemmArgs& a, hipStream_t s);  // few rows, K-contiguous operands
 
+inline int64_t total_k(const GemmArgs& a) {
+  int64_t k = 0;
+  for (int i = 0; i < a.n_segs; ++i) k += a.segs[i].k;
+  return k;
+}
+
 // Few rows against K-contiguous weights: the row engine (gemm_rows.hip).  Up
-// to 32 rows of a plain product (43 us at 32 rows, K = 14336, N = 4096; 256 x
+// to 64 rows of a gate/up product (80 us; 256 x 256 tiles 94, the row engine
+// 172 at 128) and 32 of a plain one (43 us at 32 rows, K = 14336, N = 4096; 256 x
 // 256 tiles split over K take 45 at any row count up to 128, the row engine 77
-// at 64) and 64 of a gate/up product (80 us; 256 x 256 tiles 94, the row
-// engine 172 at 128).
+// at 64).  Columns a workgroup of a plain product, 0: 32 x 256 tiles.
+// Every workgroup reads all of A from L2, which passes the weights' own time
+// where there are many rows and columns; 64 columns a workgroup read it a
+// quarter as often but leave fewer of them, and 32 x 256 tiles are faster once
+// they fill the chip.  Measured on MI355X, us with 32 x 256 tiles / 16 / 64
+// columns, K = 4096: [16, 28672] 81 / 67 / 54, [32, 28672] 84 / 81 / 62, [32,
+// 32000] 86 / 92, [1, 40960] 86 / 63 / 73, [17, 40960] 89 / 94, [16, 50264] 97 /
+// 113 / 99, [8, 65536] 128 / 116 / 108, [1, 128256] 208 / 179 / 190, [8, 128256]
+// 212 / 219 / 194, [16, 128256] 219 / 263 / 199, [32, 128256] 229 / 350 / 244;
+// K = 8192: [8, 128256] 364 / 402 / 401; K = 64: [16, 65536] 9 / 16 / 10; K =
+// 512: [1, 65536] 18 / 23 / 16, K = 1024: [8, 65536] 30 / 39 / 29.
+inline int rows_columns(const GemmArgs& a) {
+  const int64_t mn = a.M * a.N, k = total_k(a);
+  if (a.N <= 128 * 256) return mn <= 896 * 1024 ? 16 : 0;  // 32 x 256 tiles on half the CUs or fewer
+  if (a.M > 16 || k <= 128) return 0;
+  if (mn <= 512 * 1024 && k >= 2048) return 16;
+  return k <= 4096 ? 64 : 0;
+}
+
 inline bool rows_engine(int epi, const GemmArgs& a) {
   if (a.split_k != 1 || a.N <= a.M) return false;
-  if (epi == EPI_STORE_BF16) return a.M <= 32;
+  if (epi == EPI_STORE_BF16) return a.M <= 32 && rows_columns(a) > 0;
   return glu_fwd_epi(epi) && a.M <= 64 && !a.ep.vpart && !a.f16;
 }
 int launch_f16(int epi, int cfg, int al, int bl, const GemmArgs& a, hipStream_t s);  // fp16 operands
@@ -85,12 +109,6 @@ static void order_columns(GemmArgs& a, int64_t out_bn, int64_t tn) {
 }
 
 static bool plain_store(const GemmArgs& a) { return a.ep.beta == 0.f && a.ep.act == ACT_NONE && a.ep.alpha_group == 0; }
-
-static int64_t total_k(const GemmArgs& a) {
-  int64_t k = 0;
-  for (int i = 0; i < a.n_segs; ++i) k += a.segs[i].k;
-  return k;
-}
 
 // Launches the 4-wave engine with its epilogue through LDS, or returns false:
 // it needs 16-byte vectors, and of the 16-bit stores takes the plain one.  A^T B

@@ -2,7 +2,7 @@
 // [N][K]): the products of a decode step, where every weight is read once for
 // a few rows and the weights' bytes set the time.
 //
-// A workgroup owns 16 output columns (dual B: up to 32 gate and 32 up) and
+// A workgroup owns 16 or 64 output columns (dual B: up to 32 gate and 32 up) and
 // all rows; its waves split K in chunks of U 32-deep k-steps, dealt out in
 // turn so that the workgroup streams each weight row front to back.  Weights
 // go from memory straight to the registers that v_mfma_f32_16x16x32 reads (no
@@ -154,10 +154,12 @@ static int launch_one(const GemmArgs& a, hipStream_t s) {
 }
 
 // Single B: 16 columns a workgroup (32 leave CUs without one at N = 4096: 32
-// -> 43 us at 16 rows); 4, 8 and 16 waves measured equal there, and more
-// shorten the K loop where there are few workgroups.
+// -> 43 us at 16 rows), or 64 (rows_columns); 4, 8 and 16 waves measured equal
+// there, and more shorten the K loop where there are few workgroups.
 template <class T, int MB>
 static int launch_single(const GemmArgs& a, hipStream_t s) {
+  if constexpr (MB == 1)
+    if (rows_columns(a) == 64) return launch_one<T, MB, 4, 4, EPI_STORE_BF16>(a, s);
   if (a.N < 16 * 64) return launch_one<T, MB, 1, 16, EPI_STORE_BF16>(a, s);
   return launch_one<T, MB, 1, 8, EPI_STORE_BF16>(a, s);
 }

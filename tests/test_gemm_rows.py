@@ -139,3 +139,25 @@ def test_unsplit_33_to_64_rows(M, N, K, c_dtype, epi):
         # (1.1: the activation's slope; 1e-6: its own fp32 evaluation)
         bound = ulp * ref.abs() * 1.01 + 1.1 * (K + 2) * 2.0 ** -24 * (mag + c0.abs()) + 1e-6
         assert ((c.double()[:, :N] - ref).abs() <= bound).all(), (beta, pad)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(28, 32768, 72), (29, 32768, 72), (16, 32768, 520), (15, 32776, 2048), (16, 32784, 2048),
+                                   (1, 32776, 2040), (1, 32776, 128), (16, 40968, 4096), (16, 40968, 4104), (17, 32776, 520)])
+def test_many_columns(M, N, K):
+    """Either side of each line of the rule that picks 16 or 64 columns a
+    workgroup or 32-row tiles; a second segment, a C that is added to."""
+    gen = torch.Generator().manual_seed(K)
+    for dtype in (torch.bfloat16, torch.float16):
+        a, t = _mat(M, K - 8, gen, dtype), _mat(M, 8, gen, dtype)
+        b = (torch.randn(N, K - 8, device="cuda") * K ** -0.5).to(dtype)
+        z = torch.randn(N, 8, device="cuda").to(dtype)
+        c = torch.randn(M, N, device="cuda").to(dtype)
+        ref = a.double() @ b.double().t() + t.double() @ z.double().t() + c.double()
+        mag = a.double().abs() @ b.double().abs().t() + t.double().abs() @ z.double().abs().t() + c.double().abs()
+        segs = (L.GemmSegment * 2)(L.GemmSegment(a.data_ptr(), K - 8, b.data_ptr(), K - 8, K - 8, 0, 0),
+                                   L.GemmSegment(t.data_ptr(), 8, z.data_ptr(), 8, 8, 0, 0))
+        fn = L.forge_gemm_f16 if dtype == torch.float16 else L.forge_gemm
+        L.check(fn(M, N, segs, 2, ROW, COL, c.data_ptr(), N, L.dtype_code(dtype), 1.0, 1.0, L.EPI_STORE, 1,
+                   L.stream_of(c)), "forge_gemm")
+        assert ((c.double() - ref).abs() <= U[dtype] * ref.abs() * 1.01 + (K + 2) * 2.0 ** -24 * mag + 1e-6).all()
