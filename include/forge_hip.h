@@ -282,7 +282,8 @@ int64_t forge_rmsnorm_bwd_workspace(int dtype, int64_t rows, int64_t cols);
  * Any shape and stride.  fp16 / bf16 products without a bias whose operands
  * are 16-byte aligned, have a unit stride along one dimension with an extent
  * that is a multiple of 8, and a pitch that is a multiple of 8 run on the MFMA
- * core; the others do one fp32 fmaf per k in increasing k order.
+ * core, unless they are small (K up to 128 and at most 256 tiles of 64 x 64);
+ * the others do one fp32 fmaf per k in increasing k order.
  * Replaces the cuBLAS products of the fused linear + cross-entropy path
  * (kernels/cross_entropy/experiments/v2/fused_linear_cross_entropy.py:142-144,
  * 207-219: logits = X W^T + b, dX = dlogits W, dW += dlogits^T X,

@@ -4,8 +4,8 @@
 // operands, fp32 accumulation with one fmaf per k in increasing k order
 // (deterministic, and exact to fp32 rounding).  It is the path for what the
 // MFMA core does not take: fp32 models, and 16-bit operands whose extents or
-// row pitches are not multiples of 8.  16-bit products that the core does
-// take (mfma_segment below) run there: same products, fp32 accumulation, one
+// row pitches are not multiples of 8, and for short ones.  16-bit products that
+// the core does take (mfma_segment below) run there: same products, fp32 accumulation, one
 // rounding, another summation order.
 //
 // Why: this kernel does one fmaf per multiply (no matrix instruction) and is
@@ -125,6 +125,23 @@ int launch_generic(const GenArgs& g, int c_dtype, hipStream_t s) {
   return FORGE_OK;
 }
 
+// Short reductions into outputs that this kernel covers in one round of 64 x 64
+// tiles take less here than one of the core's tiles takes to start: measured on
+// MI355X, core / here: [8, 8] K = 8 10.3 / 4.5 us, [1024, 1024] K = 32 11.9 /
+// 7.2, K = 64 11.9 / 10.0, K = 128 14 / 16; A as [K][M] and B as [N][K] (staged
+// through registers there) K = 128 23.6 / 16.9; [256, 8] K = 32, A as [K][M]
+// 8.9 / 6.5.  The core's narrow tiles and its row engine start sooner: [8, 64]
+// K = 16 5.6 / 4.8, K = 32 5.4 / 6.1, [1024, 16] K = 64 6.5 / 9.0, [16, 64] K =
+// 8, B as [N][K] 3.8 / 4.7.
+bool short_product(const GenArgs& g, int al, int bl) {
+  if (((g.M + GBM - 1) / GBM) * ((g.N + GBN - 1) / GBN) > 256) return false;
+  if (al == 0 && bl == 1 && g.M <= 32 && g.N > g.M) return false;
+  if (g.K <= 16) return true;
+  const bool narrow = g.M != g.N && (g.M <= 64 || g.N <= 64 || (al == 0 && g.N <= 128));
+  if (narrow) return g.K <= 32 && ((al == 1 && g.M > g.N) || (g.M > 64 && g.N > 64));
+  return g.K <= (al == 1 && bl == 1 ? 128 : 64);
+}
+
 // The product as one segment of the MFMA core (fp16 or bf16 operands), or
 // false.  The core fetches 16-byte chunks along each operand's unit-stride
 // dimension, so that dimension's extent and the other's stride must be
@@ -142,6 +159,7 @@ bool mfma_segment(const GenArgs& g, forge_gemm_segment& seg, int& al, int& bl) {
   if (seg.lda % 8 || seg.ldb % 8 || seg.lda < 0 || seg.ldb < 0 || seg.lda > kMaxPitch || seg.ldb > kMaxPitch) return false;
   if ((al == 0 || bl == 1) && g.K % 8) return false;
   if ((al == 1 && g.M % 8) || (bl == 0 && g.N % 8)) return false;
+  if (short_product(g, al, bl)) return false;
   seg.a = g.a;
   seg.b = g.b;
   seg.k = g.K;

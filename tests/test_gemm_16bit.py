@@ -108,3 +108,14 @@ def test_fp16_range():
                                      c.data_ptr(), 64, L.DTYPE_F16, 1.0, 0.0, None, L.GEMM_ACT_NONE,
                                      L.stream_of(c)), "forge_gemm_generic")
         assert (c.float() == want).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(8, 8), (64, 64), (1024, 1024), (1032, 1024), (72, 264), (16, 264), (264, 16), (264, 128)])
+@pytest.mark.parametrize("K", [8, 16, 24, 32, 40, 64, 72, 128, 136])
+def test_short_reductions(M, N, K):
+    """Either side of the lines between the general kernel and the core."""
+    gen = torch.Generator().manual_seed(K)
+    for fa, fb in (("row", "row"), ("row", "col"), ("col", "col")):
+        a, b = _operand(M, K, fa, torch.float16, gen), _operand(K, N, fb, torch.float16, gen)
+        _check(a, b, torch.float16, alpha=0.5, beta=1.0)
