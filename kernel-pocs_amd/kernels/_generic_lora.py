@@ -26,7 +26,7 @@ from typing import Optional
 import torch
 
 from forge_hip import _lib as L
-from kernels._lora_ops import COL, ROW, skinny_split, split_for, split_gemm, split_k_for
+from kernels._lora_ops import COL, ROW, array_type, skinny_split, split_for, split_k_for, split_product
 
 GENERIC_DTYPES = (torch.float32, torch.float16)
 
@@ -43,12 +43,17 @@ _MAX_PITCH = (1 << 31) // 512 - 1
 
 
 def _mfma_layouts(a: torch.Tensor, b: torch.Tensor):
-    """(a_layout, lda, b_layout, ldb) of a @ b for the MFMA core, or None:
+    """(a_layout, b_layout, K segment) of a @ b for the MFMA core, or None:
     fp16 operands that it reads in 16-byte chunks along their unit-stride
-    dimension (the rule of forge_gemm_generic, csrc/gemm_generic.hip)."""
+    dimension (the rule of forge_gemm_generic, csrc/gemm_generic.hip; its line
+    for small products is the library's to draw).  (One query of each
+    property: a small layer's step is the host's time, 2 us a look.)"""
+    if a.dtype != torch.float16:
+        return None
     M, K = a.shape
     N = b.shape[1]
-    if a.dtype != torch.float16 or K == 0 or a.data_ptr() % 16 or b.data_ptr() % 16:
+    pa, pb = a.data_ptr(), b.data_ptr()
+    if K == 0 or (pa | pb) & 15:
         return None
     (am, ak), (bk, bn) = a.stride(), b.stride()
     if ak == 1:
@@ -63,11 +68,11 @@ def _mfma_layouts(a: torch.Tensor, b: torch.Tensor):
         bl, ldb = ROW, bk
     else:
         return None
-    if lda % 8 or ldb % 8 or lda > _MAX_PITCH or ldb > _MAX_PITCH:
+    if (lda | ldb) & 7 or lda > _MAX_PITCH or ldb > _MAX_PITCH:
         return None
     if (al == ROW or bl == COL) and K % 8 or al == COL and M % 8 or bl == ROW and N % 8:
         return None
-    return al, lda, bl, ldb
+    return al, bl, (pa, lda, pb, ldb, K, 0, 0)
 
 
 def _split(M: int, N: int, K: int, al: int, bl: int) -> int:
@@ -92,21 +97,30 @@ def _one_product(terms, out: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """sum of a @ b over terms as one fp16 product of as many K segments, or
     None where the MFMA core does not take them all in the same layouts, or an
     `out` that is not fp16 with unit stride along its rows (left to gmm)."""
+    if len(terms) > _MAX_SEGS:
+        return None
     M, N = terms[0][0].shape[0], terms[0][1].shape[1]
     if out is not None and (out.dtype != torch.float16 or out.stride(1) != 1 and N != 1):
         return None
-    lay = [_mfma_layouts(a, b) for a, b in terms]
-    if M == 0 or N == 0 or len(terms) > _MAX_SEGS or any(v is None or v[0::2] != lay[0][0::2] for v in lay):
+    segs, first = [], None
+    for i, (a, b) in enumerate(terms):
+        if i and a is terms[i - 1][0] and b is terms[i - 1][1]:  # the second of a term with scale 2
+            segs.append(segs[-1])
+            continue
+        lay = _mfma_layouts(a, b)
+        if lay is None or first is not None and lay[:2] != first:
+            return None
+        first = lay[:2]
+        segs.append(lay[2])
+    if M == 0 or N == 0:
         return None
-    al, bl = lay[0][0::2]
-    segs = [(a, v[1], b, v[3], a.shape[1]) for (a, b), v in zip(terms, lay)]
+    al, bl = first
     if out is None:
         out = torch.empty(M, N, dtype=torch.float16, device=terms[0][0].device)
-    split = _split(M, N, sum(-(-a.shape[1] // 64) * 64 for a, _ in terms), al, bl)
+    split = _split(M, N, sum(-(-sg[4] // 64) * 64 for sg in segs), al, bl)
+    arr = array_type(L.GemmSegment, len(segs))(*segs)
     if split > 1:
-        return split_gemm(M, N, segs, al, bl, split, out)
-    arr = (L.GemmSegment * len(segs))(*(L.GemmSegment(a.data_ptr(), lda, b.data_ptr(), ldb, k, 0, 0)
-                                        for a, lda, b, ldb, k in segs))
+        return split_product(M, N, arr, True, al, bl, split, out)
     L.check(L.forge_gemm_f16(M, N, arr, len(segs), al, bl, out.data_ptr(), out.stride(0), L.DTYPE_F16, 1.0, 0.0,
                              L.EPI_STORE, 1, L.stream_of(out)), "forge_gemm_f16")
     return out
@@ -121,12 +135,23 @@ def gmm_sum(pairs, lora=(), out: Optional[torch.Tensor] = None) -> torch.Tensor:
     twice: the sum is exact in the fp32 accumulators, and no operand is scaled
     in fp16 (where it could overflow or lose bits).  The 64-deep K tile that a
     segment costs is 1 us, the read-modify-write product that it replaces 33 us
-    at [2048, 8192] (MI355X).  Other scales keep that product and its alpha."""
-    if lora and all(s in (1, 2) for _, _, s in lora):
-        joined = _one_product([*pairs, *((a, b) for a, b, s in lora for _ in range(int(s)))], out)
-        if joined is not None:
-            return joined
-    total = _one_product(pairs, out)
+    at [2048, 8192] (MI355X).  Other scales keep that product and its alpha, and
+    so do terms past six segments (LoRA-QKV's dX, three base products and three
+    terms, joins at scale 1 only): a LoRA-MLP step of 2048 tokens, 2048 -> 8192,
+    takes 679 us at scale 1, 692 at 2 and 827 at 0.5 or 3."""
+    total = None
+    if pairs[0][0].dtype == torch.float16:
+        terms = list(pairs)
+        for a, b, s in lora:
+            if s != 1 and s != 2:
+                break
+            terms += [(a, b)] * int(s)
+        else:
+            total = _one_product(terms, out)
+            if total is not None:
+                return total
+        if lora:
+            total = _one_product(pairs, out)
     if total is None:
         total = out
         for i, (a, b) in enumerate(pairs):
@@ -153,11 +178,13 @@ def gmm(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None, al
             out.mul_(beta)
         return out
     assert out.stride(1) == 1 or N == 1
-    if beta == 0.0 and out.dtype == a.dtype:
+    # (no product is split into fewer than 4 K tiles a split; the host's time
+    # for this look is what a small layer's step takes)
+    if K > 7 * 64 and beta == 0.0 and a.dtype == torch.float16 and out.dtype == torch.float16:
         lay = _mfma_layouts(a, b)
-        split = _split(M, N, K, lay[0], lay[2]) if lay is not None else 1
+        split = _split(M, N, K, lay[0], lay[1]) if lay is not None else 1
         if split > 1:
-            return split_gemm(M, N, [(a, lay[1], b, lay[3], K)], lay[0], lay[2], split, out, alpha)
+            return split_product(M, N, array_type(L.GemmSegment, 1)(lay[2]), True, lay[0], lay[1], split, out, alpha)
     L.check(L.forge_gemm_generic(M, N, K, L.dtype_code(a.dtype), a.data_ptr(), a.stride(0), a.stride(1),
                                  b.data_ptr(), b.stride(0), b.stride(1), out.data_ptr(), out.stride(0),
                                  L.dtype_code(out.dtype), float(alpha), float(beta), None, L.GEMM_ACT_NONE,

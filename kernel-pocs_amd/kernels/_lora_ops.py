@@ -49,7 +49,7 @@ def ld(t: torch.Tensor) -> int:
 # (ctypes makes an array type per length on a slower path than this lookup: a
 # LoRA training step on few tokens is bound by the host, 300 us of it here)
 @functools.lru_cache(maxsize=64)
-def _array(ctype, n: int):
+def array_type(ctype, n: int):
     return ctype * n
 
 
@@ -107,7 +107,7 @@ def split_for(M: int, N: int, k_tiles: int) -> int:
 def _segments(segs) -> ctypes.Array:
     """forge_gemm_segment array from (A, lda, B, ldb, K) tuples, optionally
     extended by (n_lo, n_hi): the output columns the segment applies to."""
-    return _array(L.GemmSegment, len(segs))(
+    return array_type(L.GemmSegment, len(segs))(
         *[(sg[0].data_ptr(), sg[1], sg[2].data_ptr(), sg[3], sg[4], *(sg[5:7] if len(sg) > 5 else (0, 0))) for sg in segs])
 
 
@@ -132,7 +132,7 @@ def gemm(M: int, N: int, segs: Sequence[Tuple[torch.Tensor, int, torch.Tensor, i
         if split > 1:
             if out is None:
                 out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
-            return split_gemm(M, N, segs, a_layout, b_layout, split, out, alpha, dev)
+            return split_gemm(M, N, segs, a_layout, b_layout, split, out, alpha)
     if out is None:
         if atomic:
             out = torch.empty(M, N, dtype=torch.float32, device=dev)
@@ -150,18 +150,23 @@ def gemm(M: int, N: int, segs: Sequence[Tuple[torch.Tensor, int, torch.Tensor, i
 
 
 def split_gemm(M: int, N: int, segs, a_layout: int, b_layout: int, split: int, out: torch.Tensor,
-               alpha: float = 1.0, device=None) -> torch.Tensor:
-    """out = alpha * sum_s A_s @ B_s with K split `split` ways: each split
-    writes fp32 partials to its slice of a [split, M, N] workspace and
-    forge_splitk_reduce sums them in a fixed order (deterministic) and rounds
-    once to out's dtype.  The operands are bf16 or fp16."""
-    dev = device if device is not None else out.device
-    parts = torch.empty(split, M, N, dtype=torch.float32, device=dev)
-    arr = _segments(segs)
+               alpha: float = 1.0) -> torch.Tensor:
+    """out = alpha * sum_s A_s @ B_s with K split `split` ways (split_product);
+    segs as gemm's, bf16 or fp16 operands."""
+    return split_product(M, N, _segments(segs), segs[0][0].dtype == torch.float16, a_layout, b_layout, split, out, alpha)
+
+
+def split_product(M: int, N: int, arr: ctypes.Array, f16: bool, a_layout: int, b_layout: int, split: int,
+                  out: torch.Tensor, alpha: float = 1.0) -> torch.Tensor:
+    """The product of a forge_gemm_segment array with K split `split` ways:
+    each split writes fp32 partials to its slice of a [split, M, N] workspace
+    and forge_splitk_reduce sums them in a fixed order (deterministic) and
+    rounds once to out's dtype."""
+    parts = torch.empty(split, M, N, dtype=torch.float32, device=out.device)
     st = L.stream_of(parts)
-    fn = L.forge_gemm_f16 if segs[0][0].dtype == torch.float16 else L.forge_gemm
-    L.check(fn(M, N, arr, len(segs), a_layout, b_layout, parts.data_ptr(), N, L.DTYPE_F32, float(alpha),
-               0.0, L.EPI_STORE, int(split), st), "forge_gemm")
+    L.check((L.forge_gemm_f16 if f16 else L.forge_gemm)(M, N, arr, len(arr), a_layout, b_layout, parts.data_ptr(), N,
+                                                        L.DTYPE_F32, float(alpha), 0.0, L.EPI_STORE, int(split), st),
+            "forge_gemm")
     L.check(L.forge_splitk_reduce(parts.data_ptr(), M * N, int(split), M, N, N, out.data_ptr(), ld(out),
                                   L.dtype_code(out.dtype), 1.0, st), "forge_splitk_reduce")
     return out
@@ -203,8 +208,8 @@ def lora_a(x: torch.Tensor, mats: Sequence[torch.Tensor], scales: Sequence[float
         addrs = [a.data_ptr() for a in mats]
     if out is None:
         out = torch.empty(M, n * r, dtype=torch.bfloat16, device=x.device)
-    ptrs = _array(ctypes.c_void_p, n)(*addrs)
-    sc = _array(ctypes.c_float, n)(*[float(s) for s in scales])
+    ptrs = array_type(ctypes.c_void_p, n)(*addrs)
+    sc = array_type(ctypes.c_float, n)(*[float(s) for s in scales])
     split = skinny_split(M, n * r, K) if M > n * r else 1
     work = torch.empty(split, M, n * r, dtype=torch.float32, device=x.device) if split > 1 else None
     L.check(
@@ -310,7 +315,7 @@ def small_t_batch(mats: Sequence[torch.Tensor]) -> list:
     buf = torch.empty(o, dtype=mats[0].dtype, device=mats[0].device)
     outs = [buf.as_strided((c, r), (r, 1), off) for r, c, off in zip(rows, cols, offs)]
     k = len(mats)
-    ptrs, ints = _array(ctypes.c_void_p, k), _array(ctypes.c_int64, k)
+    ptrs, ints = array_type(ctypes.c_void_p, k), array_type(ctypes.c_int64, k)
     base, size = buf.data_ptr(), buf.element_size()
     src = ptrs(*[m.data_ptr() for m in mats])
     dst = ptrs(*[base + off * size for off in offs])
