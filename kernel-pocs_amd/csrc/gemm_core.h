@@ -10,8 +10,9 @@
 // (BM/WAVES_M) x (BN/WAVES_N) sub-tile.  256 x 256 tiles run on the 4-wave
 // engine (gemm_w4.h, v_mfma_f32_16x16x32) and a few rows on the row engine
 // (gemm_rows.hip); here are the others, on v_mfma_f32_32x32x16:
-//   * gemm_dma_kernel (narrow and skinny tiles; 256 x 256 tiles whose C is read
-//     or whose stores cannot be vectors): global -> LDS by LDS-DMA
+//   * gemm_dma_kernel (narrow and skinny tiles; 256 x 256 tiles added to a
+//     16-bit C, and of token-major operands short or activated ones and those
+//     whose stores cannot be vectors): global -> LDS by LDS-DMA
 //     (buffer_load ... lds, no VGPR staging, no ds_write), XOR-swizzled
 //     unpadded LDS rows, a 2- or 3-stage ring.  At 256 x 256 it runs 8 waves
 //     (4 x 2, 64 x 128 per wave) so that each SIMD holds two waves whose MFMA
@@ -71,9 +72,8 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
 }
 
 // Output-row mapping of B-tile rows in "dual" mode: the tile's B rows come
-// alternately (in groups of 32) from two weights, so that a wave's N tiles
-// t = 0,1,2,3 are (gate cols c..c+31, up cols c..c+31, gate c+32.., up c+32..)
-// and the matching gate/up accumulators sit in the same lane and register.
+// alternately (in groups of 32) from two weights, so that the matching gate/up
+// accumulators sit in the same lane and register (the 4-wave engine, gemm_w4.h).
 enum BMode { B_SINGLE = 0, B_DUAL = 1 };
 
 struct Seg {
@@ -217,8 +217,6 @@ __device__ __forceinline__ void transpose8x8(const uint4 (&in)[8], uint4 (&out)[
 // offset past the buffer's num_records, which the hardware returns as zeros,
 // so the K loop has no branches.  Per K tile, load() rebases the buffer
 // resource on k0 (scalar work) and masks k beyond the segment's end.
-// DUAL (B only): vector i of a thread lies in 32-row group i % 4 of a 128-row
-// wave slab; even groups read pointer 0 (gate), odd groups pointer 1 (up).
 constexpr uint32_t OOB = 0x80000000u;       // offset >= num_records -> reads 0
 constexpr int NUM_RECORDS = 0x7fffffff;
 
@@ -240,32 +238,29 @@ __device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t o
   return make_uint4((uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w);
 }
 
-template <int BROWS, int NT, bool KCONTIG, bool DUAL>
+template <int BROWS, int NT, bool KCONTIG>
 struct TileLoader {
   static constexpr int NVEC = BROWS * BK / 8;                  // 16-byte vectors per tile
   static constexpr int NBLK = (BROWS / 8) * (BK / 8);          // 8x8 blocks per tile
   static constexpr int VPT = KCONTIG ? (NVEC + NT - 1) / NT : 8 * ((NBLK + NT - 1) / NT);
   static constexpr int BPT = VPT / 8;                          // 8x8 blocks per thread (!KCONTIG)
-  static_assert(!DUAL || (KCONTIG && NT == 256 && BROWS == 256), "dual loader: 256x64 K-contiguous tile");
 
   struct Stage {  // one K tile in flight (registers)
     uint4 v[VPT];
   };
   uint32_t voff[KCONTIG ? VPT : BPT];  // byte offsets of the rows (OOB = zero-fill)
-  const char* base[2];
+  const char* base;
   int64_t ld_bytes;
 
-  // Panel p0/p1 + panel_off rows (KCONTIG) or columns (!KCONTIG);
-  // row_src(q, sel) -> index of tile row q relative to that panel start
+  // Panel p + panel_off rows (KCONTIG) or columns (!KCONTIG);
+  // row_src(q) -> index of tile row q relative to that panel start
   // (-1 = no data: zero-fill).  Relative offsets keep every byte offset
   // inside one tile panel, far below 2^31.
   template <class RowSrc>
-  __device__ __forceinline__ void setup(const void* p0, const void* p1, int64_t ld, int64_t panel_off,
-                                        RowSrc row_src) {
+  __device__ __forceinline__ void setup(const void* p, int64_t ld, int64_t panel_off, RowSrc row_src) {
     ld_bytes = ld * 2;
     const int64_t pan = KCONTIG ? panel_off * ld_bytes : panel_off * 2;
-    base[0] = p0 ? (const char*)p0 + pan : nullptr;
-    base[1] = DUAL ? (p1 ? (const char*)p1 + pan : nullptr) : base[0];
+    base = p ? (const char*)p + pan : nullptr;
     const int tid = threadIdx.x;
     if constexpr (KCONTIG) {
 #pragma unroll
@@ -273,8 +268,7 @@ struct TileLoader {
         const int v = tid + i * NT;
         const int q = v / (BK / 8);
         const int kc = (v % (BK / 8)) * 8;
-        const int sel = DUAL ? (i % 2) : 0;
-        const int64_t row = (v < NVEC && base[sel]) ? row_src(q, sel) : -1;
+        const int64_t row = (v < NVEC && base) ? row_src(q) : -1;
         voff[i] = row < 0 ? OOB : (uint32_t)(row * ld_bytes + kc * 2);
       }
     } else {
@@ -283,7 +277,7 @@ struct TileLoader {
         const int blk = tid + bi * NT;
         const int kb = (blk % (BK / 8)) * 8;   // k-block fastest: the 8 lanes of a row
         const int qb = (blk / (BK / 8)) * 8;   // group write one 128-byte LDS row span
-        const int64_t col = (blk < NBLK && base[0]) ? row_src(qb, 0) : -1;  // first of 8 contiguous rows
+        const int64_t col = (blk < NBLK && base) ? row_src(qb) : -1;  // first of 8 contiguous rows
         voff[bi] = col < 0 ? OOB : (uint32_t)(kb * ld_bytes + col * 2);
       }
     }
@@ -293,17 +287,16 @@ struct TileLoader {
     uint4* regs = st.v;
     const int tid = threadIdx.x;
     if constexpr (KCONTIG) {
-      const __amdgpu_buffer_rsrc_t r0 = make_rsrc(base[0] + k0 * 2);
-      const __amdgpu_buffer_rsrc_t r1 = make_rsrc(base[1] + k0 * 2);
+      const __amdgpu_buffer_rsrc_t r0 = make_rsrc(base + k0 * 2);
       const int kc = (tid % (BK / 8)) * 8;  // same for every i (NT is a multiple of 8)
       const bool kin = kc < kvalid;
 #pragma unroll
       for (int i = 0; i < VPT; ++i) {
         const uint32_t off = kin ? voff[i] : OOB;
-        regs[i] = buf_load16((DUAL && (i % 2)) ? r1 : r0, off);
+        regs[i] = buf_load16(r0, off);
       }
     } else {
-      const __amdgpu_buffer_rsrc_t r0 = make_rsrc(base[0] + k0 * ld_bytes);
+      const __amdgpu_buffer_rsrc_t r0 = make_rsrc(base + k0 * ld_bytes);
 #pragma unroll
       for (int bi = 0; bi < BPT; ++bi) {
         const int blk = tid + bi * NT;
@@ -447,7 +440,7 @@ constexpr int SG_DS_READ = 0x100;
 // ---------------------------------------------------------------------------
 // Staged epilogue (256 x 256 tiles, bf16 outputs): the accumulators go through
 // LDS, half a tile (128 rows) at a time in fp32, so that every thread then
-// owns contiguous 8-column chunks: side inputs (C for beta, e / g, cos / sin)
+// owns contiguous 8-column chunks: side inputs (C for beta, e / g)
 // are read and every output is written with 16-byte vector accesses instead
 // of one 2-byte access per lane and element.  Values are rounded exactly as
 // in the per-element epilogue (single rounding of the fp32 result).
@@ -493,8 +486,7 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
 // Tiles and epilogues the staged epilogue serves.
 constexpr bool staged_ok(int bm, int bn, int wm, int wn, int epi) {
   return bm == 256 && bn == 256 && (256 / wm) % 32 == 0 && (256 / wn) % 32 == 0 && 256 / wm <= 128 &&
-         (epi == EPI_STORE_BF16 || epi == EPI_STORE_F32 || glu_fwd_epi(epi) || glu_bwd_epi(epi) ||
-          epi == EPI_ROPE);
+         (epi == EPI_STORE_BF16 || epi == EPI_STORE_F32 || glu_bwd_epi(epi));
 }
 
 // Workgroup barrier that waits only for this wave's LDS accesses (lgkmcnt 0),
@@ -509,7 +501,7 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-template <class T, int WAVES_M, int WAVES_N, int BMODE, int EPI>
+template <class T, int WAVES_M, int WAVES_N, int EPI>
 __device__ __forceinline__ void epilogue_staged(const GemmArgs& args,
                                                 f32x16 (&acc)[256 / WAVES_M / 32][256 / WAVES_N / 32], int64_t m0,
                                                 int64_t n0, int lane, int wm, int wn, float* lds) {
@@ -537,39 +529,8 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs& args,
     }
     lds_barrier();
     const int64_t mrow0 = m0 + pass * 128;
-    if constexpr (BMODE == B_DUAL) {
-      // LDS column layout per wave wn: 32-col groups (gate jp=0, up jp=0, gate jp=1, up jp=1);
-      // output column c (0..127) -> wave c/64, pair (c%64)/32
-#pragma unroll 2
-      for (int it = 0; it < 128 * 16 / NT; ++it) {
-        const int id = it * NT + tid;
-        const int rr = id / 16, c = (id % 16) * 8;
-        const int64_t m = mrow0 + rr, n = n0 + c;
-        if (m >= M || n >= N) continue;
-        const int lc = (c / 64) * 128 + ((c % 64) / 32) * 64 + c % 32;
-        const float* pg = lds + rr * P + lc;
-        float e[8], g[8], h[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) { e[q] = pg[q]; g[q] = pg[32 + q]; h[q] = glu_fwd_h<EPI>(e[q], g[q]); }
-        const int64_t off = m * ep.ld_eg + n;
-        if (n + 8 <= N) {
-          if (ep.e) {  // training saves e and g; inference (e = g = null) stores h only
-            st16(ep.e + off, pack8(e));
-            st16(ep.g + off, pack8(g));
-          }
-          st16((__bf16*)ep.c + m * ep.ldc + n, pack8(h));
-        } else {
-          for (int q = 0; q < 8 && n + q < N; ++q) {
-            if (ep.e) {
-              ep.e[off + q] = (__bf16)e[q];
-              ep.g[off + q] = (__bf16)g[q];
-            }
-            ((__bf16*)ep.c)[m * ep.ldc + n + q] = (__bf16)h[q];
-          }
-        }
-      }
-    } else if constexpr (glu_bwd_epi(EPI)) {
-      // As for RoPE below: a thread's chunks share one column chunk c, so the
+    if constexpr (glu_bwd_epi(EPI)) {
+      // A thread's chunks share one column chunk c, so the
       // saved e / g chunks of four rows are read before any of them is used
       // (one row at a time left the epilogue waiting on each load).
       static_assert(NT % 32 == 0, "rows of 32 chunk-threads");
@@ -619,72 +580,6 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs& args,
               ep.g[off + q] = (__bf16)dev[q];
             }
           }
-        }
-      }
-    } else if constexpr (EPI == EPI_ROPE) {
-      // A thread's chunks share one column chunk c (rows tid / 32 + 16 it), so
-      // d and the lo / hi half are fixed: the positions of all its rows are
-      // read first, then the cos / sin chunks of four rows at a time, then
-      // those four rows are rotated and stored.  Issuing the table loads ahead
-      // keeps several in flight (one row at a time left the epilogue waiting
-      // on each load).
-      static_assert(NT % 32 == 0, "rows of 32 chunk-threads");
-      constexpr int IT = 128 * 32 / NT, RSTEP = NT / 32, GRP = IT >= 4 ? 4 : IT;
-      const int c = (tid % 32) * 8;
-      const int64_t n = n0 + c;
-      const bool rot = n < N && n < ep.rope_cols;
-      const int half = ep.head_dim / 2;
-      const int in_head = (int)(n % ep.head_dim);
-      const bool lo = in_head < half;
-      const int d = in_head % half;
-      int64_t posv[IT];
-#pragma unroll
-      for (int it = 0; it < IT; ++it) {
-        const int64_t m = mrow0 + it * RSTEP + tid / 32;
-        posv[it] = (rot && m < M) ? (ep.positions ? ep.positions[m] : m) : -1;
-      }
-#pragma unroll
-      for (int g0 = 0; g0 < IT; g0 += GRP) {
-        uint4 cv[GRP], sv[GRP];
-#pragma unroll
-        for (int j = 0; j < GRP; ++j) {
-          const int64_t pos = posv[g0 + j];
-          if (pos >= 0 && pos < ep.cs_rows) {
-            cv[j] = ld16(ep.cos + pos * ep.cs_ld + d);
-            sv[j] = ld16(ep.sin + pos * ep.cs_ld + d);
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < GRP; ++j) {
-          const int rr = (g0 + j) * RSTEP + tid / 32;
-          const int64_t m = mrow0 + rr;
-          if (m >= M || n >= N) continue;
-          const float* pv = lds + rr * P + c;
-          float v[8];
-#pragma unroll
-          for (int q = 0; q < 8; ++q) v[q] = pv[q];
-          if (rot) {
-            // the 128-column wave tile holds whole heads: partner half in LDS
-            const float* pp = lds + rr * P + (lo ? c + half : c - half);
-            const int64_t pos = posv[g0 + j];
-            float cs[8], sn[8];
-            if (pos >= 0 && pos < ep.cs_rows) {
-              unpack8(cv[j], cs);
-              unpack8(sv[j], sn);
-            } else {
-#pragma unroll
-              for (int q = 0; q < 8; ++q) cs[q] = sn[q] = __builtin_nanf("");
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-              const float x = bf16r(v[q]), xp = bf16r(pp[q]);
-              v[q] = lo ? x * cs[q] - xp * sn[q] : x * cs[q] + xp * sn[q];
-            }
-          }
-          __bf16* cp = (__bf16*)ep.c + m * ep.ldc + n;
-          if (n + 8 <= N) st16(cp, pack8(v));
-          else
-            for (int q = 0; q < 8 && n + q < N; ++q) cp[q] = (__bf16)v[q];
         }
       }
     } else {
@@ -766,7 +661,7 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs& args,
   }
 }
 
-template <class T, int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int EPI>
+template <class T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI>
 __device__ __forceinline__ void epilogue(const GemmArgs& args, f32x16 (&acc)[BM / WAVES_M / 32][BN / WAVES_N / 32],
                                          int64_t m0, int64_t n0, int lane, int wm, int wn) {
   constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N;
@@ -811,29 +706,6 @@ __device__ __forceinline__ void epilogue(const GemmArgs& args, f32x16 (&acc)[BM 
         }
       }
     }
-  } else if constexpr (glu_fwd_epi(EPI)) {
-    // wave tiles (0,1) and (2,3) are (gate, up) pairs for 32 output columns each
-#pragma unroll
-    for (int jp = 0; jp < FN / 2; ++jp) {
-      const int64_t n = n0 + wn * 64 + jp * 32 + col_in;
-      if (n >= args.N) continue;
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t m = row_base + i * 32 + 8 * (r / 4) + (r % 4);
-          if (m >= M) continue;
-          const float e = acc[i][2 * jp][r];
-          const float g = acc[i][2 * jp + 1][r];
-          const int64_t off = m * ep.ld_eg + n;
-          if (ep.e) {
-            ep.e[off] = (__bf16)e;
-            ep.g[off] = (__bf16)g;
-          }
-          ((__bf16*)ep.c)[m * ep.ldc + n] = (__bf16)glu_fwd_h<EPI>(e, g);
-        }
-      }
-    }
   } else if constexpr (glu_bwd_epi(EPI)) {
     // in-place GLU backward on the DW = dY @ W_down tile (glu_bwd_vals)
 #pragma unroll
@@ -855,56 +727,16 @@ __device__ __forceinline__ void epilogue(const GemmArgs& args, f32x16 (&acc)[BM 
         }
       }
     }
-  } else if constexpr (EPI == EPI_ROPE) {
-    // Each wave covers TN = 128 output columns aligned to a head boundary
-    // (head_dim 128: tiles 0,1 = lo half, 2,3 = hi half; head_dim 64: two
-    // heads, tiles (0,1) and (2,3)).
-    const int half_tiles = ep.head_dim / 64;  // partner distance in 32-col tiles
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t m = row_base + i * 32 + 8 * (r / 4) + (r % 4);
-        if (m >= M) continue;
-        const int64_t pos = ep.positions ? ep.positions[m] : m;
-        const bool pos_ok = pos >= 0 && pos < ep.cs_rows;
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int64_t n = n0 + wn * TN + j * 32 + col_in;
-          if (n >= args.N) continue;
-          float v = acc[i][j][r];
-          if (n < ep.rope_cols) {
-            const int jj = j % (2 * half_tiles);
-            const bool lo = jj < half_tiles;
-            const int partner = lo ? j + half_tiles : j - half_tiles;
-            float pv = 0.f;
-#pragma unroll
-            for (int q = 0; q < FN; ++q)
-              if (q == partner) pv = acc[i][q][r];
-            const int d = (int)(n % ep.head_dim) % (ep.head_dim / 2);
-            const float c = pos_ok ? (float)ep.cos[pos * ep.cs_ld + d] : __builtin_nanf("");
-            const float s = pos_ok ? (float)ep.sin[pos * ep.cs_ld + d] : __builtin_nanf("");
-            // round the projection to bf16 first: RoPE is applied to the
-            // materialised Q/K in the unfused reference path
-            const float x = bf16r(v), xp = bf16r(pv);
-            v = lo ? x * c - xp * s : x * c + xp * s;
-          }
-          ((__bf16*)ep.c)[m * ep.ldc + n] = (__bf16)v;
-        }
-      }
-    }
   }
 }
 
-template <class T, int BM, int BN, int WAVES_M, int WAVES_N, int A_LAYOUT, int B_LAYOUT, int BMODE, int EPI,
-          bool STAGED>
+template <class T, int BM, int BN, int WAVES_M, int WAVES_N, int A_LAYOUT, int B_LAYOUT, int EPI, bool STAGED>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_kernel(GemmArgs args) {
   constexpr int NT = WAVES_M * WAVES_N * 64;
   constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N;  // wave sub-tile
   constexpr int FM = TM / 32, FN = TN / 32;            // 32x32 MFMA tiles per wave
   static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile must be a multiple of 32");
-  static_assert(BMODE == B_SINGLE || TN == 128, "dual mode expects 128-row wave tiles");
 
   __shared__ __attribute__((aligned(16))) __bf16 smem[2 * (BM + BN) * LDS_PITCH];
   // stage b: A tile at smem + b*(BM+BN)*pitch, B tile right after it
@@ -912,14 +744,12 @@ void gemm_kernel(GemmArgs args) {
   auto Bs = [&](int b) { return smem + b * (BM + BN) * LDS_PITCH + BM * LDS_PITCH; };
 
   const int64_t M = args.M;
-  // output columns covered by one tile (dual: BN B-rows -> BN/2 outputs)
-  constexpr int OUT_BN = (BMODE == B_DUAL) ? BN / 2 : BN;
   const int64_t tiles_m = (M + BM - 1) / BM;
-  const int64_t tiles_n = (args.N + OUT_BN - 1) / OUT_BN;
+  const int64_t tiles_n = (args.N + BN - 1) / BN;
   int tmi, tni;
   tile_coords(tiles_m, tiles_n, tmi, tni, args);
   const int64_t m0 = (int64_t)tmi * BM;
-  const int64_t n0 = (int64_t)tni * OUT_BN;
+  const int64_t n0 = (int64_t)tni * BN;
 
   const int lane = threadIdx.x % 64;
   const int wave = threadIdx.x / 64;
@@ -931,7 +761,7 @@ void gemm_kernel(GemmArgs args) {
   int total_tiles = 0;
   for (int s = 0; s < args.n_segs; ++s) {
     const Seg& sg = args.segs[s];
-    const bool active = sg.n_hi > n0 && sg.n_lo < n0 + OUT_BN;
+    const bool active = sg.n_hi > n0 && sg.n_lo < n0 + BN;
     seg_tiles[s] = active ? (int)((sg.k + BK - 1) / BK) : 0;
     total_tiles += seg_tiles[s];
   }
@@ -947,26 +777,17 @@ void gemm_kernel(GemmArgs args) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  TileLoader<BM, NT, A_LAYOUT == ROW, false> la;
-  TileLoader<BN, NT, B_LAYOUT == COL, BMODE == B_DUAL> lb;
+  TileLoader<BM, NT, A_LAYOUT == ROW> la;
+  TileLoader<BN, NT, B_LAYOUT == COL> lb;
 
   // Points the loaders at segment s (this tile's panels of A and B).
   auto setup_seg = [&](int s) {
     const Seg& sg = args.segs[s];
-    la.setup(sg.a, sg.a, sg.lda, m0, [&](int q, int) -> int64_t { return m0 + q < M ? q : -1; });
-    if constexpr (BMODE == B_DUAL) {
-      lb.setup(sg.b, sg.b2, sg.ldb, n0, [&](int q, int) -> int64_t {
-        const int t4 = (q % 128) / 32;
-        const int rel = (q / 128) * 64 + (t4 / 2) * 32 + q % 32;
-        return n0 + rel < args.N ? rel : -1;
-      });
-    } else {
-      const int64_t off = n0 - sg.n_lo;
-      lb.setup(sg.b, sg.b, sg.ldb, off, [&](int q, int) -> int64_t {
-        const int64_t n = n0 + q;
-        return (n < args.N && n >= sg.n_lo && n < sg.n_hi) ? q : -1;
-      });
-    }
+    la.setup(sg.a, sg.lda, m0, [&](int q) -> int64_t { return m0 + q < M ? q : -1; });
+    lb.setup(sg.b, sg.ldb, n0 - sg.n_lo, [&](int q) -> int64_t {
+      const int64_t n = n0 + q;
+      return (n < args.N && n >= sg.n_lo && n < sg.n_hi) ? q : -1;
+    });
   };
 
   // cursor over (segment, k0) for the flat tile range [t_begin, t_end)
@@ -1064,9 +885,9 @@ void gemm_kernel(GemmArgs args) {
 
   if constexpr (STAGED) {
     static_assert(staged_ok(BM, BN, WAVES_M, WAVES_N, EPI), "staged epilogue: 256 x 256 tile, wave tiles of <= 128 rows");
-    epilogue_staged<T, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
+    epilogue_staged<T, WAVES_M, WAVES_N, EPI>(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
   } else {
-    epilogue<T, BM, BN, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn);
+    epilogue<T, BM, BN, WAVES_M, WAVES_N, EPI>(args, acc, m0, n0, lane, wm, wn);
   }
 }
 
@@ -1088,7 +909,7 @@ __device__ __forceinline__ int swz(int row) {
   else return (row >> 2) & 3;                      // BKT == 32: 4 rows per 256 bytes
 }
 
-template <int BROWS, int BKT, int NT, bool DUAL, int AUX = 0>
+template <int BROWS, int BKT, int NT, int AUX = 0>
 struct DmaLoader {
   static constexpr int RB = BKT * 2;          // LDS bytes per row
   static constexpr int CPR = RB / 16;         // 16-byte chunks per row
@@ -1097,25 +918,20 @@ struct DmaLoader {
   static constexpr int NW = NT / 64;
   static constexpr int IPW = NINST / NW;      // instructions per wave per tile
   static_assert(NINST % NW == 0 && IPW * RPI == BROWS / NW, "tile / wave split");
-  static_assert(!DUAL || RPI <= 32, "dual: an instruction's rows inside one 32-row group");
   uint32_t voff[IPW];   // byte offset of this lane's chunk in the panel (OOB = zero-fill)
-  const char* base[2];
+  const char* base;
   int64_t ld_bytes;
 
   template <class RowSrc>
-  __device__ __forceinline__ void setup(const void* p0, const void* p1, int64_t ld, int64_t panel_off,
-                                        RowSrc row_src) {
+  __device__ __forceinline__ void setup(const void* p, int64_t ld, int64_t panel_off, RowSrc row_src) {
     ld_bytes = ld * 2;
-    const int64_t pan = panel_off * ld_bytes;
-    base[0] = p0 ? (const char*)p0 + pan : nullptr;
-    base[1] = DUAL ? (p1 ? (const char*)p1 + pan : nullptr) : base[0];
+    base = p ? (const char*)p + panel_off * ld_bytes : nullptr;
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
 #pragma unroll
     for (int j = 0; j < IPW; ++j) {
       const int q = (wave * IPW + j) * RPI + lane / CPR;   // tile row
       const int chunk = (lane % CPR) ^ swz<BKT>(q);        // source chunk of LDS slot lane % CPR
-      const int sel = DUAL ? (((wave * IPW + j) * RPI) / 32) % 2 : 0;  // 32-row groups alternate gate / up
-      const int64_t row = base[sel] ? row_src(q, sel) : -1;
+      const int64_t row = base ? row_src(q) : -1;
       voff[j] = row < 0 ? OOB : (uint32_t)(row * ld_bytes + chunk * 16);
     }
   }
@@ -1124,8 +940,7 @@ struct DmaLoader {
   __device__ __forceinline__ void load(int64_t k0, int64_t kvalid, char* dst) {
     const int lane = threadIdx.x % 64;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const __amdgpu_buffer_rsrc_t r0 = make_rsrc(base[0] + k0 * 2);
-    const __amdgpu_buffer_rsrc_t r1 = make_rsrc(base[1] + k0 * 2);
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(base + k0 * 2);
 #pragma unroll
     for (int j = 0; j < IPW; ++j) {
       uint32_t off = voff[j];
@@ -1134,8 +949,7 @@ struct DmaLoader {
         const int chunk = (lane % CPR) ^ swz<BKT>(q);
         if (chunk * 8 >= kvalid) off = OOB;
       }
-      const int sel = DUAL ? (((wave * IPW + j) * RPI) / 32) % 2 : 0;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(sel ? r1 : r0,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r,
                                                (__attribute__((address_space(3))) void*)(dst + (wave * IPW + j) * 1024),
                                                16, off, 0, 0, AUX);
     }
@@ -1258,8 +1072,8 @@ __device__ __forceinline__ void wait_vmcnt() {
 // AT / BT: A stored [K][M] / B stored [K][N] (token-major, see DmaLoaderT).
 // CPA / CPB: cache-policy bits of the A / B buffer loads (0 = default; 2 =
 // nontemporal, for an operand that no other workgroup reads again).
-template <class T, int BM, int BN, int WAVES_M, int WAVES_N, int BMODE, int EPI, int BKT, int NSTAGE, bool STAGED,
-          int WPE, bool AT = false, bool BT = false, int CPA = 0, int CPB = 0>
+template <class T, int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int BKT, int NSTAGE, bool STAGED, int WPE,
+          bool AT = false, bool BT = false, int CPA = 0, int CPB = 0>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void gemm_dma_kernel(GemmArgs args) {
   constexpr int NT = WAVES_M * WAVES_N * 64;
@@ -1267,20 +1081,17 @@ void gemm_dma_kernel(GemmArgs args) {
   constexpr int FM = TM / 32, FN = TN / 32;
   constexpr int RB = BKT * 2;
   constexpr int A_BYTES = BM * RB, B_BYTES = BN * RB, STAGE = A_BYTES + B_BYTES;
-  static_assert(BMODE == B_SINGLE || TN == 128, "dual mode expects 128-row wave tiles");
-  static_assert(!(BT && BMODE == B_DUAL), "dual B operands are K-contiguous");
   constexpr int STAGED_B = STAGED ? STAGED_BYTES : 0;
   constexpr int SMEM = NSTAGE * STAGE > STAGED_B ? NSTAGE * STAGE : STAGED_B;
   __shared__ __attribute__((aligned(1024))) char smem[SMEM];
 
   const int64_t M = args.M;
-  constexpr int OUT_BN = (BMODE == B_DUAL) ? BN / 2 : BN;
   const int64_t tiles_m = (M + BM - 1) / BM;
-  const int64_t tiles_n = (args.N + OUT_BN - 1) / OUT_BN;
+  const int64_t tiles_n = (args.N + BN - 1) / BN;
   int tmi, tni;
   tile_coords(tiles_m, tiles_n, tmi, tni, args);
   const int64_t m0 = (int64_t)tmi * BM;
-  const int64_t n0 = (int64_t)tni * OUT_BN;
+  const int64_t n0 = (int64_t)tni * BN;
   const int lane = threadIdx.x % 64;
   const int wave = threadIdx.x / 64;
   const int wm = wave % WAVES_M;
@@ -1290,7 +1101,7 @@ void gemm_dma_kernel(GemmArgs args) {
   int total_tiles = 0;
   for (int s = 0; s < args.n_segs; ++s) {
     const Seg& sg = args.segs[s];
-    const bool active = sg.n_hi > n0 && sg.n_lo < n0 + OUT_BN;
+    const bool active = sg.n_hi > n0 && sg.n_lo < n0 + BN;
     seg_tiles[s] = active ? (int)((sg.k + BKT - 1) / BKT) : 0;
     total_tiles += seg_tiles[s];
   }
@@ -1306,28 +1117,21 @@ void gemm_dma_kernel(GemmArgs args) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  using LoaderA = std::conditional_t<AT, DmaLoaderT<BM, BKT, NT, CPA>, DmaLoader<BM, BKT, NT, false, CPA>>;
-  using LoaderB = std::conditional_t<BT, DmaLoaderT<BN, BKT, NT, CPB>, DmaLoader<BN, BKT, NT, BMODE == B_DUAL, CPB>>;
+  using LoaderA = std::conditional_t<AT, DmaLoaderT<BM, BKT, NT, CPA>, DmaLoader<BM, BKT, NT, CPA>>;
+  using LoaderB = std::conditional_t<BT, DmaLoaderT<BN, BKT, NT, CPB>, DmaLoader<BN, BKT, NT, CPB>>;
   LoaderA la;
   LoaderB lb;
   auto setup_seg = [&](int s) {
     const Seg& sg = args.segs[s];
     if constexpr (AT) la.setup(sg.a, sg.lda, m0, [&](int r) { return m0 + r < M; });
-    else la.setup(sg.a, sg.a, sg.lda, m0, [&](int q, int) -> int64_t { return m0 + q < M ? q : -1; });
+    else la.setup(sg.a, sg.lda, m0, [&](int q) -> int64_t { return m0 + q < M ? q : -1; });
     if constexpr (BT) {
       lb.setup(sg.b, sg.ldb, n0 - sg.n_lo, [&](int r) {
         const int64_t n = n0 + r;
         return n < args.N && n >= sg.n_lo && n < sg.n_hi;
       });
-    } else if constexpr (BMODE == B_DUAL) {
-      lb.setup(sg.b, sg.b2, sg.ldb, n0, [&](int q, int) -> int64_t {
-        const int t4 = (q % 128) / 32;
-        const int rel = (q / 128) * 64 + (t4 / 2) * 32 + q % 32;
-        return n0 + rel < args.N ? rel : -1;
-      });
     } else {
-      const int64_t off = n0 - sg.n_lo;
-      lb.setup(sg.b, sg.b, sg.ldb, off, [&](int q, int) -> int64_t {
+      lb.setup(sg.b, sg.ldb, n0 - sg.n_lo, [&](int q) -> int64_t {
         const int64_t n = n0 + q;
         return (n < args.N && n >= sg.n_lo && n < sg.n_hi) ? q : -1;
       });
@@ -1454,9 +1258,9 @@ void gemm_dma_kernel(GemmArgs args) {
   }
   if constexpr (STAGED) {
     static_assert(staged_ok(BM, BN, WAVES_M, WAVES_N, EPI), "staged epilogue: 256 x 256 tile, wave tiles of <= 128 rows");
-    epilogue_staged<T, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
+    epilogue_staged<T, WAVES_M, WAVES_N, EPI>(args, acc, m0, n0, lane, wm, wn, reinterpret_cast<float*>(smem));
   } else {
-    epilogue<T, BM, BN, WAVES_M, WAVES_N, BMODE, EPI>(args, acc, m0, n0, lane, wm, wn);
+    epilogue<T, BM, BN, WAVES_M, WAVES_N, EPI>(args, acc, m0, n0, lane, wm, wn);
   }
 }
 

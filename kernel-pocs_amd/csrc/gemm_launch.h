@@ -9,7 +9,7 @@ namespace fgemm {
 
 // Tile configurations.
 enum Cfg {
-  CFG_BIG = 0,       // 256 x 256: 2 x 2 waves (128 x 128 per wave); 4 x 2 on the token-major LDS-DMA path
+  CFG_BIG = 0,       // 256 x 256: 2 x 2 waves (128 x 128 per wave), or 4 x 2 (see launch_cfg)
   CFG_SKINNY_N = 1,  // N <= 32-ish (rank-r outputs): 64 x 64 tiles (2 x 2 waves) for a K-contiguous
                      // A, else 256 x 32 (4 x 1 waves)
   CFG_SKINNY_M = 2,  // 32 x 256, 1 x 4 waves: M <= 32-ish (LoRA A gradients)
@@ -150,14 +150,17 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
   if constexpr (BM == 256 && BN == 256 && AL == ROW && BL == COL) {
     // both operands K-contiguous: the 4-wave engine (128 x 128 per wave,
     // accumulators in AGPRs, a ring of five LDS half-slots fed by LDS-DMA)
-    if (launch_w4_staged<T, BMODE, EPI, false, false>(a, grid, s)) {
-    } else if (EPI == EPI_STORE_BF16 && a.ep.vec_ok && a.ep.beta != 0.f)
+    bool done = launch_w4_staged<T, BMODE, EPI, false, false>(a, grid, s);
+    if constexpr (EPI == EPI_STORE_BF16) {
       // beta reads C before the single rounding: the fp32-staged epilogue of
       // the 8-wave engine moves it as 16-byte vectors (rank-r products added
       // to a base product: K is short and C's traffic is the cost)
-      gemm_dma_kernel<T, BM, BN, 4, 2, BMODE, EPI, 64, 2, staged_ok(BM, BN, 4, 2, EPI), 2><<<grid, 512, 0, s>>>(a);
-    else
-      gemm_w4_kernel<T, BMODE, EPI, false><<<grid, 256, 0, s>>>(a);
+      if (!done && a.ep.vec_ok && a.ep.beta != 0.f) {
+        gemm_dma_kernel<T, BM, BN, 4, 2, EPI, 64, 2, true, 2><<<grid, 512, 0, s>>>(a);
+        done = true;
+      }
+    }
+    if (!done) gemm_w4_kernel<T, BMODE, EPI, false><<<grid, 256, 0, s>>>(a);
   } else if constexpr (BM == 64 && (BN == 64 || BN == 128 || BN == 256) && AL == ROW &&
                        (BL == COL || BL == ROW) && BMODE == B_SINGLE) {
     // narrow outputs (N <= 256: X A^T, dY B) with A K-contiguous: 64-row
@@ -170,7 +173,7 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
     constexpr int NS = BN == 256 ? 2 : 3;
     constexpr int WPE_N = BN == 64 ? 3 : 2;
     // (nontemporal loads of A, read by one column of tiles, measured 0.2% slower)
-    gemm_dma_kernel<T, BM, BN, WM, WN, BMODE, EPI, 64, NS, false, WPE_N, false, BL == ROW>
+    gemm_dma_kernel<T, BM, BN, WM, WN, EPI, 64, NS, false, WPE_N, false, BL == ROW>
         <<<grid, WM * WN * 64, 0, s>>>(a);
   } else if constexpr (BM == 96 && BN == 192 && AL == ROW && BL == COL && BMODE == B_SINGLE) {
     // 129..192 output columns (the three stacked rank-64 LoRA-A products of
@@ -180,17 +183,19 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
     // with two stages (two workgroups per CU): [22954, 4096] x [4096, 192]
     // 116 -> 94 us, [4096, 4096] x [4096, 192] 78 -> 61 us, bitwise-equal
     // output; 4 stages no faster than 3; 64 x 64 or 64 x 128 tiles slower.
-    gemm_dma_kernel<T, 96, 192, 3, 2, BMODE, EPI, 64, 3, false, 2><<<grid, 384, 0, s>>>(a);
+    gemm_dma_kernel<T, 96, 192, 3, 2, EPI, 64, 3, false, 2><<<grid, 384, 0, s>>>(a);
   } else if constexpr (AL == ROW && BL == ROW && BMODE == B_SINGLE && BM == 256 && BN == 256 &&
                        (EPI == EPI_STORE_BF16 || EPI == EPI_STORE_F32)) {
     // B as stored [K][N]: the 4-wave engine with transposing fragment reads of
-    // B; C read (beta) or stored by elements: the 8-wave LDS-DMA engine
-    constexpr bool DMA_STAGE = staged_ok(BM, BN, 4, 2, EPI);
+    // B; a 16-bit C that is read (beta) or activated, and stores by elements:
+    // the 8-wave LDS-DMA engine
+    // (every fp32 C with vectors is the 4-wave engine's)
+    constexpr bool DMA_STAGE = EPI == EPI_STORE_BF16;
     if (launch_w4_staged<T, BMODE, EPI, false, true>(a, grid, s)) {
     } else if (DMA_STAGE && a.ep.vec_ok)
-      gemm_dma_kernel<T, BM, BN, 4, 2, BMODE, EPI, 64, 2, DMA_STAGE, 2, false, true><<<grid, 512, 0, s>>>(a);
+      gemm_dma_kernel<T, BM, BN, 4, 2, EPI, 64, 2, DMA_STAGE, 2, false, true><<<grid, 512, 0, s>>>(a);
     else
-      gemm_dma_kernel<T, BM, BN, 4, 2, BMODE, EPI, 64, 2, false, 2, false, true><<<grid, 512, 0, s>>>(a);
+      gemm_dma_kernel<T, BM, BN, 4, 2, EPI, 64, 2, false, 2, false, true><<<grid, 512, 0, s>>>(a);
   } else if constexpr (AL == COL && BL == ROW && BMODE == B_SINGLE && BM == 256 && BN == 256) {
     // both operands token-major (A^T B reduced over tokens): as above, with
     // transposing fragment reads of both
@@ -198,9 +203,9 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
     constexpr bool DMA_STAGE = staged_ok(BM, BN, DWM, DWN, EPI);
     if (launch_w4_staged<T, BMODE, EPI, true, true>(a, grid, s)) {
     } else if (DMA_STAGE && a.ep.vec_ok)
-      gemm_dma_kernel<T, BM, BN, DWM, DWN, BMODE, EPI, 64, 2, DMA_STAGE, 2, true, true><<<grid, DWM * DWN * 64, 0, s>>>(a);
+      gemm_dma_kernel<T, BM, BN, DWM, DWN, EPI, 64, 2, DMA_STAGE, 2, true, true><<<grid, DWM * DWN * 64, 0, s>>>(a);
     else
-      gemm_dma_kernel<T, BM, BN, DWM, DWN, BMODE, EPI, 64, 2, false, 2, true, true><<<grid, DWM * DWN * 64, 0, s>>>(a);
+      gemm_dma_kernel<T, BM, BN, DWM, DWN, EPI, 64, 2, false, 2, true, true><<<grid, DWM * DWN * 64, 0, s>>>(a);
   } else if constexpr (AL == COL && BL == ROW && BMODE == B_SINGLE && ((BM == 256 && BN <= 64) || (BM == 32 && BN == 256))) {
     // skinny token reductions (LoRA weight gradients): as the skinny
     // K-contiguous case, with token-major operands
@@ -208,18 +213,18 @@ static int launch_cfg(GemmArgs a, hipStream_t s) {
     // its loads are nontemporal and leave the caches to the narrow one
     // (LoRA-MLP step 0.35%, LoRA-QKV step 0.7% faster, same box)
     constexpr int CPA_T = BM == 256 ? CP_STREAM : 0, CPB_T = BM == 256 ? 0 : CP_STREAM;
-    gemm_dma_kernel<T, BM, BN, WM, WN, BMODE, EPI, 64, SKINNY_NSTAGE, false, SKINNY_WPE, true, true, CPA_T, CPB_T>
+    gemm_dma_kernel<T, BM, BN, WM, WN, EPI, 64, SKINNY_NSTAGE, false, SKINNY_WPE, true, true, CPA_T, CPB_T>
         <<<grid, WM * WN * 64, 0, s>>>(a);
   } else if constexpr (BM == 256 && BN <= 64 && AL == ROW && BL == COL && BMODE == B_SINGLE) {
     // skinny output, K-contiguous operands (X A^T, dY B with B^T given): the
     // big operand streams through the LDS-DMA ring; ~72-80 KB of LDS lets two
     // workgroups share a CU, so two K tiles per CU are in flight
-    gemm_dma_kernel<T, BM, BN, WM, WN, BMODE, EPI, SKINNY_BKT, SKINNY_NSTAGE, false, SKINNY_WPE><<<grid, WM * WN * 64, 0, s>>>(a);
+    gemm_dma_kernel<T, BM, BN, WM, WN, EPI, SKINNY_BKT, SKINNY_NSTAGE, false, SKINNY_WPE><<<grid, WM * WN * 64, 0, s>>>(a);
   } else {
     if (staged)
-      gemm_kernel<T, BM, BN, WM, WN, AL, BL, BMODE, EPI, CAN_STAGE><<<grid, WM * WN * 64, 0, s>>>(a);
+      gemm_kernel<T, BM, BN, WM, WN, AL, BL, EPI, CAN_STAGE><<<grid, WM * WN * 64, 0, s>>>(a);
     else
-      gemm_kernel<T, BM, BN, WM, WN, AL, BL, BMODE, EPI, false><<<grid, WM * WN * 64, 0, s>>>(a);
+      gemm_kernel<T, BM, BN, WM, WN, AL, BL, EPI, false><<<grid, WM * WN * 64, 0, s>>>(a);
   }
   FORGE_CHECK_LAUNCH();
   return FORGE_OK;
