@@ -379,8 +379,8 @@ void gemm_w4_kernel(GemmArgs args) {
   // quarter of a tile held the in-order issue: loop time per K tile 3300
   // cycles against the MFMAs' 2048).
   if (n_t > 0) {
-    // prologue: A0, B0, A1 whole and the first half of B1's instructions
-    // into half-slots 0 .. 3; B1's rest and A2 follow in tile 0's k-steps
+    // prologue: A0, B0, A1 and B1 into half-slots 0 .. 3 (the wait below counts
+    // the IPH instructions of each); A2 follows in tile 0's k-steps
     at_a(0, pa_cur);
 #pragma unroll
     for (int d = 0; d < IPH; ++d) la.load_one(pa_cur, d, half_ptr(0));

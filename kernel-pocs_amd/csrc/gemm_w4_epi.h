@@ -21,8 +21,10 @@
 // whole 8192 x 14336 output (K = 0 launches): fp32 staging of 128-row halves
 // 16.2 us per round of 256 tiles.
 //
-// The direct epilogue (atomic outputs, a 16-bit C with beta != 0, and buffers
-// whose alignment rules out 16-byte vectors) works per element from registers.
+// The direct epilogue (atomic outputs, a 16-bit C with an activation or
+// per-column alphas, and buffers whose alignment rules out 16-byte vectors)
+// works per element from registers.  A 16-bit C with beta != 0 goes to the
+// 8-wave engine where vectors allow.
 #pragma once
 
 #include "gemm_core.h"
@@ -119,40 +121,40 @@ __device__ __forceinline__ void w4_epilogue_direct(const GemmArgs& args, f32x4 (
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-          const int64_t nb = n0 + wn * 128 + 16 * j + cl;
-          if (nb >= N) continue;
-          if constexpr (EPI == EPI_STORE_F32) {
-            float* cp = (float*)ep.c + (int64_t)blockIdx.z * ep.split_stride + m * ep.ldc + nb;
-            float v[4];
+        const int64_t nb = n0 + wn * 128 + 16 * j + cl;
+        if (nb >= N) continue;
+        if constexpr (EPI == EPI_STORE_F32) {
+          float* cp = (float*)ep.c + (int64_t)blockIdx.z * ep.split_stride + m * ep.ldc + nb;
+          float v[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] = col_alpha(ep, nb + q) * acc[i][j][q];
-            for (int q = 0; q < 4 && nb + q < N; ++q) {
-              float o = v[q];
-              if (ep.beta != 0.f) o += ep.beta * cp[q];
-              cp[q] = ep.act ? epi_act(ep.act, o) : o;
-            }
-          } else if constexpr (EPI == EPI_ATOMIC_F32) {
-            for (int q = 0; q < 4 && nb + q < N; ++q)
-              atomicAdd((float*)ep.c + m * ep.ldc + nb + q, col_alpha(ep, nb + q) * acc[i][j][q]);
-          } else if constexpr (EPI == EPI_STORE_BF16) {
-            T* cp = (T*)ep.c + m * ep.ldc + nb;
-            for (int q = 0; q < 4 && nb + q < N; ++q) {
-              float o = col_alpha(ep, nb + q) * acc[i][j][q];
-              if (ep.beta != 0.f) o += ep.beta * (float)cp[q];
-              if (ep.act) o = epi_act(ep.act, o);
-              cp[q] = (T)o;
-            }
-          } else if constexpr (glu_bwd_epi(EPI)) {
-            for (int q = 0; q < 4 && nb + q < N; ++q) {
-              const int64_t off = m * ep.ld_eg + nb + q;
-              float h, df, de;
-              glu_bwd_vals<EPI>(acc[i][j][q], (float)ep.e[off], (float)ep.g[off], h, df, de);
-              ((__bf16*)ep.c)[m * ep.ldc + nb + q] = (__bf16)h;
-              ep.e[off] = (__bf16)df;
-              ep.g[off] = (__bf16)de;
-            }
+          for (int q = 0; q < 4; ++q) v[q] = col_alpha(ep, nb + q) * acc[i][j][q];
+          for (int q = 0; q < 4 && nb + q < N; ++q) {
+            float o = v[q];
+            if (ep.beta != 0.f) o += ep.beta * cp[q];
+            cp[q] = ep.act ? epi_act(ep.act, o) : o;
+          }
+        } else if constexpr (EPI == EPI_ATOMIC_F32) {
+          for (int q = 0; q < 4 && nb + q < N; ++q)
+            atomicAdd((float*)ep.c + m * ep.ldc + nb + q, col_alpha(ep, nb + q) * acc[i][j][q]);
+        } else if constexpr (EPI == EPI_STORE_BF16) {
+          T* cp = (T*)ep.c + m * ep.ldc + nb;
+          for (int q = 0; q < 4 && nb + q < N; ++q) {
+            float o = col_alpha(ep, nb + q) * acc[i][j][q];
+            if (ep.beta != 0.f) o += ep.beta * (float)cp[q];
+            if (ep.act) o = epi_act(ep.act, o);
+            cp[q] = (T)o;
+          }
+        } else if constexpr (glu_bwd_epi(EPI)) {
+          for (int q = 0; q < 4 && nb + q < N; ++q) {
+            const int64_t off = m * ep.ld_eg + nb + q;
+            float h, df, de;
+            glu_bwd_vals<EPI>(acc[i][j][q], (float)ep.e[off], (float)ep.g[off], h, df, de);
+            ((__bf16*)ep.c)[m * ep.ldc + nb + q] = (__bf16)h;
+            ep.e[off] = (__bf16)df;
+            ep.g[off] = (__bf16)de;
           }
         }
+      }
     }
   }
 }

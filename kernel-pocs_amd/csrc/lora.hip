@@ -275,7 +275,7 @@ static int gate_up(int64_t M, int64_t H, int64_t I, int64_t r, const void* x, in
   if (r > 0 && xa) {
     // one K segment of 2r: gate rows take xa[:, :r] Bg^T, up rows xa[:, r:2r]
     // Bu^T (k_split = r), so both rank-r products share one K tile of the
-    // 4-wave engine (which every dual-B launch runs on) instead of two
+    // 4-wave engine (past 64 rows; the row engine takes fewer) instead of two
     a.segs[ns++] = Seg{(const __bf16*)xa, ld_xa, (const __bf16*)b_gate, (const __bf16*)b_up, ldb, 2 * r, 0, I, r};
   }
   a.n_segs = ns;

@@ -228,7 +228,7 @@ def frozen_t(w: torch.Tensor, pitch_multiple: int = 1) -> torch.Tensor:
 
     The backward GEMMs contract over the weight's output dimension, which is
     not contiguous in the nn.Linear layout; with W^T they become K-contiguous
-    and run on the LDS-DMA engine.  The copy is made once per weight (LoRA
+    (the 4-wave engine's and the row engine's faster form).  The copy is made once per weight (LoRA
     freezes the base weights) and dropped when the weight is freed, changed
     in place (tensor._version) or given new storage (data_ptr).
     pitch_multiple > 1 returns [in, out_pad] with out_pad the next multiple
