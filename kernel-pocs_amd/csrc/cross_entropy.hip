@@ -18,8 +18,7 @@
 //     C writes p/d.  Used for the common case (2-byte logits, no class
 //     weights / softcap / argmax) when the row fits in 512 * 32 * 8 elements.
 //   * ce_stream_kernel: any row length, alignment and every feature; the row
-//     is streamed twice (online max/sum, then gradient), the second read
-//     largely served by the Infinity Cache.
+//     is streamed twice (online max/sum, then gradient).
 // exp is evaluated as exp2 on log2e-prescaled values (one FMA + v_exp_f32).
 #include <atomic>
 #include <mutex>
@@ -457,14 +456,15 @@ __device__ __forceinline__ bool ce_row_head(CeArgs& a, int64_t row, int64_t y, T
 // row at 16-bit logits costs about 30 issue slots an element, so what the
 // flags switch is a template parameter or a branch per vector, never per
 // element, the divisions of 16-bit gradients by the token count are folded into
-// one scale and shift, and the soft cap is a polynomial (cap_fast).  The second pass reads
-// the Infinity Cache (a bound on the workgroups per CU, so on the rows in
-// flight, measured equal).
+// one scale and shift, and the soft cap is a polynomial (cap_fast).  Both reads
+// of a long row leave the L2 (FETCH_SIZE 1.96 GB for 1945 rows of 512 KB, and
+// the rows in flight are twice the Infinity Cache): two reads and one write are
+// the 6.2 TB/s of a copy (a bound on the rows in flight measured equal).
 // Measured on MI355X, forward + backward, before -> after the vector ALU work
-// was cut and rows were peeled: bf16 [2048, 256000] softcap 30 1102 -> 490 us,
-// [4096, 151936] 869 -> 530, [8192, 50257] (rows off 16-byte alignment, which
-// went element by element) 1637 -> 372; fp32 [4096, 128256] 1262 -> 866; bf16
-// [8192, 128256] loss, accuracy and predictions 721 -> 412.
+// was cut and rows were peeled: bf16 [2048, 256000] softcap 30 1076 -> 510 us,
+// [4096, 151936] 871 -> 542, [8192, 50257] (rows off 16-byte alignment, which
+// went element by element) 1631 -> 356; fp32 [4096, 128256] 1235 -> 883; bf16
+// [8192, 128256] loss, accuracy and predictions 649 -> 362.
 // ---------------------------------------------------------------------------
 constexpr int kStreamU = 4;  // vectors in flight per thread
 
@@ -961,12 +961,11 @@ void launch_stream_sw(const CeArgs& a, dim3 grid, hipStream_t s) {
   // Measured on MI355X, 8192 rows, 512 against 256 threads: bf16 257 columns 59
   // / 24 us, 4096 with accuracy and predictions 75 / 32, 16384 with softcap 150
   // / 118; fp32 4096 73 / 47, 8192 115 / 102; 16384 213 / 230.
-  // Long rows take 1024: half the rows in flight, which the second
-  // pass still finds in the Infinity Cache.  512 against
-  // 1024 threads: [2048, 256000] fp32 1040 / 898 us, [4096, 128256] fp32 890
-  // / 866, [4096, 151936] bf16 550 / 532, [8192, 50257] bf16 386 / 392.  With
+  // Rows of 256 KB and more take 1024: half the rows in flight.  512 against
+  // 1024 threads: [2048, 256000] fp32 1075 / 896 us, [4096, 128256] fp32 911
+  // / 872, [4096, 151936] bf16 550 / 531, [8192, 50257] bf16 352 / 387.  With
   // a softcap the arithmetic holds the kernel and the smaller workgroups'
-  // barriers cost less: [2048, 256000] bf16 494 / 519, [4096, 32000] 146 / 184.
+  // barriers cost less: [2048, 256000] bf16 510 / 509, [4096, 32000] 152 / 192.
   const int64_t bytes = a.n_cols * (int64_t)sizeof(T);
   const bool wide = !SC && bytes >= 256 * 1024;
   if (a.flags & (FORGE_CE_RETURN_ACCURACY | FORGE_CE_RETURN_PREDICTED)) {

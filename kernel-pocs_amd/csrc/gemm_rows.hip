@@ -42,8 +42,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(GemmArgs args) {
   for (int s = 0; s < args.n_segs; ++s) {
     const Seg& sg = args.segs[s];
     if (sg.n_hi <= n0 || sg.n_lo >= n0 + 16 * CB) continue;
-    // (a lane whose row does not exist reads zeros; n - n_lo >= -15 from a
-    // base of row n0 - n_lo, which is itself at least -15 and never read then)
+    // (a lane whose row does not exist reads zeros; the base, row n0 - n_lo, may
+    // lie before the operand, where no lane reads)
     const int64_t brow = n0 - sg.n_lo;
     uint32_t boff[CB];
 #pragma unroll
